@@ -106,3 +106,56 @@ def test_invalid_csr_is_rejected_before_use():
     ci2[1], ci2[2] = ci2[2], ci2[1]
     with pytest.raises(ligmg_amd.LigmgError):
         ligmg_amd.Solver((g.rowptr, ci2, g.vals))
+
+
+@pytest.mark.parametrize("n,hub,diagonal", [(1, 0, 0.0), (70, 0, 0.5), (700, 64, 1.0), (3000, 1025, 0.0),
+                                            (3000, 2999, 0.3), (5000, 4096, 0.5)])
+def test_prep_entry_chunks(n, hub, diagonal):
+    """Passes over stored entries in chunks of 1024: rows that cross chunks,
+    empty rows, hub rows, stored and missing diagonals, one-sided patterns,
+    and a submatrix that drops entries of its rows and reorders them."""
+    import torch
+    rng = np.random.default_rng(n + hub)
+    A = sp.random(n, n, density=min(1.0, 3.0 / n), random_state=rng, format="lil")
+    A[rng.integers(0, n, n // 5), :] = 0
+    if hub:
+        A[n // 2, rng.permutation(n)[:hub]] = 1.5
+    A.setdiag(np.where(rng.random(n) < diagonal, 2.0, 0.0))
+    A = A.tocsr()
+    A.eliminate_zeros()
+    A.sort_indices()
+    rp, ci, v = A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data.astype(np.float64)
+    dev = torch.device("cuda:0")
+    d = tuple(torch.from_numpy(a).to(dev) for a in (rp, ci if len(ci) else np.zeros(1, np.int32), v if len(v) else np.zeros(1)))
+    lab, k = prep.components(d)
+    nc, c = sp.csgraph.connected_components(A, directed=False)
+    top = np.full(nc, -1)
+    np.maximum.at(top, c, np.arange(n))
+    assert k == nc and np.array_equal(lab.cpu().numpy(), top[c])
+    L = prep.adjacency_to_laplacian(d)
+    for a, b in zip(L, O.adjacency_to_laplacian(rp, ci, v)):
+        assert np.array_equal(a.cpu().numpy(), b)
+    keep = rng.permutation(n)[:max(1, 2 * n // 3)]  # new id of kept vertex keep[i]: i
+    nid = np.full(n, -1, np.int32)
+    nid[keep] = np.arange(len(keep))
+    sub = A[np.sort(keep)][:, np.sort(keep)].tocoo()  # entries in the input's column order
+    rows, cols = nid[np.sort(keep)[sub.row]], nid[np.sort(keep)[sub.col]]
+    order = np.lexsort((np.arange(len(rows)), rows))
+    dn = torch.from_numpy(nid).to(dev)
+    orp = torch.empty(len(keep) + 1, dtype=torch.int32, device=dev)
+    oci = torch.empty(max(1, sub.nnz), dtype=torch.int32, device=dev)
+    ov = torch.empty(max(1, sub.nnz), dtype=torch.float64, device=dev)
+    torch.cuda.synchronize()
+    lib = _ffi.solver_lib()
+    args = (n, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), dn.data_ptr(), len(keep), _ffi.MEM_DEVICE)
+    assert lib.ligmg_extract(*args, orp.data_ptr(), oci.data_ptr(), ov.data_ptr()) == 0
+    assert np.array_equal(np.diff(orp.cpu().numpy()), np.bincount(rows, minlength=len(keep)))
+    assert np.array_equal(oci.cpu().numpy()[:sub.nnz], cols[order])
+    assert np.array_equal(ov.cpu().numpy()[:sub.nnz], sub.data[order])
+    # outputs that overlap the inputs: the same result
+    assert lib.ligmg_extract(*args, orp.data_ptr(), d[1].data_ptr(), d[2].data_ptr()) == 0
+    assert np.array_equal(d[1].cpu().numpy()[:sub.nnz], cols[order])
+    assert np.array_equal(d[2].cpu().numpy()[:sub.nnz], sub.data[order])
+    dn[int(keep[0])] = len(keep)
+    torch.cuda.synchronize()
+    assert lib.ligmg_extract(*args, orp.data_ptr(), oci.data_ptr(), ov.data_ptr()) == _ffi.ERR_INVALID
