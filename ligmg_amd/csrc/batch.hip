@@ -11,6 +11,7 @@
 #include "../../include/ligmg_amd.h"
 #include "ops.hpp"
 #include "prims.hpp"
+#include "solve_dev.hpp"
 
 namespace lg {
 
@@ -18,75 +19,18 @@ namespace {
 
 template <class T>
 struct BValOne {
+  static constexpr bool one = true;
   __device__ __forceinline__ T operator()(int64_t) const { return (T)1; }
 };
 template <class T>
 struct BValArr {
+  static constexpr bool one = false;
   const T *v;
   __device__ __forceinline__ T operator()(int64_t k) const { return v[k]; }
 };
 
-// ----------------------------------------------------------- epilogues (i, c)
-template <class T>
-struct BStore {
-  T *y;
-  int kp;
-  __device__ __forceinline__ void operator()(int64_t i, int c, double s) const {
-    y[i * kp + c] = (T)s;
-  }
-};
-template <class T>
-struct BResid {
-  const T *b;
-  T *r;
-  int kp;
-  __device__ __forceinline__ void operator()(int64_t i, int c, double s) const {
-    const int64_t o = i * kp + c;
-    r[o] = (T)((double)b[o] - s);
-  }
-};
-template <class T>
-struct BCheb {
-  const T *dinv, *b, *xc, *xp;
-  T *xn;
-  double alpha, beta;
-  int kp;
-  __device__ __forceinline__ void operator()(int64_t i, int c, double s) const {
-    const int64_t o = i * kp + c;
-    double cur = (double)xc[o];
-    double d = alpha * (cur - (xp ? (double)xp[o] : 0.0));  // null xp: zero previous iterate
-    xn[o] = (T)(cur + d + beta * (double)dinv[i] * ((double)b[o] - s));
-  }
-};
-template <class T>
-struct BInterp {
-  const T *q, *b;
-  T *x;
-  int kp;
-  __device__ __forceinline__ void operator()(int64_t i, int c, double s) const {
-    const int64_t o = i * kp + c;
-    x[o] = (T)(s + (double)q[i] * (double)b[o]);
-  }
-};
-template <class T, class Epi>
-struct BDiag {  // FP32 Laplacian form: + d[i] x[i, c]
-  const double *d;
-  const T *x;
-  Epi e;
-  int kp;
-  __device__ __forceinline__ void operator()(int64_t i, int c, double s) const {
-    e(i, c, s + d[i] * (double)x[i * kp + c]);
-  }
-};
-
-// One workgroup per unit (the SpMV units).  Complete-row units: group g of
-// kp / VW lanes handles rows g, g + G, ...; lane t of a group handles the
-// VW adjacent right-hand sides t*VW .. t*VW + VW - 1 with one wide load per
-// gathered row of X, and keeps U entries' gathers in flight.  Long-row
-// chunks: groups of kp lanes (one right-hand side each, whatever VW) split
-// the chunk's entries and reduce through LDS into kp partial sums.  Every
-// (row, right-hand side) sum of a complete row is one lane adding the row's
-// entries in stored order, so the tile (VW, U) does not change any bit.
+// VW adjacent right-hand sides of one row: 16 bytes, or the whole row of a
+// narrower block
 template <class T, int VW>
 struct BVec {
   typedef T type __attribute__((ext_vector_type(VW)));
@@ -100,68 +44,237 @@ __device__ __forceinline__ double bvec_at(const typename BVec<T, VW>::type &x, i
   if constexpr (VW == 1) return (double)x;
   else return (double)x[v];
 }
+template <class T, int VW>
+__device__ __forceinline__ typename BVec<T, VW>::type bvec_load(const T *p) {
+  return *(const typename BVec<T, VW>::type *)p;
+}
+template <class T, int VW, class F>
+__device__ __forceinline__ void bvec_store(T *p, const F &f) {
+  typename BVec<T, VW>::type y;
+  if constexpr (VW == 1) {
+    y = f(0);
+  } else {
+#pragma unroll
+    for (int v = 0; v < VW; v++) y[v] = f(v);
+  }
+  *(typename BVec<T, VW>::type *)p = y;
+}
 
+// ----------------------------------------------------------------- epilogues
+// load: a row's other operands, asked for before its sum is formed; store:
+// the result of VW adjacent right-hand sides from their sums s.
+template <class T>
+struct BStore {
+  T *y;
+  int kp;
+  template <int VW>
+  struct Pre {};
+  template <int VW>
+  __device__ __forceinline__ Pre<VW> load(int64_t, int) const {
+    return {};
+  }
+  template <int VW>
+  __device__ __forceinline__ void store(int64_t i, int c, const double *s, const Pre<VW> &) const {
+    bvec_store<T, VW>(y + i * kp + c, [&](int v) { return (T)s[v]; });
+  }
+};
+template <class T>
+struct BResid {
+  const T *b;
+  T *r;
+  int kp;
+  template <int VW>
+  struct Pre {
+    typename BVec<T, VW>::type b;
+  };
+  template <int VW>
+  __device__ __forceinline__ Pre<VW> load(int64_t i, int c) const {
+    return {bvec_load<T, VW>(b + i * kp + c)};
+  }
+  template <int VW>
+  __device__ __forceinline__ void store(int64_t i, int c, const double *s, const Pre<VW> &p) const {
+    bvec_store<T, VW>(r + i * kp + c, [&](int v) { return (T)(bvec_at<T, VW>(p.b, v) - s[v]); });
+  }
+};
+template <class T>
+struct BCheb {
+  const T *dinv, *b, *xc, *xp;
+  T *xn;
+  double alpha, beta;
+  int kp;
+  template <int VW>
+  struct Pre {
+    typename BVec<T, VW>::type b, xc, xp;
+    double dinv;
+  };
+  template <int VW>
+  __device__ __forceinline__ Pre<VW> load(int64_t i, int c) const {
+    const int64_t o = i * kp + c;
+    Pre<VW> p;
+    p.b = bvec_load<T, VW>(b + o);
+    p.xc = bvec_load<T, VW>(xc + o);
+    if (xp) p.xp = bvec_load<T, VW>(xp + o);
+    else p.xp = p.xc;
+    p.dinv = (double)dinv[i];
+    return p;
+  }
+  template <int VW>
+  __device__ __forceinline__ void store(int64_t i, int c, const double *s, const Pre<VW> &p) const {
+    bvec_store<T, VW>(xn + i * kp + c, [&](int v) {
+      const double cur = bvec_at<T, VW>(p.xc, v);
+      // null xp: zero previous iterate
+      const double d = alpha * (cur - (xp ? bvec_at<T, VW>(p.xp, v) : 0.0));
+      return (T)(cur + d + beta * p.dinv * (bvec_at<T, VW>(p.b, v) - s[v]));
+    });
+  }
+};
+template <class T>
+struct BInterp {
+  const T *q, *b;
+  T *x;
+  int kp;
+  template <int VW>
+  struct Pre {
+    typename BVec<T, VW>::type b;
+    double q;
+  };
+  template <int VW>
+  __device__ __forceinline__ Pre<VW> load(int64_t i, int c) const {
+    return {bvec_load<T, VW>(b + i * kp + c), (double)q[i]};
+  }
+  template <int VW>
+  __device__ __forceinline__ void store(int64_t i, int c, const double *s, const Pre<VW> &p) const {
+    bvec_store<T, VW>(x + i * kp + c, [&](int v) { return (T)(s[v] + p.q * bvec_at<T, VW>(p.b, v)); });
+  }
+};
+template <class T, class Epi>
+struct BDiag {  // FP32 Laplacian form: + d[i] x[i, c]
+  const double *d;
+  const T *x;
+  Epi e;
+  int kp;
+  template <int VW>
+  struct Pre {
+    typename BVec<T, VW>::type x;
+    double d;
+    typename Epi::template Pre<VW> e;
+  };
+  template <int VW>
+  __device__ __forceinline__ Pre<VW> load(int64_t i, int c) const {
+    return {bvec_load<T, VW>(x + i * kp + c), d[i], e.template load<VW>(i, c)};
+  }
+  template <int VW>
+  __device__ __forceinline__ void store(int64_t i, int c, const double *s, const Pre<VW> &p) const {
+    double t[VW];
+#pragma unroll
+    for (int v = 0; v < VW; v++) t[v] = s[v] + p.d * bvec_at<T, VW>(p.x, v);
+    e.template store<VW>(i, c, t, p.e);
+  }
+};
+
+// Y = A X by the SpMV's work units; workgroup (u, y) takes part y of the
+// rows of unit u.  It stages the part's columns, values and row offsets in
+// LDS with coalesced loads, so a row costs one round of gathers of X (U in
+// flight, masked past the row's end) with its epilogue operands already
+// asked for, instead of a chain of row pointer, column, gather and epilogue
+// loads.  A row is summed by S groups of L = kp / VW lanes (S by the unit's
+// mean row length: about 16 entries a group), group j adding entries j,
+// j + S, ... in order, and the S partials meet in an xor butterfly inside
+// one wavefront; S = 1 adds the row in stored order.  S does not depend on U
+// or on the parts, so neither changes any bit.  Long-row chunks: every group
+// of the workgroup takes a share, butterfly per wavefront, the wavefronts'
+// sums added in order into kp partial sums.
+// It is bound by gathers in flight.  One FP32 Chebyshev step, against a
+// kernel that walked the row from global memory (one group a row, whatever
+// its length): 100^3 grid (7 entries a row) x 32: 301 -> 175 us; 12
+// Barabasi-Albert graphs (7.7 M entries, hubs) x 16: 252 -> 164 us; their
+// 36-unit levels 80 -> 29 us.
 template <class T, int VW, int U, class Val, class Epi>
 __global__ void __launch_bounds__(256)
     k_spmm_units(const int32_t *__restrict__ rp, const int32_t *__restrict__ ci, Val val,
-                 const T *__restrict__ X, int kp, int lk, const int32_t *__restrict__ urow0,
+                 const T *__restrict__ X, int kp, int lg, const int32_t *__restrict__ urow0,
                  const int32_t *__restrict__ unrows, const int32_t *__restrict__ ukoff,
                  double *__restrict__ parts, Epi epi) {
   typedef typename BVec<T, VW>::type V;
+  constexpr bool ONE = Val::one;
+  __shared__ int32_t scol[UNIT_NNZ];
+  __shared__ T sval[ONE ? 1 : UNIT_NNZ];
+  __shared__ int32_t soff[UNIT_ROWS + 1];
+  __shared__ double red[256 / WAVE][64];
   const int u = blockIdx.x;
   const int row0 = urow0[u], nr = unrows[u], k0 = ukoff[u];
+  const int L = 1 << lg, G = 256 >> lg;  // lanes of a group, groups
+  const int gid = threadIdx.x >> lg, c0 = (threadIdx.x & (L - 1)) * VW;
+  auto stage = [&](int ka, int cnt) {
+    for (int t = threadIdx.x; t < cnt; t += 256) {
+      scol[t] = ci[ka + t];
+      if constexpr (!ONE) sval[t] = val(ka + t);
+    }
+  };
+  // adds entries a, a + step, ... below b to s
+  auto add = [&](double *s, int a, int b, int step) {
+    for (int j = a; j < b; j += U * step) {
+      V xx[U];
+      double vv[U];
+#pragma unroll
+      for (int t = 0; t < U; t++) {
+        const int e = j + t * step < b ? j + t * step : j;
+        xx[t] = *(const V *)(X + (int64_t)scol[e] * kp + c0);
+        if constexpr (ONE) vv[t] = 1.0;
+        else vv[t] = (double)sval[e];
+      }
+#pragma unroll
+      for (int t = 0; t < U; t++)
+#pragma unroll
+        for (int v = 0; v < VW; v++) s[v] += j + t * step < b ? vv[t] * bvec_at<T, VW>(xx[t], v) : 0.0;
+    }
+  };
+  double s[VW];
   if (nr > 0) {
-    const int lg = lk - (VW == 1 ? 0 : VW == 2 ? 1 : VW == 4 ? 2 : 3);  // log2(lanes per row)
-    const int G = 256 >> lg;
-    const int g = threadIdx.x >> lg, c0 = (threadIdx.x & ((1 << lg) - 1)) * VW;
-    for (int r = g; r < nr; r += G) {
-      const int row = row0 + r;
-      const int a = rp[row], b = rp[row + 1];
-      double s[VW];
+    const int per = (nr + gridDim.y - 1) / gridDim.y, ra = blockIdx.y * per, nl = min(per, nr - ra);
+    if (nl <= 0) return;
+    const int ka = rp[row0 + ra], cnt = rp[row0 + ra + nl] - ka;
+    for (int t = threadIdx.x; t <= nl; t += 256) soff[t] = rp[row0 + ra + t] - ka;
+    stage(ka, cnt);
+    const int avg = (rp[row0 + nr] - k0 + nr - 1) / nr;
+    int S = 1;
+    while (S * L < WAVE && 16 * S < avg) S <<= 1;
+    const int sub = gid & (S - 1), RG = G / S, rg = gid / S;
+    __syncthreads();
+    for (int r0 = 0; r0 < nl; r0 += RG) {  // same trip count for the whole workgroup
+      const int r = r0 + rg;
+      const bool ok = r < nl, mine = ok && sub == 0;
+      const int64_t row = row0 + ra + r;
+      typename Epi::template Pre<VW> pre;
+      if (mine) pre = epi.template load<VW>(row, c0);
 #pragma unroll
       for (int v = 0; v < VW; v++) s[v] = 0;
-      int j = a;
-      for (; j + U - 1 < b; j += U) {  // U independent gathers in flight
-        int cc[U];
-        double vv[U];
-        V xx[U];
+      if (ok) add(s, soff[r] + sub, soff[r + 1], S);
+      for (int off = L * S >> 1; off >= L; off >>= 1)
 #pragma unroll
-        for (int t = 0; t < U; t++) {
-          cc[t] = ci[j + t];
-          vv[t] = (double)val(j + t);
-        }
-#pragma unroll
-        for (int t = 0; t < U; t++) xx[t] = *(const V *)(X + (int64_t)cc[t] * kp + c0);
-#pragma unroll
-        for (int t = 0; t < U; t++)
-#pragma unroll
-          for (int v = 0; v < VW; v++) s[v] += vv[t] * bvec_at<T, VW>(xx[t], v);
-      }
-      for (; j < b; j++) {
-        const double vj = (double)val(j);
-        const V xj = *(const V *)(X + (int64_t)ci[j] * kp + c0);
-#pragma unroll
-        for (int v = 0; v < VW; v++) s[v] += vj * bvec_at<T, VW>(xj, v);
-      }
-#pragma unroll
-      for (int v = 0; v < VW; v++) epi(row, c0 + v, s[v]);
+        for (int v = 0; v < VW; v++) s[v] += __shfl_xor(s[v], off, WAVE);
+      if (mine) epi.template store<VW>(row, c0, s, pre);
     }
   } else {
-    const int G = 256 >> lk;
-    const int g = threadIdx.x >> lk, c = threadIdx.x & (kp - 1);
-    __shared__ double red[256];
-    const int row = row0;
-    const int cnt = min(k0 + UNIT_NNZ, rp[row + 1]) - k0;
-    double s = 0;
-    for (int t = g; t < cnt; t += G) {
-      const int j = k0 + t;
-      s += (double)val(j) * (double)X[(int64_t)ci[j] * kp + c];
-    }
-    red[threadIdx.x] = s;
+    if (blockIdx.y > 0) return;
+    const int cnt = min(k0 + UNIT_NNZ, rp[row0 + 1]) - k0;
+    stage(k0, cnt);
     __syncthreads();
-    if (g == 0) {
-      for (int gg = 1; gg < G; gg++) s += red[gg * kp + c];
-      parts[(int64_t)(-nr) * kp + c] = s;
+#pragma unroll
+    for (int v = 0; v < VW; v++) s[v] = 0;
+    add(s, gid, cnt, G);
+    for (int off = WAVE >> 1; off >= L; off >>= 1)
+#pragma unroll
+      for (int v = 0; v < VW; v++) s[v] += __shfl_xor(s[v], off, WAVE);
+    const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+    if (lane < L)
+#pragma unroll
+      for (int v = 0; v < VW; v++) red[w][c0 + v] = s[v];
+    __syncthreads();
+    if ((int)threadIdx.x < kp) {
+      double t = 0;
+      for (int q = 0; q < 256 / WAVE; q++) t += red[q][threadIdx.x];
+      parts[(int64_t)(-nr) * kp + threadIdx.x] = t;
     }
   }
 }
@@ -175,7 +288,7 @@ __global__ void k_spmm_long(const int32_t *lrow, const int32_t *lpart, int64_t n
     const int c = (int)(t % kp);
     double s = 0;
     for (int p = lpart[j]; p < lpart[j + 1]; p++) s += parts[(int64_t)p * kp + c];
-    epi(lrow[j], c, s);
+    epi.template store<1>(lrow[j], c, &s, epi.template load<1>(lrow[j], c));
   }
 }
 
@@ -196,35 +309,39 @@ const float *bvals<float>(const DCsr &A) {
   return A.v32.p;
 }
 
-// SpMM tiles (right-hand sides per lane VW, gathers in flight U) by id;
-// id 0 is the fixed tile.  VW never exceeds the block width kp.
-constexpr int SPMM_NCFG = 6;
-constexpr int SPMM_VW[SPMM_NCFG] = {1, 1, 2, 2, 4, 4};
-constexpr int SPMM_U[SPMM_NCFG] = {2, 4, 2, 4, 2, 4};
+// SpMM tiles: gathers in flight U by id.  A lane holds 16 bytes of a row of
+// X (4 FP32 or 2 FP64 right-hand sides), or the whole row of a narrower block.
+constexpr int SPMM_NCFG = 2;
+constexpr int SPMM_U[SPMM_NCFG] = {4, 8};
 
 template <class T>
 constexpr int prec_slot() {
   return std::is_same<T, float>::value ? 1 : 0;
 }
-
-template <class T, int VW, int U, class Val, class Epi>
-void launch_spmm_tile(const DCsr &A, Val val, const T *X, int kp, Epi epi, double *parts, hipStream_t s) {
-  hipLaunchKernelGGL((k_spmm_units<T, VW, U, Val, Epi>), dim3((unsigned)A.U.nunits), dim3(256), 0, s, A.rp.p,
-                     A.ci.p, val, X, kp, log2i(kp), A.U.row0.p, A.U.nrows.p, A.U.koff.p, parts, epi);
-  LG_LAUNCH_CHECK();
+template <class T>
+constexpr int spmm_vw(int kp) {
+  return std::min<int>(16 / (int)sizeof(T), kp);
+}
+// the tile without timing: rows that one round of 4 gathers covers take 4
+inline int spmm_rule(const DCsr &A) { return A.nnz <= 4 * A.n ? 0 : 1; }
+// parts of a unit's rows: operators of few units spread over the CUs
+inline unsigned spmm_parts(int64_t nunits) {
+  unsigned y = 1;
+  while (nunits * y < 1024 && y < 16) y <<= 1;
+  return y;
 }
 
-template <class T, class Val, class Epi>
-void launch_spmm_cfg(int cfg, const DCsr &A, Val val, const T *X, int kp, Epi epi, DevBuf<double> &parts,
-                     hipStream_t s) {
-  switch (cfg) {
-    case 1: launch_spmm_tile<T, 1, 4>(A, val, X, kp, epi, parts.p, s); break;
-    case 2: launch_spmm_tile<T, 2, 2>(A, val, X, kp, epi, parts.p, s); break;
-    case 3: launch_spmm_tile<T, 2, 4>(A, val, X, kp, epi, parts.p, s); break;
-    case 4: launch_spmm_tile<T, 4, 2>(A, val, X, kp, epi, parts.p, s); break;
-    case 5: launch_spmm_tile<T, 4, 4>(A, val, X, kp, epi, parts.p, s); break;
-    default: launch_spmm_tile<T, 1, 2>(A, val, X, kp, epi, parts.p, s); break;
-  }
+template <class T, int VW, class Val, class Epi>
+void launch_spmm_vw(int cfg, const DCsr &A, Val val, const T *X, int kp, Epi epi, double *parts, hipStream_t s) {
+  const dim3 grid((unsigned)A.U.nunits, spmm_parts(A.U.nunits));
+  const int lg = log2i(kp / VW);
+  if (cfg == 0)
+    hipLaunchKernelGGL((k_spmm_units<T, VW, 4, Val, Epi>), grid, dim3(256), 0, s, A.rp.p, A.ci.p, val, X, kp, lg,
+                       A.U.row0.p, A.U.nrows.p, A.U.koff.p, parts, epi);
+  else
+    hipLaunchKernelGGL((k_spmm_units<T, VW, 8, Val, Epi>), grid, dim3(256), 0, s, A.rp.p, A.ci.p, val, X, kp, lg,
+                       A.U.row0.p, A.U.nrows.p, A.U.koff.p, parts, epi);
+  LG_LAUNCH_CHECK();
 }
 
 template <class T, class Val, class Epi>
@@ -234,8 +351,13 @@ void launch_spmm(const DCsr &A, Val val, const T *X, int kp, Epi epi, DevBuf<dou
   LG_CHECK(parts.n >= (size_t)std::max<int64_t>(A.U.nparts, 1) * kp, LIGMG_ERR_INVALID,
            "spmm partial-sum buffer too small");
   int cfg = A.U.spmm_cfg[prec_slot<T>()][log2i(kp)];
-  if (cfg < 0 || SPMM_VW[cfg] > kp) cfg = 0;
-  launch_spmm_cfg<T>(cfg, A, val, X, kp, epi, parts, s);
+  if (cfg < 0) cfg = spmm_rule(A);
+  switch (spmm_vw<T>(kp)) {
+    case 1: launch_spmm_vw<T, 1>(cfg, A, val, X, kp, epi, parts.p, s); break;
+    case 2: launch_spmm_vw<T, 2>(cfg, A, val, X, kp, epi, parts.p, s); break;
+    default:
+      if constexpr (sizeof(T) == 4) launch_spmm_vw<T, 4>(cfg, A, val, X, kp, epi, parts.p, s);
+  }
   if (A.U.nlong) {
     hipLaunchKernelGGL((k_spmm_long<Epi>), dim3(grid_for(A.U.nlong * kp, 256)), dim3(256), 0, s,
                        A.U.lrow.p, A.U.lpart.p, A.U.nlong, kp, (const double *)parts.p, epi);
@@ -357,118 +479,293 @@ __global__ void __launch_bounds__(256) k_dense_mfma(const double *__restrict__ P
   }
 }
 
-template <class T>
-__global__ void k_dense_small(const double *__restrict__ Pm, int64_t n, const T *__restrict__ X,
-                              int kp, T *__restrict__ Y) {
-  // kp < 16: one thread per output entry
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n * kp;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t i = t / kp;
-    const int c = (int)(t % kp);
-    double s = 0;
-    for (int64_t j = 0; j < n; j++) s += Pm[i * n + j] * (double)X[j * kp + c];
-    Y[t] = (T)s;
+// kp < 16: one wavefront per row of the matrix, KP sums per lane.  (One
+// thread per output walked the row alone: 24 us for 157 x 157 x 4, 3.8 us now.)
+template <class T, int KP>
+__global__ void __launch_bounds__(256) k_dense_small(const double *__restrict__ Pm, int64_t n,
+                                                     const T *__restrict__ X, T *__restrict__ Y) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int64_t i = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / WAVE;
+  if (i >= n) return;  // the whole wavefront
+  double s[KP] = {};
+#pragma unroll 4
+  for (int64_t j = lane; j < n; j += WAVE) {
+    const double a = Pm[i * n + j];
+#pragma unroll
+    for (int c = 0; c < KP; c++) s[c] += a * (double)X[j * KP + c];
+  }
+#pragma unroll
+  for (int c = 0; c < KP; c++) {
+    s[c] = sdev::wave_sum(s[c]);
+    if (lane == 0) Y[i * KP + c] = (T)s[c];
   }
 }
 
 // -------------------------------------------------- per-(block, column) dots
-// part[(s * np + j) * kp + c] for segment s; out[(blk * np + j) * kp + c]
-template <class T>
-__global__ void __launch_bounds__(256) k_bred1(int np, int kp, int lk, const T *a0, const T *b0,
-                                               const T *a1, const T *b1, const int64_t *lo,
-                                               const int64_t *hi, double *part) {
-  const int s = blockIdx.x;
-  const int G = 256 >> lk;
-  const int g = threadIdx.x >> lk, c = threadIdx.x & (kp - 1);
-  double acc0 = 0, acc1 = 0;
-  for (int64_t i = lo[s] + g; i < hi[s]; i += G) {
-    const int64_t o = i * kp + c;
-    acc0 += (double)a0[o] * (b0 ? (double)b0[o] : 1.0);
-    if (np > 1) acc1 += (double)a1[o] * (b1 ? (double)b1[o] : 1.0);
+// The vector passes below take a segment of rows per workgroup
+// (RedPlan::build with block_seg_rows(kp) rows) and VW = 2 adjacent columns
+// per thread (1 when kp = 1), four rows in flight.  With 4096-row segments and
+// 8-byte accesses a 10^6 x 32 block had 245 workgroups, less than one per CU:
+// the update took 852 us for 1.73 GB (2.0 TB/s), now 305 us (5.7 TB/s, part
+// of it from the Infinity Cache).
+
+// this workgroup's rows [lo, hi); the thread takes rows lo + g, lo + g + G,
+// ... and columns c .. c + VW - 1
+template <int VW>
+struct BSeg {
+  int64_t lo, hi;
+  int G, g, c;
+  __device__ __forceinline__ BSeg(int64_t l, int64_t h, int kp) : lo(l), hi(h) {
+    const int L = kp / VW;  // a power of two
+    G = 256 / L;
+    g = threadIdx.x / L;
+    c = (threadIdx.x & (L - 1)) * VW;
   }
-  __shared__ double red[2][256];
-  red[0][threadIdx.x] = acc0;
-  red[1][threadIdx.x] = acc1;
+};
+
+// sums of the workgroup's per-thread partials: part[c + v], columns combined
+// over the row groups in order
+template <int VW>
+__device__ __forceinline__ void bseg_sum(const BSeg<VW> &B, int kp, const double *acc, double (*red)[256],
+                                         double *part) {
+#pragma unroll
+  for (int v = 0; v < VW; v++) red[v][threadIdx.x] = acc[v];
   __syncthreads();
-  if (g == 0) {
-    for (int j = 0; j < np; j++) {
+  if (B.g == 0) {
+    const int L = kp / VW;
+#pragma unroll
+    for (int v = 0; v < VW; v++) {
       double t = 0;
-      for (int gg = 0; gg < G; gg++) t += red[j][gg * kp + c];
-      part[((int64_t)s * np + j) * kp + c] = t;
+      for (int gg = 0; gg < B.G; gg++) t += red[v][gg * L + threadIdx.x];
+      part[B.c + v] = t;
     }
   }
+  __syncthreads();
+}
+
+// part[(s * np + j) * kp + c] for segment s; out[(blk * np + j) * kp + c]
+template <class T, int VW>
+__global__ void __launch_bounds__(256) k_bred1(int np, int kp, const T *a0, const T *b0, const T *a1, const T *b1,
+                                               const int64_t *lo, const int64_t *hi, double *part) {
+  const int s = blockIdx.x;
+  const BSeg<VW> B(lo[s], hi[s], kp);
+  double acc0[VW] = {}, acc1[VW] = {};
+  for (int64_t i = B.lo + B.g; i < B.hi; i += 4 * B.G) {
+    typename BVec<T, VW>::type x0[4], y0[4], x1[4], y1[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const int64_t o = min(i + t * B.G, B.hi - 1) * kp + B.c;
+      x0[t] = bvec_load<T, VW>(a0 + o);
+      if (b0) y0[t] = bvec_load<T, VW>(b0 + o);
+      if (np > 1) {
+        x1[t] = a1 == a0 ? x0[t] : bvec_load<T, VW>(a1 + o);
+        if (b1) y1[t] = bvec_load<T, VW>(b1 + o);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+      if (i + t * B.G < B.hi)
+#pragma unroll
+        for (int v = 0; v < VW; v++) {
+          acc0[v] += bvec_at<T, VW>(x0[t], v) * (b0 ? bvec_at<T, VW>(y0[t], v) : 1.0);
+          if (np > 1) acc1[v] += bvec_at<T, VW>(x1[t], v) * (b1 ? bvec_at<T, VW>(y1[t], v) : 1.0);
+        }
+  }
+  __shared__ double red[VW][256];
+  bseg_sum<VW>(B, kp, acc0, red, part + (int64_t)s * np * kp);
+  if (np > 1) bseg_sum<VW>(B, kp, acc1, red, part + ((int64_t)s * np + 1) * kp);
 }
 
 // out[blk, j, c] = sum of the segment partials of block blk: one workgroup
-// per (block, j); thread (g, c) adds segments g, g + G, ... (G = 256 / kp)
+// per (block, j); thread (g, c) adds segments g, g + G, ... (G = 1024 / kp)
 // in order, and the G partials of a column are added in g order.
-__global__ void __launch_bounds__(256) k_bred2(int np, int kp, int lk, const int32_t *bseg, const double *part,
-                                               double *out) {
+__global__ void __launch_bounds__(1024) k_bred2(int np, int kp, int lk, const int32_t *bseg, const double *part,
+                                                double *out) {
   const int blk = blockIdx.x, j = blockIdx.y;
-  const int G = 256 >> lk;
+  const int G = 1024 >> lk;
   const int g = threadIdx.x >> lk, c = threadIdx.x & (kp - 1);
   double acc = 0;
-  for (int sg = bseg[blk] + g; sg < bseg[blk + 1]; sg += G) acc += part[((int64_t)sg * np + j) * kp + c];
-  __shared__ double red[256];
+  const int end = bseg[blk + 1];
+#pragma unroll 8
+  for (int sg = bseg[blk] + g; sg < end; sg += G) acc += part[((int64_t)sg * np + j) * kp + c];
+  __shared__ double red[1024];
   red[threadIdx.x] = acc;
   __syncthreads();
-  if (g == 0) {
+  // 16 partials a thread, then the rest in order
+  for (int n = G; n > 1; n = (n + 15) / 16) {
+    const int m = (n + 15) / 16;
     double t = 0;
-    for (int gg = 0; gg < G; gg++) t += red[gg * kp + c];
-    out[((int64_t)blk * np + j) * kp + c] = t;
+    if (g < m)
+      for (int q = 16 * g; q < min(16 * g + 16, n); q++) t += red[q * kp + c];
+    __syncthreads();
+    if (g < m) red[threadIdx.x] = t;
+    __syncthreads();
   }
+  if (g == 0) out[((int64_t)blk * np + j) * kp + c] = red[c];
 }
 
-template <class T>
-__global__ void __launch_bounds__(256) k_bsub_mean(T *a, int kp, int lk, const int64_t *lo,
-                                                   const int64_t *hi, const int32_t *segblk,
-                                                   const int64_t *bptr, const double *sums) {
+template <class T, int VW>
+__global__ void __launch_bounds__(256) k_bsub_mean(T *a, int kp, const int64_t *lo, const int64_t *hi,
+                                                   const int32_t *segblk, const int64_t *bptr, const double *sums) {
   const int s = blockIdx.x;
   const int blk = segblk[s];
-  const int G = 256 >> lk;
-  const int g = threadIdx.x >> lk, c = threadIdx.x & (kp - 1);
-  const T m = (T)(sums[(int64_t)blk * kp + c] / (double)(bptr[blk + 1] - bptr[blk]));
-  for (int64_t i = lo[s] + g; i < hi[s]; i += G) a[i * kp + c] -= m;
+  const BSeg<VW> B(lo[s], hi[s], kp);
+  T m[VW];
+#pragma unroll
+  for (int v = 0; v < VW; v++) m[v] = (T)(sums[(int64_t)blk * kp + B.c + v] / (double)(bptr[blk + 1] - bptr[blk]));
+#pragma unroll 4
+  for (int64_t i = B.lo + B.g; i < B.hi; i += B.G) {
+    const typename BVec<T, VW>::type x = bvec_load<T, VW>(a + i * kp + B.c);
+    bvec_store<T, VW>(a + i * kp + B.c, [&](int v) {
+      if constexpr (VW == 1) return x - m[0];
+      else return x[v] - m[v];
+    });
+  }
 }
 
 // z = c - (block mean), in FP64; with w set, also the segment partials of
-// z.w exactly as the block dots form them (part[s * kp + c])
-__global__ void __launch_bounds__(256) k_bsub_mean_f2d(double *z, const float *cv, int kp, int lk,
-                                                       const int64_t *lo, const int64_t *hi,
-                                                       const int32_t *segblk, const int64_t *bptr,
-                                                       const double *sums, const double *w, double *part) {
+// z.w as the block dots form them (part[s * kp + c])
+template <int VW>
+__global__ void __launch_bounds__(256) k_bsub_mean_f2d(double *z, const float *cv, int kp, const int64_t *lo,
+                                                       const int64_t *hi, const int32_t *segblk,
+                                                       const int64_t *bptr, const double *sums, const double *w,
+                                                       double *part) {
   const int s = blockIdx.x;
   const int blk = segblk[s];
-  const int G = 256 >> lk;
-  const int g = threadIdx.x >> lk, c = threadIdx.x & (kp - 1);
-  const double m = sums[(int64_t)blk * kp + c] / (double)(bptr[blk + 1] - bptr[blk]);
-  double acc = 0;
-  for (int64_t i = lo[s] + g; i < hi[s]; i += G) {
-    const int64_t o = i * kp + c;
-    const double zv = (double)cv[o] - m;
-    z[o] = zv;
-    if (w) acc += zv * w[o];
+  const BSeg<VW> B(lo[s], hi[s], kp);
+  double m[VW], acc[VW] = {};
+#pragma unroll
+  for (int v = 0; v < VW; v++) m[v] = sums[(int64_t)blk * kp + B.c + v] / (double)(bptr[blk + 1] - bptr[blk]);
+  for (int64_t i = B.lo + B.g; i < B.hi; i += 4 * B.G) {
+    typename BVec<float, VW>::type x[4];
+    typename BVec<double, VW>::type y[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const int64_t o = min(i + t * B.G, B.hi - 1) * kp + B.c;
+      x[t] = bvec_load<float, VW>(cv + o);
+      if (w) y[t] = bvec_load<double, VW>(w + o);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      if (i + t * B.G >= B.hi) continue;
+      double zv[VW];
+#pragma unroll
+      for (int v = 0; v < VW; v++) {
+        zv[v] = bvec_at<float, VW>(x[t], v) - m[v];
+        if (w) acc[v] += zv[v] * bvec_at<double, VW>(y[t], v);
+      }
+      bvec_store<double, VW>(z + (i + t * B.G) * kp + B.c, [&](int v) { return zv[v]; });
+    }
   }
   if (!w) return;  // uniform over the workgroup
-  __shared__ double red[256];
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  if (g == 0) {
-    double t = 0;
-    for (int gg = 0; gg < G; gg++) t += red[gg * kp + c];
-    part[(int64_t)s * kp + c] = t;
+  __shared__ double red[VW][256];
+  bseg_sum<VW>(B, kp, acc, red, part + (int64_t)s * kp);
+}
+
+// x += alpha p, r -= alpha q per (block, column); alpha = 0 marks a finished
+// column, whose x and r stay.  Also writes the segment partials of r.r as
+// the block dots form them (part[s * kp + c]), and r in FP32 when r32 is set
+// (the mixed outer preconditioner's input).
+template <class T, int VW>
+__global__ void __launch_bounds__(256) k_kr_bupdate(T *x, T *r, const T *p, const T *q, int kp, const int64_t *lo,
+                                                    const int64_t *hi, const int32_t *segblk, const double *sc,
+                                                    double *part, float *r32) {
+  const int s = blockIdx.x;
+  const BSeg<VW> B(lo[s], hi[s], kp);
+  T at[VW];
+  bool any = false;
+  double acc[VW] = {};
+#pragma unroll
+  for (int v = 0; v < VW; v++) {
+    const double a = sc[((int64_t)segblk[s] * kp + B.c + v) * sdev::SC_N + sdev::SC_ALPHA];
+    at[v] = (T)a;
+    any |= a != 0.0;
+  }
+  typedef typename BVec<T, VW>::type V;
+  for (int64_t i = B.lo + B.g; i < B.hi; i += 4 * B.G) {
+    V xv[4], rv[4], pv[4], qv[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const int64_t o = min(i + t * B.G, B.hi - 1) * kp + B.c;
+      rv[t] = bvec_load<T, VW>(r + o);
+      if (any) {
+        xv[t] = bvec_load<T, VW>(x + o);
+        pv[t] = bvec_load<T, VW>(p + o);
+        qv[t] = bvec_load<T, VW>(q + o);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      if (i + t * B.G >= B.hi) continue;
+      const int64_t o = (i + t * B.G) * kp + B.c;
+      T xn[VW], rn[VW];
+#pragma unroll
+      for (int v = 0; v < VW; v++) {
+        if constexpr (VW == 1) {
+          rn[v] = any ? rv[t] - at[v] * qv[t] : rv[t];
+          if (any) xn[v] = xv[t] + at[v] * pv[t];
+        } else {
+          // a finished column of a pair keeps its bits (alpha p may not be 0)
+          const bool on = any && at[v] != (T)0;
+          rn[v] = on ? rv[t][v] - at[v] * qv[t][v] : rv[t][v];
+          if (any) xn[v] = on ? xv[t][v] + at[v] * pv[t][v] : xv[t][v];
+        }
+        acc[v] += (double)rn[v] * (double)rn[v];
+      }
+      if (any) {
+        bvec_store<T, VW>(x + o, [&](int v) { return xn[v]; });
+        bvec_store<T, VW>(r + o, [&](int v) { return rn[v]; });
+      }
+      if (r32) bvec_store<float, VW>(r32 + o, [&](int v) { return (float)rn[v]; });
+    }
+  }
+  __shared__ double red[VW][256];
+  bseg_sum<VW>(B, kp, acc, red, part + (int64_t)s * kp);
+}
+
+// p = z + beta p
+template <class T, int VW>
+__global__ void __launch_bounds__(256) k_kr_bpupdate(T *p, const T *z, int kp, const int64_t *lo, const int64_t *hi,
+                                                     const int32_t *segblk, const double *sc) {
+  const int s = blockIdx.x;
+  const BSeg<VW> B(lo[s], hi[s], kp);
+  T bt[VW];
+#pragma unroll
+  for (int v = 0; v < VW; v++)
+    bt[v] = (T)sc[((int64_t)segblk[s] * kp + B.c + v) * sdev::SC_N + sdev::SC_BETA];
+  typedef typename BVec<T, VW>::type V;
+  for (int64_t i = B.lo + B.g; i < B.hi; i += 4 * B.G) {
+    V pv[4], zv[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const int64_t o = min(i + t * B.G, B.hi - 1) * kp + B.c;
+      pv[t] = bvec_load<T, VW>(p + o);
+      zv[t] = bvec_load<T, VW>(z + o);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+      if (i + t * B.G < B.hi)
+        bvec_store<T, VW>(p + (i + t * B.G) * kp + B.c, [&](int v) {
+          if constexpr (VW == 1) return zv[t] + bt[0] * pv[t];
+          else return zv[t][v] + bt[v] * pv[t][v];
+        });
   }
 }
 
 }  // namespace
 
 // ---------------------------------------------------------------- host side
-// Times every tile that fits kp on A (the operator's own values and
+// Operators of less work than this take the rule's tile: timing it costs
+// more than a wrong pick over a solve.
+constexpr int64_t SPMM_TUNE_MIN = (int64_t)32 << 20;
+
+// Times every tile on A (the operator's own values and
 // Laplacian-form diagonal, X of zeros, a plain store) and records the
 // fastest for this precision and width; a tile already picked is kept.
 template <class T>
 int tune_spmm(DCsr &A, int kp, DevBuf<double> &parts, hipStream_t s) {
   int8_t &pick = A.U.spmm_cfg[prec_slot<T>()][log2i(kp)];
+  if (pick < 0 && A.nnz * kp < SPMM_TUNE_MIN) pick = (int8_t)spmm_rule(A);
   if (pick >= 0 || A.U.nunits == 0) return pick < 0 ? 0 : pick;
   DevBuf<T> X((size_t)std::max<int64_t>(A.ncols, 1) * kp), Y((size_t)std::max<int64_t>(A.n, 1) * kp);
   fill_u8((uint8_t *)X.p, 0, (int64_t)X.bytes(), s);
@@ -478,7 +775,6 @@ int tune_spmm(DCsr &A, int kp, DevBuf<double> &parts, hipStream_t s) {
   float best = 0;
   int besti = 0;
   for (int c = 0; c < SPMM_NCFG; c++) {
-    if (SPMM_VW[c] > kp) continue;
     A.U.spmm_cfg[prec_slot<T>()][log2i(kp)] = (int8_t)c;
     op_bspmv<T>(A, X.p, Y.p, kp, parts, s);  // warm
     LG_HIP(hipEventRecord(e0, s));
@@ -498,10 +794,7 @@ int tune_spmm(DCsr &A, int kp, DevBuf<double> &parts, hipStream_t s) {
   return besti;
 }
 
-void spmm_tile(int cfg, int *vw, int *u) {
-  *vw = SPMM_VW[cfg];
-  *u = SPMM_U[cfg];
-}
+void spmm_tile(int cfg, int *u) { *u = SPMM_U[cfg]; }
 
 template <class T>
 void op_bspmv(const DCsr &A, const T *X, T *Y, int kp, DevBuf<double> &parts, hipStream_t s) {
@@ -544,8 +837,15 @@ void op_bdense_apply(const double *Pm, int64_t n, const T *X, T *Y, int kp, hipS
     else if (kp == 32) hipLaunchKernelGGL((k_dense_mfma<T, 2>), dim3(g), dim3(256), 0, s, Pm, (int)n, X, kp, Q, Y);
     else hipLaunchKernelGGL((k_dense_mfma<T, 4>), dim3(g), dim3(256), 0, s, Pm, (int)n, X, kp, Q, Y);
   } else {
-    hipLaunchKernelGGL(k_dense_small<T>, dim3(grid_for(n * kp, 256, 16384)), dim3(256), 0, s, Pm, n, X,
-                       kp, Y);
+    const dim3 g((unsigned)((n + 3) / 4));
+    switch (kp) {
+      case 1: hipLaunchKernelGGL((k_dense_small<T, 1>), g, dim3(256), 0, s, Pm, n, X, Y); break;
+      case 2: hipLaunchKernelGGL((k_dense_small<T, 2>), g, dim3(256), 0, s, Pm, n, X, Y); break;
+      case 4: hipLaunchKernelGGL((k_dense_small<T, 4>), g, dim3(256), 0, s, Pm, n, X, Y); break;
+      default:
+        LG_CHECK(kp == 8, LIGMG_ERR_INVALID, "dense apply: kp must be a power of two");
+        hipLaunchKernelGGL((k_dense_small<T, 8>), g, dim3(256), 0, s, Pm, n, X, Y);
+    }
   }
   LG_LAUNCH_CHECK();
 }
@@ -566,18 +866,20 @@ void RedPlan::bdots(int np, int kp, const T *a0, const T *b0, const T *a1, const
                     DevBuf<double> &bpart, hipStream_t s) const {
   if (nseg == 0) return;
   LG_CHECK(bpart.n >= (size_t)nseg * np * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
-  hipLaunchKernelGGL(k_bred1<T>, dim3(nseg), dim3(256), 0, s, np, kp, log2i(kp), a0, b0, a1, b1, seg_lo.p,
-                     seg_hi.p, bpart.p);
+  if (kp == 1)
+    hipLaunchKernelGGL((k_bred1<T, 1>), dim3(nseg), dim3(256), 0, s, np, kp, a0, b0, a1, b1, seg_lo.p, seg_hi.p,
+                       bpart.p);
+  else
+    hipLaunchKernelGGL((k_bred1<T, 2>), dim3(nseg), dim3(256), 0, s, np, kp, a0, b0, a1, b1, seg_lo.p, seg_hi.p,
+                       bpart.p);
   LG_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_bred2, dim3((unsigned)nb, (unsigned)np), dim3(256), 0, s, np, kp, log2i(kp), bseg.p, bpart.p,
-                     out);
-  LG_LAUNCH_CHECK();
+  bdots_finish(np, kp, out, bpart, s);
 }
 
 void RedPlan::bdots_finish(int np, int kp, double *out, const DevBuf<double> &bpart, hipStream_t s) const {
   if (nseg == 0) return;
   LG_CHECK(bpart.n >= (size_t)nseg * np * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
-  hipLaunchKernelGGL(k_bred2, dim3((unsigned)nb, (unsigned)np), dim3(256), 0, s, np, kp, log2i(kp), bseg.p, bpart.p,
+  hipLaunchKernelGGL(k_bred2, dim3((unsigned)nb, (unsigned)np), dim3(1024), 0, s, np, kp, log2i(kp), bseg.p, bpart.p,
                      out);
   LG_LAUNCH_CHECK();
 }
@@ -586,16 +888,50 @@ void op_bsub_block_mean_f2d(double *z, const float *c, int kp, const RedPlan &P,
                             const double *w, DevBuf<double> *bpart) {
   if (P.nseg == 0) return;
   if (w) LG_CHECK(bpart && bpart->n >= (size_t)P.nseg * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
-  hipLaunchKernelGGL(k_bsub_mean_f2d, dim3(P.nseg), dim3(256), 0, s, z, c, kp, log2i(kp), P.seg_lo.p, P.seg_hi.p,
-                     P.bseg.p + P.nb + 1, P.bptr.p, sums, w, w ? bpart->p : nullptr);
+  if (kp == 1)
+    hipLaunchKernelGGL(k_bsub_mean_f2d<1>, dim3(P.nseg), dim3(256), 0, s, z, c, kp, P.seg_lo.p, P.seg_hi.p,
+                       P.bseg.p + P.nb + 1, P.bptr.p, sums, w, w ? bpart->p : nullptr);
+  else
+    hipLaunchKernelGGL(k_bsub_mean_f2d<2>, dim3(P.nseg), dim3(256), 0, s, z, c, kp, P.seg_lo.p, P.seg_hi.p,
+                       P.bseg.p + P.nb + 1, P.bptr.p, sums, w, w ? bpart->p : nullptr);
   LG_LAUNCH_CHECK();
 }
 
 template <class T>
 void op_bsub_block_mean(T *a, int kp, const RedPlan &P, const double *sums, hipStream_t s) {
   if (P.nseg == 0) return;
-  hipLaunchKernelGGL(k_bsub_mean<T>, dim3(P.nseg), dim3(256), 0, s, a, kp, log2i(kp), P.seg_lo.p,
-                     P.seg_hi.p, P.bseg.p + P.nb + 1, P.bptr.p, sums);
+  if (kp == 1)
+    hipLaunchKernelGGL((k_bsub_mean<T, 1>), dim3(P.nseg), dim3(256), 0, s, a, kp, P.seg_lo.p, P.seg_hi.p,
+                       P.bseg.p + P.nb + 1, P.bptr.p, sums);
+  else
+    hipLaunchKernelGGL((k_bsub_mean<T, 2>), dim3(P.nseg), dim3(256), 0, s, a, kp, P.seg_lo.p, P.seg_hi.p,
+                       P.bseg.p + P.nb + 1, P.bptr.p, sums);
+  LG_LAUNCH_CHECK();
+}
+
+template <class T>
+void op_kr_bupdate(T *x, T *r, const T *p, const T *q, int kp, const RedPlan &P, const double *sc,
+                   DevBuf<double> &bpart, float *r32, hipStream_t s) {
+  if (P.nseg == 0) return;
+  LG_CHECK(bpart.n >= (size_t)P.nseg * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
+  if (kp == 1)
+    hipLaunchKernelGGL((k_kr_bupdate<T, 1>), dim3(P.nseg), dim3(256), 0, s, x, r, p, q, kp, P.seg_lo.p, P.seg_hi.p,
+                       P.bseg.p + P.nb + 1, sc, bpart.p, r32);
+  else
+    hipLaunchKernelGGL((k_kr_bupdate<T, 2>), dim3(P.nseg), dim3(256), 0, s, x, r, p, q, kp, P.seg_lo.p, P.seg_hi.p,
+                       P.bseg.p + P.nb + 1, sc, bpart.p, r32);
+  LG_LAUNCH_CHECK();
+}
+
+template <class T>
+void op_kr_bpupdate(T *p, const T *z, int kp, const RedPlan &P, const double *sc, hipStream_t s) {
+  if (P.nseg == 0) return;
+  if (kp == 1)
+    hipLaunchKernelGGL((k_kr_bpupdate<T, 1>), dim3(P.nseg), dim3(256), 0, s, p, z, kp, P.seg_lo.p, P.seg_hi.p,
+                       P.bseg.p + P.nb + 1, sc);
+  else
+    hipLaunchKernelGGL((k_kr_bpupdate<T, 2>), dim3(P.nseg), dim3(256), 0, s, p, z, kp, P.seg_lo.p, P.seg_hi.p,
+                       P.bseg.p + P.nb + 1, sc);
   LG_LAUNCH_CHECK();
 }
 
@@ -612,7 +948,10 @@ void op_bsub_block_mean(T *a, int kp, const RedPlan &P, const double *sums, hipS
   template void op_bdense_apply<T>(const double *, int64_t, const T *, T *, int, hipStream_t);       \
   template void RedPlan::bdots<T>(int, int, const T *, const T *, const T *, const T *, double *,    \
                                   DevBuf<double> &, hipStream_t) const;                              \
-  template void op_bsub_block_mean<T>(T *, int, const RedPlan &, const double *, hipStream_t);
+  template void op_bsub_block_mean<T>(T *, int, const RedPlan &, const double *, hipStream_t);         \
+  template void op_kr_bupdate<T>(T *, T *, const T *, const T *, int, const RedPlan &, const double *,  \
+                                 DevBuf<double> &, float *, hipStream_t);                            \
+  template void op_kr_bpupdate<T>(T *, const T *, int, const RedPlan &, const double *, hipStream_t);
 LG_BINST(double)
 LG_BINST(float)
 #undef LG_BINST

@@ -3,6 +3,8 @@
 // float); matrix values are read in the same precision (A.v or A.v32), or
 // as 1 for pattern-only operators.
 #pragma once
+#include <algorithm>
+
 #include "hierarchy.hpp"
 
 namespace lg {
@@ -59,7 +61,8 @@ struct RedPlan {
   DevBuf<int64_t> bptr;            // nb + 1 block offsets
   mutable DevBuf<double> part;     // nseg * 4
   std::vector<int64_t> hbptr;
-  void build(int64_t n, const std::vector<int64_t> &blocks, hipStream_t s);
+  // segments of at most seg_rows rows (0: the vector dots' length)
+  void build(int64_t n, const std::vector<int64_t> &blocks, hipStream_t s, int64_t seg_rows = 0);
   // out[c*np + j] = sum over block c of a_j[i] * b_j[i] (b_j == nullptr:
   // 1), j < np (np <= 4), accumulated in FP64.
   template <class T>
@@ -93,8 +96,8 @@ void op_bspmv(const DCsr &A, const T *X, T *Y, int kp, DevBuf<double> &parts, hi
 // the candidates once (kept in A.U); returns the tile id
 template <class T>
 int tune_spmm(DCsr &A, int kp, DevBuf<double> &parts, hipStream_t s);
-// right-hand sides per lane and gathers in flight of tile id cfg
-void spmm_tile(int cfg, int *vw, int *u);
+// gathers in flight of tile id cfg
+void spmm_tile(int cfg, int *u);
 template <class T>
 void op_bresidual(const DCsr &A, const T *X, const T *B, T *R, int kp, DevBuf<double> &parts,
                   hipStream_t s);
@@ -117,6 +120,20 @@ void op_bsub_block_mean(T *a, int kp, const RedPlan &P, const double *sums, hipS
 // bdots_finish).
 void op_bsub_block_mean_f2d(double *z, const float *c, int kp, const RedPlan &P, const double *sums, hipStream_t s,
                             const double *w = nullptr, DevBuf<double> *bpart = nullptr);
+// Rows of a block vector's segment: 8192 entries, 16 pairs for each of a
+// workgroup's 256 threads, at most the vector dots' 4096 rows; longer where
+// there would be more than 2048 segments, whose partials one workgroup adds.
+inline int64_t block_seg_rows(int64_t n, int kp) {
+  const int64_t rows = kp >= 2 ? 8192 / kp : 4096;
+  return std::max(rows, (n + 2047) / 2048);
+}
+// x += alpha p, r -= alpha q, the segment partials of r.r in bpart (bdots'
+// layout) and, with r32 set, r in FP32; p = z + beta p
+template <class T>
+void op_kr_bupdate(T *x, T *r, const T *p, const T *q, int kp, const RedPlan &P, const double *sc,
+                   DevBuf<double> &bpart, float *r32, hipStream_t s);
+template <class T>
+void op_kr_bpupdate(T *p, const T *z, int kp, const RedPlan &P, const double *sc, hipStream_t s);
 // column-major n x k caller block <-> row-major n x kp internal block; the
 // caller's vertex of internal row i is perm[i] (identity when perm is null)
 void op_to_block(const double *B, int64_t n, int k, int kp, double *X, const int32_t *perm, hipStream_t s);

@@ -784,7 +784,8 @@ LG_INST(double)
 LG_INST(float)
 #undef LG_INST
 
-void RedPlan::build(int64_t n_, const std::vector<int64_t> &blocks, hipStream_t s) {
+void RedPlan::build(int64_t n_, const std::vector<int64_t> &blocks, hipStream_t s, int64_t seg_rows) {
+  if (seg_rows <= 0) seg_rows = RED_CHUNK;
   n = n_;
   hbptr = blocks;
   if (hbptr.size() < 2) hbptr = {0, n};
@@ -793,9 +794,9 @@ void RedPlan::build(int64_t n_, const std::vector<int64_t> &blocks, hipStream_t 
   std::vector<int32_t> bs(nb + 1, 0), segblk;
   for (int c = 0; c < nb; c++) {
     bs[c] = (int32_t)lo.size();
-    for (int64_t a = hbptr[c]; a < hbptr[c + 1]; a += RED_CHUNK) {
+    for (int64_t a = hbptr[c]; a < hbptr[c + 1]; a += seg_rows) {
       lo.push_back(a);
-      hi.push_back(std::min<int64_t>(a + RED_CHUNK, hbptr[c + 1]));
+      hi.push_back(std::min<int64_t>(a + seg_rows, hbptr[c + 1]));
       segblk.push_back(c);
     }
   }

@@ -108,54 +108,6 @@ __global__ void k_kr_bstore(int nb, int kp, int np, const double *out, int s0, i
   sc[t * SC_N + s0] = out[((int64_t)blk * np) * kp + c];
   if (np > 1) sc[t * SC_N + s1] = out[((int64_t)blk * np + 1) * kp + c];
 }
-// x += alpha p, r -= alpha q per (block, column); alpha = 0 marks a finished
-// column, whose x and r stay.  Also writes the segment partials of r.r
-// exactly as the block dots form them (part[s * kp + c]: the same loop and
-// combining order), and r in FP32 when r32 is set (the mixed outer
-// preconditioner's input).
-template <class T>
-__global__ void __launch_bounds__(256) k_kr_bupdate(T *x, T *r, const T *p, const T *q, int kp,
-                                                    int lk, const int64_t *lo, const int64_t *hi,
-                                                    const int32_t *segblk, const double *sc, double *part,
-                                                    float *r32) {
-  const int s = blockIdx.x;
-  const int G = 256 >> lk, g = threadIdx.x >> lk, c = threadIdx.x & (kp - 1);
-  const double a = sc[((int64_t)segblk[s] * kp + c) * SC_N + SC_ALPHA];
-  const T at = (T)a;
-  double acc = 0;
-  for (int64_t i = lo[s] + g; i < hi[s]; i += G) {
-    const int64_t o = i * kp + c;
-    T rv = r[o];
-    if (a != 0.0) {
-      x[o] += at * p[o];
-      rv -= at * q[o];
-      r[o] = rv;
-    }
-    acc += (double)rv * (double)rv;
-    if (r32) r32[o] = (float)rv;
-  }
-  __shared__ double red[256];
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  if (g == 0) {
-    double t = 0;
-    for (int gg = 0; gg < G; gg++) t += red[gg * kp + c];
-    part[(int64_t)s * kp + c] = t;
-  }
-}
-template <class T>
-__global__ void __launch_bounds__(256) k_kr_bpupdate(T *p, const T *z, int kp, int lk,
-                                                     const int64_t *lo, const int64_t *hi,
-                                                     const int32_t *segblk, const double *sc) {
-  const int s = blockIdx.x;
-  const int G = 256 >> lk, g = threadIdx.x >> lk, c = threadIdx.x & (kp - 1);
-  const T b = (T)sc[((int64_t)segblk[s] * kp + c) * SC_N + SC_BETA];
-  for (int64_t i = lo[s] + g; i < hi[s]; i += G) {
-    const int64_t o = i * kp + c;
-    p[o] = z[o] + b * p[o];
-  }
-}
-
 template <class T>
 struct KWork {
   DevBuf<T> r, z, p, q, x;
@@ -219,6 +171,7 @@ struct Solver {
   std::vector<BLevelWork<double>> BW64;
   std::vector<BLevelWork<float>> BW32;
   int bkp = 0;  // block width the batch buffers are sized for
+  std::vector<RedPlan> bred;  // block reductions (segments by bkp) of the levels with Krylov vectors
   DevBuf<double> bparts, bpart_red, bsc_out;
   KWork<double> bouter;
   std::vector<std::vector<double>> al_pre, be_pre, al_post, be_post;
@@ -1645,10 +1598,15 @@ struct Solver {
     // scratch sized once for every operator, so no buffer is reallocated
     // while kernels that use it are queued
     int64_t maxparts = 1, maxseg = 1;
+    bred.clear();
+    bred.resize(H.size());
     for (size_t l = 0; l < H.size(); l++) {
       const DLevel &L = H[l];
       for (const DCsr *M : {&L.A, &L.M, &L.P, &L.R}) maxparts = std::max(maxparts, M->U.nparts);
-      maxseg = std::max<int64_t>(maxseg, red[l].nseg);
+      // the outer solve's levels, and those a K-cycle iterates on
+      if (l > 1 && (!o.kcycle || L.kind == LIGMG_LEVEL_ELIM)) continue;
+      bred[l].build(L.A.n, L.blocks, s, block_seg_rows(L.A.n, kp));
+      maxseg = std::max<int64_t>(maxseg, bred[l].nseg);
     }
     bparts.alloc((size_t)maxparts * kp);
     bpart_red.alloc((size_t)maxseg * 2 * kp);
@@ -1670,18 +1628,18 @@ struct Solver {
           std::string line;
           const char *nm[4] = {"A", "M", "P", "R"};
           for (int j = 0; j < 4; j++) {
-            int vw, u;
+            int u;
             if (t64[j] >= 0) {
-              spmm_tile(t64[j], &vw, &u);
-              line += std::string(" ") + nm[j] + " fp64 " + std::to_string(vw) + "x" + std::to_string(u);
+              spmm_tile(t64[j], &u);
+              line += std::string(" ") + nm[j] + " fp64 " + std::to_string(u);
             }
             if (t32[j] >= 0) {
-              spmm_tile(t32[j], &vw, &u);
-              line += std::string(" ") + nm[j] + " fp32 " + std::to_string(vw) + "x" + std::to_string(u);
+              spmm_tile(t32[j], &u);
+              line += std::string(" ") + nm[j] + " fp32 " + std::to_string(u);
             }
           }
           if (!line.empty())
-            fprintf(stderr, "[ligmg] spmm tiles k=%d level %zu (rhs per lane x gathers in flight):%s\n", kp, l,
+            fprintf(stderr, "[ligmg] spmm tiles k=%d level %zu (gathers in flight):%s\n", kp, l,
                     line.c_str());
         }
       }
@@ -1773,7 +1731,7 @@ struct Solver {
         BLevelWork<float> &bw = BW32[lvl];
         if (!r32_ready) op_d2f(r, bw.b.p, n * kp, s);
         const float *c = bcycle<float>(lvl, bw.b.p, kp);
-        const RedPlan &R = red[lvl];
+        const RedPlan &R = bred[lvl];
         R.bdots<float>(1, kp, c, nullptr, nullptr, nullptr, bsc_out.p, bpart_red, s);
         op_bsub_block_mean_f2d(z, c, kp, R, bsc_out.p, s, w, &bpart_red);
         return w != nullptr;
@@ -1783,7 +1741,7 @@ struct Solver {
     } else {
       d2d(z, bcycle<T>(lvl, r, kp), n * kp, s);
     }
-    const RedPlan &R = red[lvl];
+    const RedPlan &R = bred[lvl];
     R.bdots<T>(1, kp, z, nullptr, nullptr, nullptr, bsc_out.p, bpart_red, s);
     op_bsub_block_mean<T>(z, kp, R, bsc_out.p, s);
     return false;
@@ -1804,8 +1762,8 @@ struct Solver {
   int bkrylov(size_t lvl, const DCsr &A, T *x, const T *b, KWork<T> &K, int kp, int type,
               double rtol, int maxit, bool host_check, std::vector<int> *iters_set, int *status,
               bool outer_prec) {
-    const RedPlan &R = red[lvl];
-    const int ns = R.nb * kp, lk = ilog2(kp);
+    const RedPlan &R = bred[lvl];
+    const int ns = R.nb * kp;
     const bool fcg = fcg_like(type);
     auto grid1 = dim3((ns + 63) / 64);
     hipLaunchKernelGGL(k_kr_init, grid1, dim3(64), 0, s, ns, K.sc.p);
@@ -1836,10 +1794,7 @@ struct Solver {
       float *r32 = nullptr;
       if constexpr (std::is_same<T, double>::value)
         if (outer_prec && mixed) r32 = BW32[lvl].b.p;
-      LG_CHECK(bpart_red.n >= (size_t)R.nseg * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
-      hipLaunchKernelGGL(k_kr_bupdate<T>, dim3(R.nseg), dim3(256), 0, s, x, K.r.p, K.p.p, K.q.p, kp, lk,
-                         R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1, K.sc.p, bpart_red.p, r32);
-      LG_LAUNCH_CHECK();
+      op_kr_bupdate<T>(x, K.r.p, K.p.p, K.q.p, kp, R, K.sc.p, bpart_red, r32, s);
       it++;
       R.bdots_finish(1, kp, K.out.p, bpart_red, s);
       hipLaunchKernelGGL(k_kr_bstore, dim3((R.nb * kp + 63) / 64), dim3(64), 0, s, R.nb, kp, 1, K.out.p, SC_RN2,
@@ -1874,9 +1829,7 @@ struct Solver {
         bdot<T>(R, kp, K.r.p, K.z.p, (const T *)nullptr, (const T *)nullptr, K, SC_GN, SC_GN);
       }
       hipLaunchKernelGGL(k_kr_beta, grid1, dim3(64), 0, s, ns, fcg ? 1 : 0, K.sc.p);
-      hipLaunchKernelGGL(k_kr_bpupdate<T>, dim3(R.nseg), dim3(256), 0, s, K.p.p, K.z.p, kp, lk,
-                         R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1, K.sc.p);
-      LG_LAUNCH_CHECK();
+      op_kr_bpupdate<T>(K.p.p, K.z.p, kp, R, K.sc.p, s);
     }
     if (host_check && status) *status = LIGMG_DIVERGED_ITS;
     return it;
@@ -1923,8 +1876,8 @@ int Solver::solve_batch(int k, const double *Bin, double *Xout, int mem, ligmg_i
   op_to_block(bin.p, n, k, kp, b0b.p, perm.p, s);
   if (do_once) op_bspmv<double>(L0.R, b0b.p, rhs.p, kp, bparts, s);
   else d2d(rhs.p, b0b.p, n * kp, s);
-  red[base].bdots<double>(1, kp, rhs.p, nullptr, nullptr, nullptr, bsc_out.p, bpart_red, s);
-  op_bsub_block_mean<double>(rhs.p, kp, red[base], bsc_out.p, s);
+  bred[base].bdots<double>(1, kp, rhs.p, nullptr, nullptr, nullptr, bsc_out.p, bpart_red, s);
+  op_bsub_block_mean<double>(rhs.p, kp, bred[base], bsc_out.p, s);
   fill_zero<double>(bouter.x.p, nbse * kp);
   std::vector<int> its;
   int status = 0;
@@ -1937,7 +1890,7 @@ int Solver::solve_batch(int k, const double *Bin, double *Xout, int mem, ligmg_i
   auto t1 = std::chrono::steady_clock::now();
   // full residual per column (worst column reported)
   op_bresidual<double>(L0.A, solb.p, b0b.p, tmp.p, kp, bparts, s);
-  red[0].bdots<double>(2, kp, tmp.p, tmp.p, b0b.p, b0b.p, bsc_out.p, bpart_red, s);
+  bred[0].bdots<double>(2, kp, tmp.p, tmp.p, b0b.p, b0b.p, bsc_out.p, bpart_red, s);
   std::vector<double> d = download(bsc_out.p, (size_t)red[0].nb * 2 * kp, s);
   double worst = 0;
   for (int c = 0; c < k; c++) {

@@ -156,3 +156,25 @@ def test_grid3d_48_iterations_match_oracle():
     X, info, its = ligmg_amd.Solver(g, ligmg_amd.Options(precision=_ffi.PREC_MIXED, **opts)).solve_batch(B)
     print(f"batched mixed iterations {its.min()}..{its.max()}")
     assert info.status == _ffi.CONVERGED and np.all(np.abs(its - rinfo.iters) <= 2)
+
+
+@pytest.mark.parametrize("k", [2, 3, 8, 33, 64])
+@pytest.mark.parametrize("prec", [_ffi.PREC_FP64, _ffi.PREC_MIXED])
+def test_batch_hub_rows_and_segments(k, prec):
+    """Rows of every class of the block SpMM (whole, split over groups, hub
+    chunks of 2048), block-vector segments with a remainder, and a width
+    whose tiles are timed: the single solves' columns, and the same bits
+    with the tuner off."""
+    g = graphs.rmat_config(15, "lognormal", pendants=True)
+    assert int(np.diff(g.rowptr).max()) > 2 * 2048 and g.n % (8192 // 64) != 0
+    B = graphs.rhs(g.n, k, 5).reshape(g.n, k, order="F")
+    X = []
+    for tune in (1, 0):
+        s = ligmg_amd.Solver(g, ligmg_amd.Options(precision=prec, outer_ksp_type=_ffi.KSP_FCG, spmm_tune=tune))
+        x, info, its = s.solve_batch(B)
+        assert info.status == _ffi.CONVERGED and info.full_rel_residual <= 1e-7
+        X.append(x)
+    assert np.array_equal(X[0], X[1])
+    for c in {0, k // 2, k - 1}:
+        one = s.solve(np.ascontiguousarray(B[:, c]))
+        assert rel(X[0][:, c], one.solution) <= 1e-7 and abs(int(its[c]) - one.iters()) <= 1
