@@ -1,0 +1,29 @@
+// The coarse levels of a V-cycle as one dense matrix (collapse.hip).
+#pragma once
+#include <vector>
+
+#include "hierarchy.hpp"
+
+namespace lg {
+
+// Largest level collapsed.  A product with 1024^2 entries (8 MiB, resident in
+// the L2s) takes about 4 us, the levels below it 50 to 150 us of dependent
+// launches: R-MAT 10 solve 1.37 -> 0.70 ms, 256 x 256 grid 14.6 -> 12.3 ms; forming
+// it costs a setup about 0.2 ms.
+constexpr int64_t COLLAPSE_MAX_N = 1024;
+
+// What the cycle does besides its operators: smoother coefficients per level
+// (al[l][k] and be[l][k] of step k), the smoother, the constant correction.
+struct CycleCoeffs {
+  const std::vector<std::vector<double>> &al_pre, &be_pre, &al_post, &be_post;
+  int pre_smooth, post_smooth;
+  bool jacobi;
+  double scale;  // 4/3 with the constant correction, else 1
+};
+
+// out: the row-major n x n matrix of the FP64 V-cycle from level l down
+// (n = H[l].A.n).  Queues its work on s.
+void collapse_cycle(const std::vector<DLevel> &H, const CycleCoeffs &C, size_t l, DevBuf<double> &out,
+                    hipStream_t s);
+
+}  // namespace lg

@@ -264,6 +264,7 @@ __global__ void k_dense_apply(const double *__restrict__ Pm, int64_t n, const T 
   const int64_t nw = (int64_t)gridDim.x * blockDim.x / WAVE;
   for (int64_t row = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / WAVE; row < n; row += nw) {
     double s = 0;
+#pragma unroll 8
     for (int64_t j = lane; j < n; j += WAVE) s += Pm[row * n + j] * (double)x[j];
     s = wave_sum(s);
     if (lane == 0) y[row] = (T)s;

@@ -24,6 +24,7 @@
 #include "prims.hpp"
 #include "setup.hpp"
 #include "solve_dev.hpp"
+#include "collapse.hpp"
 #include "tail.hpp"
 #include "petsc_io.hpp"
 
@@ -205,6 +206,10 @@ struct Solver {
     const void *in = nullptr, *out = nullptr;
   };
   std::vector<TailProg> tail_prog[2];
+  // V-cycles: the cycle from level dense_l0 down as one dense matrix
+  // (dense_l0 = H.size(): none)
+  size_t dense_l0 = 0;
+  DevBuf<double> dense_m;
   TailParams tail_p;
   static constexpr int64_t TAIL_MAX_INSTR = 1 << 18;
 
@@ -422,6 +427,8 @@ struct Solver {
     for (auto &r : red) maxnb = std::max(maxnb, r.nb);
     dsc.alloc((size_t)8 * maxnb);
     phase("slices");
+    setup_dense(base);
+    phase("dense");
     setup_tail();
     LG_HIP(hipStreamSynchronize(s));
     phase("tail");
@@ -890,9 +897,9 @@ struct Solver {
   const T *rec_cycle(std::vector<TailInstr> &c, size_t l, const T *b) {
     DLevel &L = H[l];
     LevelWork<T> &w = work<T>(l);
-    if (L.kind == LIGMG_LEVEL_COARSE) {
-      TailInstr I = ti(TI_DENSE, L.n);
-      I.p[0] = L.pinv.p;
+    if (L.kind == LIGMG_LEVEL_COARSE || l == dense_l0) {
+      TailInstr I = ti(TI_DENSE, L.A.n);
+      I.p[0] = l == dense_l0 ? dense_m.p : L.pinv.p;
       I.p[1] = b;
       I.p[2] = w.B[0].p;
       c.push_back(I);
@@ -1057,6 +1064,21 @@ struct Solver {
     return rec[e];
   }
 
+  // The first level (from the outer solve's on) of at most COLLAPSE_MAX_N
+  // vertices, with the levels below it, becomes one matrix: V-cycles only
+  // (a K-cycle's inner Krylov solves are not linear).
+  void setup_dense(size_t base) {
+    dense_l0 = H.size();
+    if (o.kcycle) return;
+    size_t l = base;
+    while (H[l].A.n > COLLAPSE_MAX_N && H[l].kind != LIGMG_LEVEL_COARSE) l++;
+    if (H[l].kind == LIGMG_LEVEL_COARSE) return;  // already one dense matrix
+    collapse_cycle(H, {al_pre, be_pre, al_post, be_post, o.pre_smooth, o.post_smooth,
+                       o.smoother_type == LIGMG_SMOOTHER_JACOBI, o.constant_correction ? 4.0 / 3.0 : 1.0},
+                   l, dense_m, s);
+    dense_l0 = l;
+  }
+
   void setup_tail() {
     const size_t nl = H.size();
     tail_l0 = nl;
@@ -1068,6 +1090,19 @@ struct Solver {
     while (l0 < nl && tail_count(l0 - 1) > TAIL_MAX_INSTR) l0++;
     if (l0 >= nl) return;
     tail_l0 = l0;
+    // a tail that starts at the collapsed level or below is only entered by
+    // solves and cycles from there (need_tail)
+    if (tail_l0 < dense_l0) record_tail();
+  }
+
+  // Called before a cycle from level lvl: its corrections enter the tail
+  // where the collapsed level does not come first.
+  void need_tail(size_t lvl) {
+    if (lvl > dense_l0 && tail_l0 < H.size() && tail_sched.empty()) record_tail();
+  }
+
+  void record_tail() {
+    const size_t nl = H.size(), l0 = tail_l0;
     tail_sched.clear();
     tail_sched.resize(4 * nl);
     for (size_t l = l0; l < nl; l++) {
@@ -1139,8 +1174,8 @@ struct Solver {
   const T *cycle(size_t l, const T *b) {
     DLevel &L = H[l];
     LevelWork<T> &w = work<T>(l);
-    if (L.kind == LIGMG_LEVEL_COARSE) {
-      op_dense_apply<T>(L.pinv.p, L.n, b, w.B[0].p, s);
+    if (L.kind == LIGMG_LEVEL_COARSE || l == dense_l0) {
+      op_dense_apply<T>(l == dense_l0 ? dense_m.p : L.pinv.p, L.A.n, b, w.B[0].p, s);
       return w.B[0].p;
     }
     if (L.kind == LIGMG_LEVEL_ELIM) {
@@ -1208,6 +1243,7 @@ struct Solver {
   template <class T>
   const T *recurse(size_t l, const T *bc) {
     const DLevel &N = H[l + 1];
+    if (l + 1 == dense_l0) return cycle<T>(l + 1, bc);
     if (l + 1 >= tail_l0) {
       const TailProg &P = tail_prog[pidx<T>()][l];
       LG_CHECK(P.in == bc, LIGMG_ERR_INVALID, "fused tail entered with an unrecorded right-hand side");
@@ -1651,8 +1687,8 @@ struct Solver {
   const T *bcycle(size_t l, const T *b, int kp) {
     DLevel &L = H[l];
     BLevelWork<T> &w = bwork<T>(l);
-    if (L.kind == LIGMG_LEVEL_COARSE) {
-      op_bdense_apply<T>(L.pinv.p, L.n, b, w.B[0].p, kp, s);
+    if (L.kind == LIGMG_LEVEL_COARSE || l == dense_l0) {
+      op_bdense_apply<T>(l == dense_l0 ? dense_m.p : L.pinv.p, L.A.n, b, w.B[0].p, kp, s);
       return w.B[0].p;
     }
     if (L.kind == LIGMG_LEVEL_ELIM) {
@@ -2032,6 +2068,7 @@ int Solver::solve(const double *b, double *x, int mem, ligmg_info *info, double 
   const size_t base = do_once ? (size_t)from + 1 : (size_t)from;
   const DLevel &B = H[base];
   const int64_t nb_ = B.A.n;
+  need_tail(base);
   if (outer.x.n < (size_t)nb_ || outer.sc.n < (size_t)red[base].nb * SC_N) outer.alloc(nb_, red[base].nb);
   rhs_base.ensure(std::max<int64_t>(nb_, 1));
   double *rhs = rhs_base.p;
@@ -2713,6 +2750,7 @@ int ligmg_apply_cycle(ligmg_handle h, int32_t l, int32_t prec, const double *r, 
   if (!h || l < 0 || l >= (int)h->S.H.size() || !r || !z) return LIGMG_ERR_INVALID;
   try {
     lg::Solver &S = h->S;
+    S.need_tail((size_t)l);
     const bool f32 = prec == LIGMG_PREC_MIXED;
     LG_CHECK(!f32 || S.mixed, LIGMG_ERR_INVALID,
              "ligmg_apply_cycle: FP32 cycles exist only with precision = LIGMG_PREC_MIXED");

@@ -682,6 +682,7 @@ void cheby_coeffs(double lo, double hi, int steps, std::vector<double> &al, std:
 
 void cheby_apply(const Csr &A, const std::vector<double> &dinv, double lo, double hi, int steps,
                  double *x, const double *b) {
+  if (steps <= 0) return;  // no smoothing: x stays
   std::vector<double> al, be;
   cheby_coeffs(lo, hi, steps, al, be);
   std::vector<double> prev(x, x + A.n), Ax(A.n), nx(A.n);
