@@ -101,6 +101,27 @@ struct DevBuf {
   size_t bytes() const { return n * sizeof(T); }
 };
 
+// Pinned host memory the GPU writes directly.
+template <class T>
+struct PinnedBuf {
+  T *p = nullptr;
+  size_t n = 0;
+  PinnedBuf() = default;
+  PinnedBuf(const PinnedBuf &) = delete;
+  PinnedBuf &operator=(const PinnedBuf &) = delete;
+  ~PinnedBuf() {
+    if (p) (void)hipHostFree(p);
+  }
+  void ensure(size_t count) {
+    if (count <= n) return;
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    n = 0;
+    LG_HIP(hipHostMalloc((void **)&p, count * sizeof(T), hipHostMallocCoherent));
+    n = count;
+  }
+};
+
 template <class T>
 inline void to_device(T *dst, const T *src, size_t count, hipStream_t s) {
   if (count) LG_HIP(hipMemcpyAsync(dst, src, count * sizeof(T), hipMemcpyHostToDevice, s));

@@ -67,12 +67,6 @@ struct RedPlan {
   // 1), j < np (np <= 4), accumulated in FP64.
   template <class T>
   void dots(int np, const T *const *a, const T *const *b, double *out, hipStream_t s) const;
-  // Krylov form (np <= 2): block c's results go to the scalar slots
-  // sc[c * SC_N + s0] (and s1), then the scalar step `post` (KrPost) runs on
-  // them in the same launch.  Same bits as dots + the separate scalar kernels.
-  template <class T>
-  void dots_sc(int np, const T *const *a, const T *const *b, double *sc, int s0, int s1, int post, int fcg,
-               double rtol, hipStream_t s) const;
   // out[c] = sum over block c of a[i]
   template <class T> void sums(const T *a, double *out, hipStream_t s) const;
   // block vectors (n x kp row-major): out[(blk * np + j) * kp + c] = sum over
@@ -84,6 +78,29 @@ struct RedPlan {
   // wrote to bpart in bdots' layout
   void bdots_finish(int np, int kp, double *out, const DevBuf<double> &bpart, hipStream_t s) const;
 };
+
+// What the host sees of a block's convergence, in pinned memory; seq counts
+// the norms of a solve from 1.
+struct KrHost {
+  double rn2, active;
+  unsigned long long seq, pad;
+};
+// One Krylov iteration on a level (sc: SC_N scalars per block): the start
+// from x = 0, the norm of r with the convergence flag, then z = c - mean
+// (with z.w: q for FCG, r for CG), p = z + beta p, the dots of q = A p (r only
+// for FCG), and x += alpha p, r -= alpha q.  r32: also r in FP32.
+template <class T>
+void kr_begin(const RedPlan &R, const T *b, T *x, T *r, float *r32, hipStream_t s);
+void kr_norm(const RedPlan &R, double *sc, bool init, double rtol, KrHost *host, unsigned long long *seq,
+             hipStream_t s);
+template <class T, class C>
+void kr_center(const RedPlan &R, T *z, const C *c, const T *w, hipStream_t s);
+template <class T>
+void kr_pupdate(const RedPlan &R, T *p, const T *z, double *sc, bool fcg, hipStream_t s);
+template <class T>
+void kr_dots(const RedPlan &R, const T *p, const T *q, const T *r, hipStream_t s);
+template <class T>
+void kr_update(const RedPlan &R, T *x, T *r, const T *p, const T *q, double *sc, bool fcg, float *r32, hipStream_t s);
 
 // a -= mean of a over each block, means taken from sums[c] (device)
 template <class T> void op_sub_block_mean(T *a, const RedPlan &P, const double *sums, hipStream_t s);

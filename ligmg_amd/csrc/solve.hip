@@ -277,53 +277,271 @@ __global__ void k_dense_apply(const double *__restrict__ Pm, int64_t n, const T 
 // grid 61 -> 50 ms per right-hand side).
 constexpr int RED_CHUNK = 4096;
 
+// Items lo + vt, lo + vt + 256, ... of a segment in batches of RED_BATCH:
+// load(t, i) asks for item i into slot t (past the end: the last item), then
+// use(t, i) takes the slots in order.  One item at a time, a segment was a
+// chain of 16 dependent waits (8.1 us for a two-product dot on 0.7 M entries).
+constexpr int RED_BATCH = 8;
+template <class Load, class Use>
+__device__ __forceinline__ void seg_items(int64_t lo, int64_t hi, int vt, const Load &load, const Use &use) {
+  for (int64_t i = lo + vt; i < hi; i += 256 * RED_BATCH) {
+#pragma unroll
+    for (int t = 0; t < RED_BATCH; t++) load(t, min(i + t * 256, hi - 1));
+#pragma unroll
+    for (int t = 0; t < RED_BATCH; t++)
+      if (i + t * 256 < hi) use(t, i + t * 256);
+  }
+}
+
+// The sum of v over a 256-thread workgroup, on thread 0: butterfly per
+// wavefront, the wavefront sums in order.  ws: 4 doubles of LDS per call.
+__device__ __forceinline__ double block_sum(double v, double *ws) {
+  v = wave_sum(v);
+  if ((threadIdx.x & (WAVE - 1)) == 0) ws[threadIdx.x / WAVE] = v;
+  __syncthreads();
+  return ((ws[0] + ws[1]) + ws[2]) + ws[3];
+}
+
 template <class T>
 __global__ void __launch_bounds__(256) k_red_stage1(int np, const T *a0, const T *b0, const T *a1,
                                                     const T *b1, const T *a2, const T *b2,
                                                     const T *a3, const T *b3, const int64_t *lo,
                                                     const int64_t *hi, double *part) {
   const int s = blockIdx.x;
-  const int64_t l = lo[s], h = hi[s];
   double acc[4] = {0, 0, 0, 0};
   const T *A[4] = {a0, a1, a2, a3};
   const T *B[4] = {b0, b1, b2, b3};
-  for (int64_t i = l + threadIdx.x; i < h; i += 256) {
+  for (int64_t i = lo[s] + threadIdx.x; i < hi[s]; i += 256) {
 #pragma unroll
     for (int j = 0; j < 4; j++)
       if (j < np) acc[j] += (double)A[j][i] * (B[j] ? (double)B[j][i] : 1.0);
   }
   __shared__ double ws[4][4];
-  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
 #pragma unroll
   for (int j = 0; j < 4; j++) {
-    double v = wave_sum(acc[j]);
-    if (lane == 0) ws[j][w] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < 4 && (int)threadIdx.x < np) {
-    int j = threadIdx.x;
-    part[s * 4 + j] = ((ws[j][0] + ws[j][1]) + ws[j][2]) + ws[j][3];
+    const double v = block_sum(acc[j], ws[j]);
+    if (threadIdx.x == 0 && j < np) part[s * 4 + j] = v;
   }
 }
 
-// Where a block's dot results go: out[c * np + j], or the Krylov scalar
-// slots of block c followed by its scalar step.
-struct RedSink {
-  double *out = nullptr;
-  double *sc = nullptr;
-  int s0 = 0, s1 = 0, post = KP_NONE, fcg = 0;
-  double rtol = 0;
-  __device__ __forceinline__ void put(int c, int np, const double *v) const {
-    if (!sc) {
-      for (int j = 0; j < np; j++) out[c * np + j] = v[j];
-      return;
-    }
-    double *S = sc + c * SC_N;
-    S[s0] = v[0];
-    if (np > 1) S[s1] = v[1];
-    kr_post(S, post, fcg, rtol);
+// ------------------------------------------------ Krylov steps (CG, FCG)
+// One iteration's vector work on a level, segments as in the dots above.  The
+// scalars need no launch of their own: the kernel after a dot adds the
+// segment partials itself, every workgroup the sums of its block in
+// k_red_stage2's order, and the first workgroup of a block stores them.  (A
+// dot, its second stage, the update, the norm and its second stage, the copy,
+// the block sums and the mean were 13 launches of 2-8 us per iteration; these
+// are 7.)  Partial slots of a segment: 0, 1 dots, 2 r.r, 3 block sums.
+enum { KS_DOT = 0, KS_DOT1 = 1, KS_RR = 2, KS_SUM = 3 };
+
+// Sums of slots j0 .. j0 + N - 1 over block c, on every thread of the
+// workgroup (q: N * WAVE doubles of LDS): lane l of wavefront 0 adds segments
+// l G .. l G + G - 1 in order, then the lane sums are added in order.
+template <int N>
+__device__ __forceinline__ void block_partials(const int32_t *bseg, int c, const double *part, int j0, double (*q)[WAVE],
+                                               double *out) {
+  const int g0 = bseg[c], g1 = bseg[c + 1];
+  const int G = (g1 - g0 + WAVE - 1) / WAVE;
+  if (threadIdx.x < WAVE) {
+    const int a = min(g0 + (int)threadIdx.x * G, g1), b = min(a + G, g1);
+    double s[N] = {};
+#pragma unroll 4
+    for (int g = a; g < b; g++)
+#pragma unroll
+      for (int j = 0; j < N; j++) s[j] += part[g * 4 + j0 + j];
+#pragma unroll
+    for (int j = 0; j < N; j++) q[j][threadIdx.x] = s[j];
   }
-};
+  __syncthreads();
+  const int used = G > 0 ? (g1 - g0 + G - 1) / G : 0;  // lanes that hold a sum
+#pragma unroll
+  for (int j = 0; j < N; j++) {
+    double s = 0;
+    for (int l = 0; l < used; l++) s += q[j][l];
+    out[j] = s;
+  }
+}
+
+// x = 0, r = b (the residual of a zero iterate), the partials of b.b
+template <class T>
+__global__ void __launch_bounds__(256) k_kr_begin(const T *b, T *x, T *r, float *r32, const int64_t *lo,
+                                                  const int64_t *hi, double *part) {
+  const int s = blockIdx.x;
+  double acc = 0;
+  T v[RED_BATCH];
+  seg_items(lo[s], hi[s], threadIdx.x, [&](int t, int64_t i) { v[t] = b[i]; },
+            [&](int t, int64_t i) {
+              x[i] = (T)0;
+              r[i] = v[t];
+              if (r32) r32[i] = (float)v[t];
+              acc += (double)v[t] * (double)v[t];
+            });
+  __shared__ double ws[4];
+  const double sum = block_sum(acc, ws);
+  if (threadIdx.x == 0) part[s * 4 + KS_RR] = sum;
+}
+
+// One wavefront per block: r.r from its partials, the convergence flag, and
+// a copy of both for the host.  init: the first one, where r.r is also b.b.
+__global__ void __launch_bounds__(WAVE) k_kr_norm(const int32_t *bseg, const double *part, double *sc, int init,
+                                                  double rtol, KrHost *host, unsigned long long *seq) {
+  __shared__ double q[1][WAVE];
+  const int c = blockIdx.x;
+  double rr[1];
+  block_partials<1>(bseg, c, part, KS_RR, q, rr);
+  if (threadIdx.x != 0) return;
+  double *S = sc + c * SC_N;
+  if (init) {
+    kr_init(S);
+    S[SC_BN2] = rr[0];
+  }
+  S[SC_RN2] = rr[0];
+  kr_check(S, rtol);
+  if (!host) return;
+  const unsigned long long k = init ? 1 : seq[c] + 1;
+  seq[c] = k;
+  volatile KrHost *h = host + c;
+  h->rn2 = rr[0];
+  h->active = S[SC_ACTIVE];
+  __threadfence_system();
+  h->seq = k;
+}
+
+// partials of p.q and, with r set, p.r
+template <class T>
+__global__ void __launch_bounds__(256) k_kr_dots(const T *p, const T *q, const T *r, const int64_t *lo,
+                                                 const int64_t *hi, double *part) {
+  const int s = blockIdx.x;
+  double a0 = 0, a1 = 0;
+  T pv[RED_BATCH], qv[RED_BATCH], rv[RED_BATCH];
+  seg_items(lo[s], hi[s], threadIdx.x,
+            [&](int t, int64_t i) {
+              pv[t] = p[i];
+              qv[t] = q[i];
+              if (r) rv[t] = r[i];
+            },
+            [&](int t, int64_t) {
+              a0 += (double)pv[t] * (double)qv[t];
+              if (r) a1 += (double)pv[t] * (double)rv[t];
+            });
+  __shared__ double ws[2][4];
+  const double s0 = block_sum(a0, ws[0]), s1 = block_sum(a1, ws[1]);
+  if (threadIdx.x == 0) {
+    part[s * 4 + KS_DOT] = s0;
+    part[s * 4 + KS_DOT1] = s1;
+  }
+}
+
+// alpha = (FCG: p.r, CG: r.z) / p.q; x += alpha p, r -= alpha q, the
+// partials of r.r, and r in FP32 when r32 is set
+template <class T>
+__global__ void __launch_bounds__(256) k_kr_update(T *x, T *r, const T *p, const T *q, float *r32,
+                                                   const int64_t *lo, const int64_t *hi, const int32_t *segblk,
+                                                   const int32_t *bseg, double *part, double *sc, int fcg) {
+  __shared__ double qs[2][WAVE], ws[4];
+  const int s = blockIdx.x, c = segblk[s];
+  double d[2];
+  block_partials<2>(bseg, c, part, KS_DOT, qs, d);
+  double *S = sc + c * SC_N;
+  const double num = fcg ? d[1] : S[SC_GN];
+  const double a = (S[SC_ACTIVE] != 0 && d[0] != 0) ? num / d[0] : 0.0;
+  if (s == bseg[c] && threadIdx.x == 0) {
+    S[SC_DELTA] = d[0];
+    S[SC_T1] = d[1];
+    S[SC_ALPHA] = a;
+    if (!fcg) S[SC_GAMMA] = num;
+  }
+  const T at = (T)a;
+  double acc = 0;
+  T xv[RED_BATCH], rv[RED_BATCH], pv[RED_BATCH], qv[RED_BATCH];
+  seg_items(lo[s], hi[s], threadIdx.x,
+            [&](int t, int64_t i) {
+              rv[t] = r[i];
+              if (a != 0.0) {
+                xv[t] = x[i];
+                pv[t] = p[i];
+                qv[t] = q[i];
+              }
+            },
+            [&](int t, int64_t i) {
+              if (a != 0.0) {
+                x[i] = xv[t] + at * pv[t];
+                rv[t] -= at * qv[t];
+                r[i] = rv[t];
+              }
+              if (r32) r32[i] = (float)rv[t];
+              acc += (double)rv[t] * (double)rv[t];
+            });
+  const double sum = block_sum(acc, ws);
+  if (threadIdx.x == 0) part[s * 4 + KS_RR] = sum;
+}
+
+// partials of the block sums of c
+template <class C>
+__global__ void __launch_bounds__(256) k_kr_sum(const C *c, const int64_t *lo, const int64_t *hi, double *part) {
+  const int s = blockIdx.x;
+  double acc = 0;
+  C v[RED_BATCH];
+  seg_items(lo[s], hi[s], threadIdx.x, [&](int t, int64_t i) { v[t] = c[i]; },
+            [&](int t, int64_t) { acc += (double)v[t]; });
+  __shared__ double ws[4];
+  const double sum = block_sum(acc, ws);
+  if (threadIdx.x == 0) part[s * 4 + KS_SUM] = sum;
+}
+
+// z = c - (block mean), the partials of z.w
+template <class T, class C>
+__global__ void __launch_bounds__(256) k_kr_center(T *z, const C *cv, const T *w, const int64_t *lo,
+                                                   const int64_t *hi, const int32_t *segblk, const int32_t *bseg,
+                                                   const int64_t *bptr, double *part) {
+  __shared__ double qs[1][WAVE], ws[4];
+  const int s = blockIdx.x, c = segblk[s];
+  double sum[1];
+  block_partials<1>(bseg, c, part, KS_SUM, qs, sum);
+  const T m = (T)(sum[0] / (double)(bptr[c + 1] - bptr[c]));
+  double acc = 0;
+  C v[RED_BATCH];
+  T wv[RED_BATCH];
+  seg_items(lo[s], hi[s], threadIdx.x,
+            [&](int t, int64_t i) {
+              v[t] = cv[i];
+              wv[t] = w[i];
+            },
+            [&](int t, int64_t i) {
+              const T zv = (T)v[t] - m;
+              z[i] = zv;
+              acc += (double)zv * (double)wv[t];
+            });
+  const double dot = block_sum(acc, ws);
+  if (threadIdx.x == 0) part[s * 4 + KS_DOT] = dot;
+}
+
+// beta = (FCG: -z.q / p.q, CG: r.z / the last one); p = z + beta p.  Before
+// the first step p.q and the last r.z are 0, beta is 0 and p is not read.
+template <class T>
+__global__ void __launch_bounds__(256) k_kr_pupdate(T *p, const T *z, const int64_t *lo, const int64_t *hi,
+                                                    const int32_t *segblk, const int32_t *bseg, const double *part,
+                                                    double *sc, int fcg) {
+  __shared__ double qs[1][WAVE];
+  const int s = blockIdx.x, c = segblk[s];
+  double d[1];
+  block_partials<1>(bseg, c, part, KS_DOT, qs, d);
+  double *S = sc + c * SC_N;
+  const double den = fcg ? S[SC_DELTA] : S[SC_GAMMA];
+  const double be = (S[SC_ACTIVE] != 0 && den != 0) ? (fcg ? -d[0] : d[0]) / den : 0.0;
+  if (s == bseg[c] && threadIdx.x == 0) {
+    S[SC_BETA] = be;
+    if (!fcg) S[SC_GN] = d[0];
+  }
+  const T bt = (T)be;
+  T zv[RED_BATCH], pv[RED_BATCH];
+  seg_items(lo[s], hi[s], threadIdx.x,
+            [&](int t, int64_t i) {
+              zv[t] = z[i];
+              if (be != 0.0) pv[t] = p[i];
+            },
+            [&](int t, int64_t i) { p[i] = be != 0.0 ? zv[t] + bt * pv[t] : zv[t]; });
+}
 
 // Both stages in one workgroup for plans of at most RED_FUSE_SEGS segments:
 // four 256-thread groups reduce segments g, g + 4, ... with the tree of
@@ -336,7 +554,7 @@ template <class T>
 __global__ void __launch_bounds__(1024) k_red_fused(int np, int nseg, int nb, const T *a0, const T *b0,
                                                     const T *a1, const T *b1, const T *a2, const T *b2,
                                                     const T *a3, const T *b3, const int64_t *lo,
-                                                    const int64_t *hi, const int32_t *bseg, RedSink sink) {
+                                                    const int64_t *hi, const int32_t *bseg, double *out) {
   __shared__ double part[RED_FUSE_SEGS * 4];
   __shared__ double ws[4][4][4];  // group, product, wavefront
   const int grp = threadIdx.x / 256, vt = threadIdx.x % 256;
@@ -368,13 +586,11 @@ __global__ void __launch_bounds__(1024) k_red_fused(int np, int nseg, int nb, co
   }
   if ((int)threadIdx.x < nb) {
     const int c = threadIdx.x;
-    double v[4];
     for (int j = 0; j < np; j++) {
       double s = 0;
       for (int g = bseg[c]; g < bseg[c + 1]; g++) s += part[g * 4 + j];
-      v[j] = s;
+      out[c * np + j] = s;
     }
-    sink.put(c, np, v);
   }
 }
 
@@ -383,7 +599,7 @@ __global__ void __launch_bounds__(1024) k_red_fused(int np, int nseg, int nb, co
 // the 64 lane sums in order.  With at most 64 segments per block this is the
 // plain in-order sum of the segment sums (the fused kernel's second stage).
 __global__ void __launch_bounds__(WAVE) k_red_stage2(int np, const int32_t *bseg, const double *part,
-                                                    RedSink sink) {
+                                                    double *out) {
   __shared__ double q[4][WAVE];
   const int c = blockIdx.x, lane = threadIdx.x;
   const int g0 = bseg[c], g1 = bseg[c + 1];
@@ -396,13 +612,11 @@ __global__ void __launch_bounds__(WAVE) k_red_stage2(int np, const int32_t *bseg
   }
   __syncthreads();
   if (lane != 0) return;
-  double v[4];
   for (int j = 0; j < np; j++) {
     double s = 0;
     for (int l = 0; l < WAVE; l++) s += q[j][l];
-    v[j] = s;
+    out[c * np + j] = s;
   }
-  sink.put(c, np, v);
 }
 
 template <class T>
@@ -818,7 +1032,7 @@ void RedPlan::build(int64_t n_, const std::vector<int64_t> &blocks, hipStream_t 
 
 namespace {
 template <class T>
-void run_dots(const RedPlan &R, int np, const T *const *a, const T *const *b, const RedSink &sink,
+void run_dots(const RedPlan &R, int np, const T *const *a, const T *const *b, double *out,
               hipStream_t s) {
   if (R.nseg == 0) return;
   const T *A[4] = {nullptr, nullptr, nullptr, nullptr}, *B[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -828,37 +1042,21 @@ void run_dots(const RedPlan &R, int np, const T *const *a, const T *const *b, co
   }
   if (R.nseg <= RED_FUSE_SEGS && R.nb <= 1024) {  // one launch; a thread per block for the second stage
     hipLaunchKernelGGL(k_red_fused<T>, dim3(1), dim3(1024), 0, s, np, R.nseg, R.nb, A[0], B[0], A[1], B[1],
-                       A[2], B[2], A[3], B[3], R.seg_lo.p, R.seg_hi.p, R.bseg.p, sink);
+                       A[2], B[2], A[3], B[3], R.seg_lo.p, R.seg_hi.p, R.bseg.p, out);
     LG_LAUNCH_CHECK();
     return;
   }
   hipLaunchKernelGGL(k_red_stage1<T>, dim3(R.nseg), dim3(256), 0, s, np, A[0], B[0], A[1], B[1], A[2],
                      B[2], A[3], B[3], R.seg_lo.p, R.seg_hi.p, R.part.p);
   LG_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_red_stage2, dim3(R.nb), dim3(WAVE), 0, s, np, R.bseg.p, R.part.p, sink);
+  hipLaunchKernelGGL(k_red_stage2, dim3(R.nb), dim3(WAVE), 0, s, np, R.bseg.p, (const double *)R.part.p, out);
   LG_LAUNCH_CHECK();
 }
 }  // namespace
 
 template <class T>
 void RedPlan::dots(int np, const T *const *a, const T *const *b, double *out, hipStream_t s) const {
-  RedSink sink;
-  sink.out = out;
-  run_dots<T>(*this, np, a, b, sink, s);
-}
-
-template <class T>
-void RedPlan::dots_sc(int np, const T *const *a, const T *const *b, double *sc, int s0, int s1, int post,
-                      int fcg, double rtol, hipStream_t s) const {
-  LG_CHECK(np >= 1 && np <= 2, 1, "dots_sc: one or two products");
-  RedSink sink;
-  sink.sc = sc;
-  sink.s0 = s0;
-  sink.s1 = s1;
-  sink.post = post;
-  sink.fcg = fcg;
-  sink.rtol = rtol;
-  run_dots<T>(*this, np, a, b, sink, s);
+  run_dots<T>(*this, np, a, b, out, s);
 }
 
 template <class T>
@@ -879,12 +1077,59 @@ template void RedPlan::dots<double>(int, const double *const *, const double *co
                                     hipStream_t) const;
 template void RedPlan::dots<float>(int, const float *const *, const float *const *, double *,
                                    hipStream_t) const;
-template void RedPlan::dots_sc<double>(int, const double *const *, const double *const *, double *, int, int,
-                                       int, int, double, hipStream_t) const;
-template void RedPlan::dots_sc<float>(int, const float *const *, const float *const *, double *, int, int, int,
-                                      int, double, hipStream_t) const;
 template void RedPlan::sums<double>(const double *, double *, hipStream_t) const;
 template void RedPlan::sums<float>(const float *, double *, hipStream_t) const;
+#define LG_SEGS dim3((unsigned)R.nseg), dim3(256), 0, s
+template <class T>
+void kr_begin(const RedPlan &R, const T *b, T *x, T *r, float *r32, hipStream_t s) {
+  hipLaunchKernelGGL(k_kr_begin<T>, LG_SEGS, b, x, r, r32, R.seg_lo.p, R.seg_hi.p, R.part.p);
+  LG_LAUNCH_CHECK();
+}
+void kr_norm(const RedPlan &R, double *sc, bool init, double rtol, KrHost *host, unsigned long long *seq,
+             hipStream_t s) {
+  hipLaunchKernelGGL(k_kr_norm, dim3((unsigned)R.nb), dim3(WAVE), 0, s, R.bseg.p, (const double *)R.part.p, sc,
+                     init ? 1 : 0, rtol, host, seq);
+  LG_LAUNCH_CHECK();
+}
+template <class T>
+void kr_dots(const RedPlan &R, const T *p, const T *q, const T *r, hipStream_t s) {
+  hipLaunchKernelGGL(k_kr_dots<T>, LG_SEGS, p, q, r, R.seg_lo.p, R.seg_hi.p, R.part.p);
+  LG_LAUNCH_CHECK();
+}
+template <class T>
+void kr_update(const RedPlan &R, T *x, T *r, const T *p, const T *q, double *sc, bool fcg, float *r32, hipStream_t s) {
+  hipLaunchKernelGGL(k_kr_update<T>, LG_SEGS, x, r, p, q, r32, R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1, R.bseg.p,
+                     R.part.p, sc, fcg ? 1 : 0);
+  LG_LAUNCH_CHECK();
+}
+template <class T, class C>
+void kr_center(const RedPlan &R, T *z, const C *c, const T *w, hipStream_t s) {
+  hipLaunchKernelGGL(k_kr_sum<C>, LG_SEGS, c, R.seg_lo.p, R.seg_hi.p, R.part.p);
+  LG_LAUNCH_CHECK();
+  hipLaunchKernelGGL((k_kr_center<T, C>), LG_SEGS, z, c, w, R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1, R.bseg.p,
+                     R.bptr.p, R.part.p);
+  LG_LAUNCH_CHECK();
+}
+template <class T>
+void kr_pupdate(const RedPlan &R, T *p, const T *z, double *sc, bool fcg, hipStream_t s) {
+  hipLaunchKernelGGL(k_kr_pupdate<T>, LG_SEGS, p, z, R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1, R.bseg.p,
+                     (const double *)R.part.p, sc, fcg ? 1 : 0);
+  LG_LAUNCH_CHECK();
+}
+#undef LG_SEGS
+#define LG_KR(T)                                                                                          \
+  template void kr_begin<T>(const RedPlan &, const T *, T *, T *, float *, hipStream_t);                  \
+  template void kr_dots<T>(const RedPlan &, const T *, const T *, const T *, hipStream_t);                \
+  template void kr_update<T>(const RedPlan &, T *, T *, const T *, const T *, double *, bool, float *,    \
+                             hipStream_t);                                                                \
+  template void kr_pupdate<T>(const RedPlan &, T *, const T *, double *, bool, hipStream_t);
+LG_KR(double)
+LG_KR(float)
+#undef LG_KR
+template void kr_center<double, double>(const RedPlan &, double *, const double *, const double *, hipStream_t);
+template void kr_center<double, float>(const RedPlan &, double *, const float *, const double *, hipStream_t);
+template void kr_center<float, float>(const RedPlan &, float *, const float *, const float *, hipStream_t);
+
 template void op_sub_block_mean<double>(double *, const RedPlan &, const double *, hipStream_t);
 template void op_sub_block_mean<float>(float *, const RedPlan &, const double *, hipStream_t);
 

@@ -9,6 +9,8 @@
 //                     aggregation.hpp:209-241, elimination.hpp:33-52
 //   Krylov        <- petsc_fcg (PETSc KSPCG/FCG)   cg.hpp:18-116
 #include <algorithm>
+#include <array>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -53,30 +55,6 @@ __global__ void k_kr_beta(int nb, int fcg, double *sc) {
 __global__ void k_kr_init(int nb, double *sc) {
   int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c < nb) kr_init(sc + c * SC_N);
-}
-
-// x += alpha_c p ; r -= alpha_c q   (segment-per-workgroup, block-aware)
-template <class T>
-__global__ void __launch_bounds__(256) k_kr_update(T *x, T *r, const T *p, const T *q,
-                                                   const int64_t *lo, const int64_t *hi,
-                                                   const int32_t *segblk, const double *sc) {
-  const int s = blockIdx.x;
-  const double a = sc[segblk[s] * SC_N + SC_ALPHA];
-  if (a == 0.0) return;
-  const T at = (T)a;
-  for (int64_t i = lo[s] + threadIdx.x; i < hi[s]; i += 256) {
-    x[i] += at * p[i];
-    r[i] -= at * q[i];
-  }
-}
-// p = z + beta_c p
-template <class T>
-__global__ void __launch_bounds__(256) k_kr_pupdate(T *p, const T *z, const int64_t *lo,
-                                                    const int64_t *hi, const int32_t *segblk,
-                                                    const double *sc) {
-  const int s = blockIdx.x;
-  const T b = (T)sc[segblk[s] * SC_N + SC_BETA];
-  for (int64_t i = lo[s] + threadIdx.x; i < hi[s]; i += 256) p[i] = z[i] + b * p[i];
 }
 
 // FGMRES: y += sum_t coef[blk * K + t] V_t (V_t = V + t ld), added in t order
@@ -190,6 +168,11 @@ struct Solver {
     const void *r, *z;
   };
   std::vector<std::pair<GraphKey, hipGraphExec_t>> graphs;
+  // captured outer iterations, keyed by everything they read or write that
+  // another solve may have moved
+  std::vector<std::pair<std::array<const void *, 9>, hipGraphExec_t>> it_graphs;
+  PinnedBuf<KrHost> kr_host;         // per block, written by the norm kernel
+  DevBuf<unsigned long long> kr_seq;
   // fused coarse tail: levels tail_l0.. (H.size(): none), the row
   // schedules of their operators (A, P, R, M per level), the device tables
   // the programs index, and one recorded program per entry level and
@@ -215,6 +198,7 @@ struct Solver {
 
   ~Solver() {
     for (auto &g : graphs) (void)hipGraphExecDestroy(g.second);
+    for (auto &g : it_graphs) (void)hipGraphExecDestroy(g.second);
     if (s) (void)hipStreamDestroy(s);
   }
 
@@ -964,7 +948,10 @@ struct Solver {
     TailInstr I = ti(TI_KR_INIT);
     I.lvl = (int32_t)lvl;
     c.push_back(I);
-    rec_spmv<T>(c, lvl, 0, x, TE_RESID, b, K.r.p);
+    TailInstr Z = ti(TI_COPY, n);  // the residual of x = 0
+    Z.p[0] = K.r.p;
+    Z.p[1] = b;
+    c.push_back(Z);
     rec_dots<T>(c, lvl, 2, b, b, K.r.p, K.r.p, SC_BN2, SC_RN2, TP_CHECK);
     rec_precond<T>(c, lvl, K.r.p, K.z.p);
     TailInstr C = ti(TI_COPY, n);
@@ -1254,86 +1241,131 @@ struct Solver {
     // K-cycle: kcycle_iters steps of FCG on the next level (multigrid.hpp:113-126)
     LevelWork<T> &wn = work<T>(l + 1);
     KWork<T> &K = wn.kw;
-    fill_zero<T>(K.x.p, N.A.n);
-    krylov<T>(l + 1, N.A, K.x.p, bc, K, o.kcycle_ksp_type, o.tol, o.kcycle_iters, false, nullptr,
-              nullptr);
+    krylov<T>(l + 1, N.A, K.x.p, bc, K, o.kcycle_ksp_type, o.tol, o.kcycle_iters);
     return K.x.p;
   }
 
   // ---------------------------------------------------------------- Krylov
-  // CG / FCG on level lvl's matrix with per-block coefficients.  With
-  // host_check the residual norms come back every iteration (outer loop,
-  // history, stopping test); otherwise exactly maxit iterations run with
-  // device-side convergence flags (K-cycle inner solves, no host sync).
+  // CG / FCG from x = 0 on level lvl's matrix with per-block coefficients.
+  // The outer solve reads the residual norms every iteration (history,
+  // stopping test) and replays its iteration from a captured graph; a
+  // K-cycle's inner solve runs exactly maxit iterations with device-side
+  // convergence flags and no host step.
   template <class T>
-  int krylov(size_t lvl, const DCsr &A, T *x, const T *b, KWork<T> &K, int type, double rtol,
-             int maxit, bool host_check, std::vector<double> *hist, int *status,
-             bool outer_prec = false) {
+  void iterate(size_t lvl, const DCsr &A, T *x, KWork<T> &K, bool fcg, double rtol, bool outer_solve, bool norm) {
     const RedPlan &R = red[lvl];
-    const int nb = R.nb;
-    const int64_t n = A.n;
-    const bool fcg = fcg_like(type);
-    hipLaunchKernelGGL(k_kr_init, dim3((nb + 63) / 64), dim3(64), 0, s, nb, K.sc.p);
-    // r = b - A x
-    op_residual<T>(A, x, b, K.r.p, s);
-    dot2<T>(R, b, b, K.r.p, K.r.p, K, SC_BN2, SC_RN2, KP_CHECK, 0, rtol);
-    std::vector<double> hsc;
-    if (status) *status = LIGMG_CONVERGED;
-    if (host_check) {
-      hsc = download(K.sc.p, (size_t)nb * SC_N, s);
-      if (hist) hist->push_back(total_norm(hsc, nb));
-      if (!any_active(hsc, nb)) return 0;
-    }
-    apply_prec<T>(lvl, K.r.p, K.z.p, outer_prec);
-    d2d(K.p.p, K.z.p, n, s);
-    dot1<T>(R, K.r.p, K.z.p, K, SC_GAMMA);
-    int it = 0;
-    while (it < maxit) {
-      op_spmv<T>(A, K.p.p, K.q.p, s);
-      if (fcg) dot2<T>(R, K.p.p, K.q.p, K.p.p, K.r.p, K, SC_DELTA, SC_T1, KP_ALPHA, 1);
-      else dot1<T>(R, K.p.p, K.q.p, K, SC_DELTA, KP_ALPHA, 0);
-      hipLaunchKernelGGL(k_kr_update<T>, dim3(R.nseg), dim3(256), 0, s, x, K.r.p, K.p.p, K.q.p,
-                         R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1, K.sc.p);
-      LG_LAUNCH_CHECK();
-      it++;
-      dot1<T>(R, K.r.p, K.r.p, K, SC_RN2, KP_CHECK, 0, rtol);
-      if (host_check) {
-        hsc = download(K.sc.p, (size_t)nb * SC_N, s);
-        double tn = total_norm(hsc, nb);
-        if (hist) hist->push_back(tn);
-        if (tn != tn) {
-          if (status) *status = LIGMG_DIVERGED_NAN;
-          return it;
-        }
-        if (!any_active(hsc, nb)) return it;
+    const T *w = fcg ? K.q.p : K.r.p;
+    float *r32 = nullptr;
+    bool done = false;
+    if constexpr (std::is_same<T, double>::value) {
+      if (outer_solve && mixed) {
+        r32 = W32[lvl].b.p;
+        kr_center<double, float>(R, K.z.p, cycle<float>(lvl, r32), w, s);
+        done = true;
       }
-      if (it >= maxit) break;
-      apply_prec<T>(lvl, K.r.p, K.z.p, outer_prec);
-      if (fcg) dot1<T>(R, K.z.p, K.q.p, K, SC_T1, KP_BETA, 1);
-      else dot1<T>(R, K.r.p, K.z.p, K, SC_GN, KP_BETA, 0);
-      hipLaunchKernelGGL(k_kr_pupdate<T>, dim3(R.nseg), dim3(256), 0, s, K.p.p, K.z.p, R.seg_lo.p,
-                         R.seg_hi.p, R.bseg.p + R.nb + 1, K.sc.p);
-      LG_LAUNCH_CHECK();
     }
-    if (host_check && status) *status = LIGMG_DIVERGED_ITS;
-    return it;
+    // PETSc removes the attached nullspace from preconditioned vectors
+    // (util.hpp:530-534): z is the cycle's result minus its block means
+    if (!done) kr_center<T, T>(R, K.z.p, cycle<T>(lvl, K.r.p), w, s);
+    kr_pupdate<T>(R, K.p.p, K.z.p, K.sc.p, fcg, s);
+    op_spmv<T>(A, K.p.p, K.q.p, s);
+    kr_dots<T>(R, K.p.p, K.q.p, fcg ? K.r.p : nullptr, s);
+    kr_update<T>(R, x, K.r.p, K.p.p, K.q.p, K.sc.p, fcg, r32, s);
+    if (norm) kr_norm(R, K.sc.p, false, rtol, outer_solve ? kr_host.p : nullptr, kr_seq.p, s);
   }
 
+  // the K-cycle's inner solve
   template <class T>
-  void apply_prec(size_t lvl, const T *r, T *z, bool outer_prec) {
-    if constexpr (std::is_same<T, double>::value) {
-      if (outer_prec) {
-        precond_outer(lvl, r, z);
-        return;
+  void krylov(size_t lvl, const DCsr &A, T *x, const T *b, KWork<T> &K, int type, double rtol, int maxit) {
+    kr_begin<T>(red[lvl], b, x, K.r.p, nullptr, s);
+    kr_norm(red[lvl], K.sc.p, true, rtol, nullptr, nullptr, s);
+    for (int it = 0; it < maxit; it++) iterate<T>(lvl, A, x, K, fcg_like(type), rtol, false, it + 1 < maxit);
+  }
+
+  // Waits for the seq-th norm of the running outer solve and returns the
+  // residual norm over all blocks; active: whether any block still iterates.
+  double wait_norm(int nb, unsigned long long seq, bool *active) {
+    double t = 0;
+    *active = false;
+    for (int c = 0; c < nb; c++) {
+      volatile KrHost *h = kr_host.p + c;
+      for (uint64_t spins = 1; h->seq < seq; spins++) {
+        if (spins % 4096) continue;
+        const hipError_t e = hipStreamQuery(s);  // a failed or finished stream ends the wait
+        if (e == hipErrorNotReady) continue;
+        LG_HIP(e);
+        LG_CHECK(h->seq >= seq, LIGMG_ERR_DEVICE, "residual norm missing after its launch");
       }
+      std::atomic_thread_fence(std::memory_order_acquire);
+      t += h->rn2;
+      *active |= h->active != 0;
     }
-    precond<T>(lvl, r, z);
+    return std::sqrt(t);
+  }
+
+  int krylov_solve(size_t lvl, double *x, const double *b, KWork<double> &K, std::vector<double> &hist, int *status) {
+    const RedPlan &R = red[lvl];
+    const DCsr &A = H[lvl].A;
+    const bool fcg = fcg_like(o.outer_ksp_type);
+    kr_host.ensure((size_t)R.nb);
+    kr_seq.ensure((size_t)R.nb);
+    for (int c = 0; c < R.nb; c++) kr_host.p[c].seq = 0;  // the stream is idle here
+    std::atomic_thread_fence(std::memory_order_release);
+    kr_begin<double>(R, b, x, K.r.p, mixed ? W32[lvl].b.p : nullptr, s);
+    kr_norm(R, K.sc.p, true, o.tol, kr_host.p, kr_seq.p, s);
+    *status = LIGMG_CONVERGED;
+    bool active = false;
+    hist.push_back(wait_norm(R.nb, 1, &active));
+    if (!active) return 0;
+    for (int it = 1; it <= o.iters; it++) {
+      if (!o.use_graphs) iterate<double>(lvl, A, x, K, fcg, o.tol, true, true);
+      else LG_HIP(hipGraphLaunch(iteration_graph(lvl, A, x, K, fcg), s));
+      const double tn = wait_norm(R.nb, (unsigned long long)it + 1, &active);
+      hist.push_back(tn);
+      if (tn != tn) {
+        *status = LIGMG_DIVERGED_NAN;
+        return it;
+      }
+      if (!active) return it;
+    }
+    *status = LIGMG_DIVERGED_ITS;
+    return o.iters;
+  }
+
+  // the outer iteration from level lvl on these vectors, captured once
+  hipGraphExec_t iteration_graph(size_t lvl, const DCsr &A, double *x, KWork<double> &K, bool fcg) {
+    const std::array<const void *, 9> key = {&A, x, K.r.p, K.z.p, K.p.p, K.q.p, K.sc.p, kr_host.p, kr_seq.p};
+    for (auto &g : it_graphs)
+      if (g.first == key) return g.second;
+    hipGraphExec_t e = capture([&] { iterate<double>(lvl, A, x, K, fcg, o.tol, true, true); });
+    it_graphs.push_back({key, e});
+    return e;
+  }
+
+  template <class F>
+  hipGraphExec_t capture(const F &f) {
+    hipGraph_t graph;
+    {
+      PoolCaptureScope cap;
+      LG_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+      try {
+        f();
+      } catch (...) {
+        (void)hipStreamEndCapture(s, &graph);
+        throw;
+      }
+      LG_HIP(hipStreamEndCapture(s, &graph));
+    }
+    hipGraphExec_t exec;
+    const hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(graph);
+    LG_HIP(e);
+    return exec;
   }
 
   int krylov_outer(size_t base, const double *rhs, std::vector<double> &h, int *status) {
     if (o.outer_ksp_type == LIGMG_KSP_FGMRES) return fgmres(base, outer.x.p, rhs, &h, status);
-    return krylov<double>(base, H[base].A, outer.x.p, rhs, outer, o.outer_ksp_type, o.tol, o.iters,
-                          true, &h, status, true);
+    return krylov_solve(base, outer.x.p, rhs, outer, h, status);
   }
 
   // FGMRES(m) outer solve: restarted flexible GMRES with PETSc KSPFGMRES's
@@ -1421,7 +1453,7 @@ struct Solver {
       bool done = false;
       for (int j = 0; j < m; j++) {
         d2d(K.r.p, V(j), n, s);
-        apply_prec<double>(lvl, K.r.p, K.z.p, true);
+        precond_outer(lvl, K.r.p, K.z.p);
         d2d(Z(j), K.z.p, n, s);
         op_spmv<double>(A, Z(j), V(j + 1), s);
         // classical Gram-Schmidt: h_i = <w, v_i>, i <= j, four at a time
@@ -1509,45 +1541,13 @@ struct Solver {
     }
   }
 
-  static double total_norm(const std::vector<double> &hsc, int nb) {
-    double t = 0;
-    for (int c = 0; c < nb; c++) t += hsc[c * SC_N + SC_RN2];
-    return std::sqrt(t);
-  }
   static bool any_active(const std::vector<double> &hsc, int nb) {
     for (int c = 0; c < nb; c++)
       if (hsc[c * SC_N + SC_ACTIVE] != 0) return true;
     return false;
   }
 
-  template <class T>
-  // dot products into the scalar slots, followed in the same launch by the
-  // scalar step post (KrPost)
-  void dot1(const RedPlan &R, const T *a, const T *b, KWork<T> &K, int slot, int post = KP_NONE, int fcg = 0,
-            double rtol = 0) {
-    const T *A_[1] = {a}, *B_[1] = {b};
-    R.dots_sc<T>(1, A_, B_, K.sc.p, slot, slot, post, fcg, rtol, s);
-  }
-  template <class T>
-  void dot2(const RedPlan &R, const T *a0, const T *b0, const T *a1, const T *b1, KWork<T> &K, int s0,
-            int s1, int post = KP_NONE, int fcg = 0, double rtol = 0) {
-    const T *A_[2] = {a0, a1}, *B_[2] = {b0, b1};
-    R.dots_sc<T>(2, A_, B_, K.sc.p, s0, s1, post, fcg, rtol, s);
-  }
-
-  // z = M r with the constant removed per block (PETSc removes the attached
-  // nullspace from preconditioned vectors; util.hpp:530-534)
-  template <class T>
-  void precond(size_t lvl, const T *r, T *z) {
-    const int64_t n = H[lvl].A.n;
-    const T *c = cycle<T>(lvl, r);
-    d2d(z, c, n, s);
-    const RedPlan &R = red[lvl];
-    R.sums<T>(z, dsc.p, s);
-    op_sub_block_mean<T>(z, R, dsc.p, s);
-  }
-
-  // outer preconditioner in FP64, cycle in FP32 when mixed.  With
+  // FGMRES: outer preconditioner in FP64, cycle in FP32 when mixed.  With
   // o.use_graphs the whole application (hundreds of launches on the coarse
   // levels) is captured once per (level, r, z) and replayed as a hipGraph;
   // it contains no host synchronisation and no memset nodes.
@@ -1558,21 +1558,7 @@ struct Solver {
           LG_HIP(hipGraphLaunch(g.second, s));
           return;
         }
-      hipGraph_t graph;
-      {
-        PoolCaptureScope cap;
-        LG_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        try {
-          precond_outer_eager(lvl, r, z);
-        } catch (...) {
-          (void)hipStreamEndCapture(s, &graph);
-          throw;
-        }
-        LG_HIP(hipStreamEndCapture(s, &graph));
-      }
-      hipGraphExec_t exec;
-      LG_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-      (void)hipGraphDestroy(graph);
+      const hipGraphExec_t exec = capture([&] { precond_outer_eager(lvl, r, z); });
       graphs.push_back({{lvl, r, z}, exec});
       LG_HIP(hipGraphLaunch(exec, s));
       return;
@@ -2050,6 +2036,7 @@ int Solver::solve(const double *b, double *x, int mem, ligmg_info *info, double 
   // caller order -> solve layout: the input permutation and level 0's
   // layout for level 0, the level's own layout below it
   const int32_t *ip = from == 0 ? perm.p : L0.sperm.p;
+  LG_HIP(hipStreamSynchronize(s));  // idle, unless an earlier solve failed
   if (ip) {
     const double *src = b;
     if (mem == LIGMG_MEM_HOST) {
@@ -2062,7 +2049,6 @@ int Solver::solve(const double *b, double *x, int mem, ligmg_info *info, double 
   } else {
     d2d(b0.p, b, n, s);
   }
-  LG_HIP(hipStreamSynchronize(s));
   auto t0 = std::chrono::steady_clock::now();
   const bool do_once = o.top_elim && L0.kind == LIGMG_LEVEL_ELIM;
   const size_t base = do_once ? (size_t)from + 1 : (size_t)from;
@@ -2076,7 +2062,7 @@ int Solver::solve(const double *b, double *x, int mem, ligmg_info *info, double 
   else d2d(rhs, b0.p, n, s);
   red[base].sums<double>(rhs, dsc.p, s);
   op_sub_block_mean<double>(rhs, red[base], dsc.p, s);
-  fill_zero<double>(outer.x.p, nb_);
+  if (o.outer_ksp_type == LIGMG_KSP_FGMRES) fill_zero<double>(outer.x.p, nb_);
   std::vector<double> h;
   int status = 0;
   // the outer loop always runs in FP64 (custom preconditioner bridge)
@@ -2090,12 +2076,6 @@ int Solver::solve(const double *b, double *x, int mem, ligmg_info *info, double 
   const double *A_[2] = {tmp0.p, b0.p}, *B_[2] = {tmp0.p, b0.p};
   RedPlan &R0 = red[from];
   R0.dots<double>(2, A_, B_, dsc.p, s);
-  std::vector<double> d = download(dsc.p, 2 * R0.nb, s);
-  double rr = 0, bb = 0;
-  for (int c = 0; c < R0.nb; c++) {
-    rr += d[c * 2];
-    bb += d[c * 2 + 1];
-  }
   if (ip) {
     if (mem == LIGMG_MEM_HOST) {
       scatter_vec(n, ip, sol.p, tmp0.p, s);
@@ -2108,7 +2088,12 @@ int Solver::solve(const double *b, double *x, int mem, ligmg_info *info, double 
   } else {
     d2d(x, sol.p, n, s);
   }
-  LG_HIP(hipStreamSynchronize(s));
+  const std::vector<double> d = download(dsc.p, 2 * R0.nb, s);  // waits for all of it
+  double rr = 0, bb = 0;
+  for (int c = 0; c < R0.nb; c++) {
+    rr += d[c * 2];
+    bb += d[c * 2 + 1];
+  }
   if (info) {
     // cycle_complexity (multigrid.hpp:372-387): the work of the levels from
     // the base level down, over the nnz of level 0 whatever `from` is;
