@@ -48,6 +48,23 @@ __host__ __device__ inline int row_lanes(int64_t cnt, int64_t nr, int items) {
 constexpr int64_t ROW_ITEMS_BIG_NNZ = (int64_t)16 << 20;
 inline int row_items_for(int64_t nnz) { return nnz >= ROW_ITEMS_BIG_NNZ ? 16 : 4; }
 
+// Whether an operator's rows go straight to groups of K lanes (k_spmv_rows)
+// instead of staged units: K by the mean row length, at most ROW_ROUNDS
+// rounds of ROW_U entries a lane for the longest row.  Small operators are a
+// chain of latencies, which the row kernel shortens (Chebyshev step of a
+// 65 K-vertex grid's levels 6.3 -> 3.7 us, a 97-workgroup interpolation 4.0 ->
+// 2.7 us); large ones are bound by cache accesses, which the units' coalesced
+// streams save (9.1 M entries: 81 us staged, 88 us by rows; at 1.2 M the rows
+// still win).
+constexpr int ROW_U = 4;
+constexpr int ROW_ROUNDS = 8;
+constexpr int64_t ROW_MAX_NNZ = (int64_t)2 << 20;
+inline int row_kernel_lanes(int64_t n, int64_t nnz, int64_t longest) {
+  if (n == 0 || nnz == 0 || nnz > ROW_MAX_NNZ) return 0;
+  const int K = row_lanes(nnz, n, ROW_U);
+  return longest <= (int64_t)ROW_ROUNDS * ROW_U * K ? K : 0;
+}
+
 struct Units {
   int64_t nunits = 0, nlong = 0, nparts = 0;
   DevBuf<int32_t> row0;   // first row
@@ -57,6 +74,9 @@ struct Units {
   DevBuf<int32_t> lpart;  // nlong + 1 slot offsets
   DevBuf<double> parts;   // partial sums (also used as float storage)
   int32_t row_items = 4;  // entries per lane of the row reduction (row_items_for)
+  // lanes per row of the row kernel (k_spmv_rows) when the operator's rows
+  // suit it, else 0: the units above
+  int32_t row_k = 0;
   // batched SpMM tile picked per precision (0 FP64, 1 FP32) and log2 of the
   // block width; -1 until tuned (the fixed tile is used)
   int8_t spmm_cfg[2][8] = {{-1, -1, -1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1, -1, -1}};

@@ -28,6 +28,16 @@ void make_v32(DCsr &A, hipStream_t s, bool laplacian = false);
 
 // y = A x
 template <class T> void op_spmv(const DCsr &A, const T *x, T *y, hipStream_t s);
+// The first Chebyshev step of the cycle that takes y as its right-hand side,
+// x = beta dinv y, written by y's producer (null x: none).
+template <class T>
+struct FirstStep {
+  const T *dinv = nullptr;
+  T *x = nullptr;
+  double beta = 0;
+};
+template <class T>
+void op_spmv_first(const DCsr &A, const T *x, T *y, const FirstStep<T> &f, hipStream_t s);
 // r = b - A x
 template <class T> void op_residual(const DCsr &A, const T *x, const T *b, T *r, hipStream_t s);
 // One Chebyshev step: xn = xc + alpha (xc - xp) + beta dinv (b - A xc).
@@ -41,6 +51,10 @@ void op_interp(const DCsr &P, const T *q, const T *xc, const T *b, T *x, hipStre
 // x[i] += xc[agg[i]]
 template <class T>
 void op_prolong_add(const int32_t *agg, int64_t n, const T *xc, T *x, hipStream_t s);
+// x[i] += (P xc + q b)[agg[i]], for P of short rows (row_k 1)
+template <class T>
+void op_prolong_interp(const int32_t *agg, int64_t n, const DCsr &P, const T *q, const T *xc, const T *b, T *x,
+                       hipStream_t s);
 // y = pinv x (dense n x n, FP64 matrix; T vectors)
 template <class T>
 void op_dense_apply(const double *Pinv, int64_t n, const T *x, T *y, hipStream_t s);
@@ -88,9 +102,10 @@ struct KrHost {
 // One Krylov iteration on a level (sc: SC_N scalars per block): the start
 // from x = 0, the norm of r with the convergence flag, then z = c - mean
 // (with z.w: q for FCG, r for CG), p = z + beta p, the dots of q = A p (r only
-// for FCG), and x += alpha p, r -= alpha q.  r32: also r in FP32.
-template <class T>
-void kr_begin(const RedPlan &R, const T *b, T *x, T *r, float *r32, hipStream_t s);
+// for FCG), and x += alpha p, r -= alpha q.  rf: also r in the cycle's type F;
+// f: the cycle's first step from r.
+template <class T, class F>
+void kr_begin(const RedPlan &R, const T *b, T *x, T *r, F *rf, const FirstStep<F> &f, hipStream_t s);
 void kr_norm(const RedPlan &R, double *sc, bool init, double rtol, KrHost *host, unsigned long long *seq,
              hipStream_t s);
 template <class T, class C>
@@ -99,8 +114,9 @@ template <class T>
 void kr_pupdate(const RedPlan &R, T *p, const T *z, double *sc, bool fcg, hipStream_t s);
 template <class T>
 void kr_dots(const RedPlan &R, const T *p, const T *q, const T *r, hipStream_t s);
-template <class T>
-void kr_update(const RedPlan &R, T *x, T *r, const T *p, const T *q, double *sc, bool fcg, float *r32, hipStream_t s);
+template <class T, class F>
+void kr_update(const RedPlan &R, T *x, T *r, const T *p, const T *q, double *sc, bool fcg, F *rf,
+               const FirstStep<F> &f, hipStream_t s);
 
 // a -= mean of a over each block, means taken from sums[c] (device)
 template <class T> void op_sub_block_mean(T *a, const RedPlan &P, const double *sums, hipStream_t s);

@@ -18,16 +18,30 @@ using namespace sdev;
 // the last one hands accumulator + its own sum to the real epilogue
 struct EpiAccSet {
   double *acc;
+  struct Pre {};
+  __device__ __forceinline__ Pre load(int64_t) const { return {}; }
+  __device__ __forceinline__ void put(int64_t i, double s, const Pre &) const { acc[i] = s; }
   __device__ __forceinline__ void operator()(int64_t i, double s) const { acc[i] = s; }
 };
 struct EpiAccAdd {
   double *acc;
+  struct Pre {
+    double a;
+  };
+  __device__ __forceinline__ Pre load(int64_t i) const { return {acc[i]}; }
+  __device__ __forceinline__ void put(int64_t i, double s, const Pre &p) const { acc[i] = p.a + s; }
   __device__ __forceinline__ void operator()(int64_t i, double s) const { acc[i] += s; }
 };
 template <class Epi>
 struct EpiAccFinal {
   const double *acc;
   Epi e;
+  struct Pre {
+    double a;
+    typename Epi::Pre e;
+  };
+  __device__ __forceinline__ Pre load(int64_t i) const { return {acc[i], e.load(i)}; }
+  __device__ __forceinline__ void put(int64_t i, double s, const Pre &p) const { e.put(i, p.a + s, p.e); }
   __device__ __forceinline__ void operator()(int64_t i, double s) const { e(i, acc[i] + s); }
 };
 
@@ -148,6 +162,39 @@ __global__ void __launch_bounds__(SPMV_BLOCK)
   }
 }
 
+// Operators of short, even rows: a group of K = 1 << lk lanes per row, straight from
+// memory.  A row is one round of ROW_U entries a lane in flight (masked past
+// its end) with its epilogue operands asked for at the start, a chain of
+// three loads; the staged units above take seven and two barriers.  The sum is
+// theirs: K strided partials and an xor butterfly.
+template <class T, class Val, class Epi>
+__global__ void __launch_bounds__(256) k_spmv_rows(int64_t n, const int32_t *__restrict__ rp,
+                                                   const int32_t *__restrict__ ci, Val val,
+                                                   const T *__restrict__ x, int lk, Epi epi) {
+  const int64_t row = (blockIdx.x * (int64_t)256 + threadIdx.x) >> lk;
+  const int K = 1 << lk, g = threadIdx.x & (K - 1);
+  double s = 0;
+  typename Epi::Pre pre;
+  if (row < n) {
+    const int a = rp[row] + g, b = rp[row + 1];
+    if (g == 0) pre = epi.load(row);
+    for (int k = a; k < b; k += K * ROW_U) {
+      T xx[ROW_U], vv[ROW_U];
+#pragma unroll
+      for (int t = 0; t < ROW_U; t++) {
+        const int e = k + t * K < b ? k + t * K : k;
+        xx[t] = x[ci[e]];
+        vv[t] = val(e);
+      }
+#pragma unroll
+      for (int t = 0; t < ROW_U; t++)
+        if (k + t * K < b) s += (double)vv[t] * (double)xx[t];
+    }
+  }
+  s = group_sum(s, K);
+  if (row < n && g == 0) epi.put(row, s, pre);
+}
+
 // One wavefront per long row: its chunk partials added left to right from
 // 0.0 (wave_seq_fold keeps a block of partials in flight; one lane per row
 // waited on each load in turn).
@@ -165,6 +212,13 @@ __global__ void __launch_bounds__(256) k_spmv_long(const int32_t *lrow, const in
 template <class T, class Val, class Epi>
 void launch_spmv(const DCsr &A, Val val, const T *x, Epi epi, hipStream_t s) {
   if (A.U.nunits == 0) return;
+  if (A.U.row_k) {
+    const int lk = __builtin_ctz(A.U.row_k);
+    hipLaunchKernelGGL((k_spmv_rows<T, Val, Epi>), dim3((unsigned)((A.n * A.U.row_k + 255) / 256)), dim3(256), 0, s,
+                       A.n, A.rp.p, A.ci.p, val, x, lk, epi);
+    LG_LAUNCH_CHECK();
+    return;
+  }
   double *parts = A.U.parts.p;
   const int upw = spmv_upw(A.U.nunits);
   const int64_t grid = (A.U.nunits + upw - 1) / upw;
@@ -241,6 +295,36 @@ __global__ void k_prolong_add(const int32_t *agg, int64_t n, const T *xc, T *x) 
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
     x[i] += xc[agg[i]];
+}
+
+// x[i] += e[agg[i]] with e = P xc + q b of the elimination level below: the
+// entries of the vertex's P row (at most a few) in order, e rounded as its own
+// vector would be.  One launch (2-5 us) and that vector's round trip less than
+// interpolating first.
+template <class T>
+__global__ void __launch_bounds__(256) k_prolong_interp(const int32_t *__restrict__ agg, int64_t n,
+                                                        const int32_t *__restrict__ rp,
+                                                        const int32_t *__restrict__ ci, const T *__restrict__ v,
+                                                        const T *__restrict__ q, const T *__restrict__ xc,
+                                                        const T *__restrict__ b, T *__restrict__ x) {
+  const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (i >= n) return;
+  const int c = agg[i], k0 = rp[c], k1 = rp[c + 1];
+  const T xi = x[i], qc = q[c], bc = b[c];
+  double s = 0;
+  for (int k = k0; k < k1; k += ROW_U) {
+    T xx[ROW_U], vv[ROW_U];
+#pragma unroll
+    for (int t = 0; t < ROW_U; t++) {
+      const int e = k + t < k1 ? k + t : k;
+      xx[t] = xc[ci[e]];
+      vv[t] = v[e];
+    }
+#pragma unroll
+    for (int t = 0; t < ROW_U; t++)
+      if (k + t < k1) s += (double)vv[t] * (double)xx[t];
+  }
+  x[i] = xi + (T)(s + (double)qc * (double)bc);
 }
 
 // Laplacian-form FP32 copy: off-diagonals rounded, diagonal slot 0, and the
@@ -362,18 +446,25 @@ __device__ __forceinline__ void block_partials(const int32_t *bseg, int c, const
   }
 }
 
-// x = 0, r = b (the residual of a zero iterate), the partials of b.b
-template <class T>
-__global__ void __launch_bounds__(256) k_kr_begin(const T *b, T *x, T *r, float *r32, const int64_t *lo,
+// x = 0, r = b (the residual of a zero iterate), the partials of b.b; rf and
+// f as in kr_update
+template <class T, class F>
+__global__ void __launch_bounds__(256) k_kr_begin(const T *b, T *x, T *r, F *rf, FirstStep<F> f, const int64_t *lo,
                                                   const int64_t *hi, double *part) {
   const int s = blockIdx.x;
   double acc = 0;
   T v[RED_BATCH];
-  seg_items(lo[s], hi[s], threadIdx.x, [&](int t, int64_t i) { v[t] = b[i]; },
+  F dv[RED_BATCH];
+  seg_items(lo[s], hi[s], threadIdx.x,
+            [&](int t, int64_t i) {
+              v[t] = b[i];
+              if (f.x) dv[t] = f.dinv[i];
+            },
             [&](int t, int64_t i) {
               x[i] = (T)0;
               r[i] = v[t];
-              if (r32) r32[i] = (float)v[t];
+              if (rf) rf[i] = (F)v[t];
+              if (f.x) f.x[i] = cheb_first<F>(f.beta, dv[t], (F)v[t]);
               acc += (double)v[t] * (double)v[t];
             });
   __shared__ double ws[4];
@@ -433,9 +524,10 @@ __global__ void __launch_bounds__(256) k_kr_dots(const T *p, const T *q, const T
 }
 
 // alpha = (FCG: p.r, CG: r.z) / p.q; x += alpha p, r -= alpha q, the
-// partials of r.r, and r in FP32 when r32 is set
-template <class T>
-__global__ void __launch_bounds__(256) k_kr_update(T *x, T *r, const T *p, const T *q, float *r32,
+// partials of r.r; with rf set r in the cycle's type, with f.x set the cycle's
+// first step from r
+template <class T, class F>
+__global__ void __launch_bounds__(256) k_kr_update(T *x, T *r, const T *p, const T *q, F *rf, FirstStep<F> f,
                                                    const int64_t *lo, const int64_t *hi, const int32_t *segblk,
                                                    const int32_t *bseg, double *part, double *sc, int fcg) {
   __shared__ double qs[2][WAVE], ws[4];
@@ -454,9 +546,11 @@ __global__ void __launch_bounds__(256) k_kr_update(T *x, T *r, const T *p, const
   const T at = (T)a;
   double acc = 0;
   T xv[RED_BATCH], rv[RED_BATCH], pv[RED_BATCH], qv[RED_BATCH];
+  F dv[RED_BATCH];
   seg_items(lo[s], hi[s], threadIdx.x,
             [&](int t, int64_t i) {
               rv[t] = r[i];
+              if (f.x) dv[t] = f.dinv[i];
               if (a != 0.0) {
                 xv[t] = x[i];
                 pv[t] = p[i];
@@ -469,7 +563,8 @@ __global__ void __launch_bounds__(256) k_kr_update(T *x, T *r, const T *p, const
                 rv[t] -= at * qv[t];
                 r[i] = rv[t];
               }
-              if (r32) r32[i] = (float)rv[t];
+              if (rf) rf[i] = (F)rv[t];
+              if (f.x) f.x[i] = cheb_first<F>(f.beta, dv[t], (F)rv[t]);
               acc += (double)rv[t] * (double)rv[t];
             });
   const double sum = block_sum(acc, ws);
@@ -694,6 +789,14 @@ __global__ void k_unit_chain(int64_t M, const int32_t *J, int K, int64_t stride,
     islong[m] = lng ? 1 : 0;
   }
 }
+// longest: the largest row length (zeroed before)
+__global__ void __launch_bounds__(256) k_longest_row(int64_t n, const int32_t *rp, int32_t *longest) {
+  int32_t m = 0;
+  for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x)
+    m = max(m, rp[r + 1] - rp[r]);
+  for (int off = WAVE / 2; off >= 1; off >>= 1) m = max(m, __shfl_xor(m, off, WAVE));
+  if ((threadIdx.x & (WAVE - 1)) == 0) atomicMax(longest, m);
+}
 __global__ void k_unit_fill(int64_t M, const int32_t *start, const int32_t *J0, const int32_t *rp,
                             const int32_t *uoff, const int32_t *poff, const int32_t *loff, const int32_t *islong,
                             int32_t *row0, int32_t *nrows, int32_t *koff, int32_t *lrow, int32_t *lpart) {
@@ -766,6 +869,9 @@ void build_units_host(DCsr &A, hipStream_t s) {
     r = r1;
   }
   lpart.push_back((int32_t)parts);
+  int64_t longest = 0;
+  for (int64_t i = 0; i < n; i++) longest = std::max<int64_t>(longest, rp[i + 1] - rp[i]);
+  A.U.row_k = row_kernel_lanes(n, rp[n] - rp[0], longest);
   set_units(A.U, rp[n] - rp[0], row0, nrows, koff, lrow, lpart, parts, s);
 }
 
@@ -808,10 +914,16 @@ void build_units(DCsr &A, hipStream_t s) {
   const int64_t parts = exclusive_scan_i32(pcnt.p, poff.p, M + 1, s);
   const int64_t nlong = exclusive_scan_i32(islong.p, loff.p, M + 1, s);
   Units &U = A.U;
-  int32_t ends[2];
+  DevBuf<int32_t> longest(1);
+  fill_i32(longest.p, 0, 1, s);
+  hipLaunchKernelGGL(k_longest_row, dim3(grid_for(n, 256, 256)), dim3(256), 0, s, n, A.rp.p, longest.p);
+  LG_LAUNCH_CHECK();
+  int32_t ends[3];
   to_host(&ends[0], A.rp.p, 1, s);
   to_host(&ends[1], A.rp.p + n, 1, s);
+  to_host(&ends[2], longest.p, 1, s);
   LG_HIP(hipStreamSynchronize(s));
+  U.row_k = row_kernel_lanes(n, (int64_t)ends[1] - ends[0], ends[2]);
   U.nunits = nunits;
   U.row_items = row_items_for((int64_t)ends[1] - ends[0]);
   U.nlong = nlong;
@@ -945,6 +1057,12 @@ void op_spmv(const DCsr &A, const T *x, T *y, hipStream_t s) {
 }
 
 template <class T>
+void op_spmv_first(const DCsr &A, const T *x, T *y, const FirstStep<T> &f, hipStream_t s) {
+  if (f.x) dispatch_spmv<T>(A, x, EpiFirst<T>{y, f.dinv, f.x, f.beta}, s);
+  else op_spmv<T>(A, x, y, s);
+}
+
+template <class T>
 void op_residual(const DCsr &A, const T *x, const T *b, T *r, hipStream_t s) {
   dispatch_spmv<T>(A, x, EpiResid<T>{b, r}, s);
 }
@@ -973,6 +1091,16 @@ void op_prolong_add(const int32_t *agg, int64_t n, const T *xc, T *x, hipStream_
 }
 
 template <class T>
+void op_prolong_interp(const int32_t *agg, int64_t n, const DCsr &P, const T *q, const T *xc, const T *b, T *x,
+                       hipStream_t s) {
+  const T *v = vals_of<T>(P);
+  LG_CHECK(v && P.U.row_k == 1, LIGMG_ERR_INVALID, "prolong_interp: P must have values and short rows");
+  hipLaunchKernelGGL(k_prolong_interp<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, agg, n, P.rp.p, P.ci.p, v,
+                     q, xc, b, x);
+  LG_LAUNCH_CHECK();
+}
+
+template <class T>
 void op_dense_apply(const double *Pm, int64_t n, const T *x, T *y, hipStream_t s) {
   hipLaunchKernelGGL(k_dense_apply<T>, dim3(grid_for(n * WAVE, 256)), dim3(256), 0, s, Pm, n, x, y);
   LG_LAUNCH_CHECK();
@@ -989,6 +1117,9 @@ void op_f2d(const float *a, double *b, int64_t n, hipStream_t s) {
 
 #define LG_INST(T)                                                                                \
   template void op_spmv<T>(const DCsr &, const T *, T *, hipStream_t);                            \
+  template void op_spmv_first<T>(const DCsr &, const T *, T *, const FirstStep<T> &, hipStream_t); \
+  template void op_prolong_interp<T>(const int32_t *, int64_t, const DCsr &, const T *, const T *, \
+                                     const T *, T *, hipStream_t);                                \
   template void op_residual<T>(const DCsr &, const T *, const T *, T *, hipStream_t);             \
   template void op_cheb_step<T>(const DCsr &, const T *, const T *, const T *, const T *, T *,    \
                                 double, double, hipStream_t);                                     \
@@ -1080,9 +1211,9 @@ template void RedPlan::dots<float>(int, const float *const *, const float *const
 template void RedPlan::sums<double>(const double *, double *, hipStream_t) const;
 template void RedPlan::sums<float>(const float *, double *, hipStream_t) const;
 #define LG_SEGS dim3((unsigned)R.nseg), dim3(256), 0, s
-template <class T>
-void kr_begin(const RedPlan &R, const T *b, T *x, T *r, float *r32, hipStream_t s) {
-  hipLaunchKernelGGL(k_kr_begin<T>, LG_SEGS, b, x, r, r32, R.seg_lo.p, R.seg_hi.p, R.part.p);
+template <class T, class F>
+void kr_begin(const RedPlan &R, const T *b, T *x, T *r, F *rf, const FirstStep<F> &f, hipStream_t s) {
+  hipLaunchKernelGGL((k_kr_begin<T, F>), LG_SEGS, b, x, r, rf, f, R.seg_lo.p, R.seg_hi.p, R.part.p);
   LG_LAUNCH_CHECK();
 }
 void kr_norm(const RedPlan &R, double *sc, bool init, double rtol, KrHost *host, unsigned long long *seq,
@@ -1096,9 +1227,10 @@ void kr_dots(const RedPlan &R, const T *p, const T *q, const T *r, hipStream_t s
   hipLaunchKernelGGL(k_kr_dots<T>, LG_SEGS, p, q, r, R.seg_lo.p, R.seg_hi.p, R.part.p);
   LG_LAUNCH_CHECK();
 }
-template <class T>
-void kr_update(const RedPlan &R, T *x, T *r, const T *p, const T *q, double *sc, bool fcg, float *r32, hipStream_t s) {
-  hipLaunchKernelGGL(k_kr_update<T>, LG_SEGS, x, r, p, q, r32, R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1, R.bseg.p,
+template <class T, class F>
+void kr_update(const RedPlan &R, T *x, T *r, const T *p, const T *q, double *sc, bool fcg, F *rf,
+               const FirstStep<F> &f, hipStream_t s) {
+  hipLaunchKernelGGL((k_kr_update<T, F>), LG_SEGS, x, r, p, q, rf, f, R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1, R.bseg.p,
                      R.part.p, sc, fcg ? 1 : 0);
   LG_LAUNCH_CHECK();
 }
@@ -1117,14 +1249,19 @@ void kr_pupdate(const RedPlan &R, T *p, const T *z, double *sc, bool fcg, hipStr
   LG_LAUNCH_CHECK();
 }
 #undef LG_SEGS
-#define LG_KR(T)                                                                                          \
-  template void kr_begin<T>(const RedPlan &, const T *, T *, T *, float *, hipStream_t);                  \
-  template void kr_dots<T>(const RedPlan &, const T *, const T *, const T *, hipStream_t);                \
-  template void kr_update<T>(const RedPlan &, T *, T *, const T *, const T *, double *, bool, float *,    \
-                             hipStream_t);                                                                \
+#define LG_KR(T)                                                                                \
+  template void kr_dots<T>(const RedPlan &, const T *, const T *, const T *, hipStream_t);      \
   template void kr_pupdate<T>(const RedPlan &, T *, const T *, double *, bool, hipStream_t);
 LG_KR(double)
 LG_KR(float)
+#undef LG_KR
+#define LG_KR(T, F)                                                                                               \
+  template void kr_begin<T, F>(const RedPlan &, const T *, T *, T *, F *, const FirstStep<F> &, hipStream_t);     \
+  template void kr_update<T, F>(const RedPlan &, T *, T *, const T *, const T *, double *, bool, F *,            \
+                                const FirstStep<F> &, hipStream_t);
+LG_KR(double, double)
+LG_KR(double, float)
+LG_KR(float, float)
 #undef LG_KR
 template void kr_center<double, double>(const RedPlan &, double *, const double *, const double *, hipStream_t);
 template void kr_center<double, float>(const RedPlan &, double *, const float *, const double *, hipStream_t);

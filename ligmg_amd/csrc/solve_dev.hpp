@@ -27,39 +27,81 @@ struct ValArr {
 // Row sums are always accumulated in FP64 (a product of two FP32 numbers
 // is exact in FP64), so the FP32 path only rounds storage, not the
 // heavily cancelling Laplacian row sums of hub vertices.
+// load(i) reads row i's other operands (asked for before the sum is known
+// where a kernel can), put(i, s, load(i)) writes the result.
 template <class T>
 struct EpiStore {
   T *y;
-  __device__ __forceinline__ void operator()(int64_t r, double s) const { y[r] = (T)s; }
+  struct Pre {};
+  __device__ __forceinline__ Pre load(int64_t) const { return {}; }
+  __device__ __forceinline__ void put(int64_t r, double s, const Pre &) const { y[r] = (T)s; }
+  __device__ __forceinline__ void operator()(int64_t r, double s) const { put(r, s, load(r)); }
+};
+// first Chebyshev step from a zero iterate: xn = beta dinv b
+template <class T>
+__device__ __forceinline__ T cheb_first(double beta, T dinv, T b) {
+  return (T)(beta * (double)dinv * (double)b);
+}
+
+// y = s and the next cycle's first Chebyshev step from y
+template <class T>
+struct EpiFirst {
+  T *y;
+  const T *dinv;
+  T *x;
+  double beta;
+  struct Pre {
+    T dinv;
+  };
+  __device__ __forceinline__ Pre load(int64_t i) const { return {dinv[i]}; }
+  __device__ __forceinline__ void put(int64_t i, double s, const Pre &p) const {
+    const T v = (T)s;
+    y[i] = v;
+    x[i] = cheb_first<T>(beta, p.dinv, v);
+  }
+  __device__ __forceinline__ void operator()(int64_t i, double s) const { put(i, s, load(i)); }
 };
 template <class T>
 struct EpiResid {
   const T *b;
   T *r;
-  __device__ __forceinline__ void operator()(int64_t i, double s) const {
-    r[i] = (T)((double)b[i] - s);
-  }
+  struct Pre {
+    T b;
+  };
+  __device__ __forceinline__ Pre load(int64_t i) const { return {b[i]}; }
+  __device__ __forceinline__ void put(int64_t i, double s, const Pre &p) const { r[i] = (T)((double)p.b - s); }
+  __device__ __forceinline__ void operator()(int64_t i, double s) const { put(i, s, load(i)); }
 };
 template <class T>
 struct EpiCheb {
   const T *dinv, *b, *xc, *xp;
   T *xn;
   double alpha, beta;
-  __device__ __forceinline__ void operator()(int64_t i, double s) const {
-    double c = (double)xc[i];
-    // a null xp is a zero previous iterate (second step from a zero guess);
-    // every other caller passes alpha = 0 with it
-    double d = alpha * (c - (xp ? (double)xp[i] : 0.0));
-    xn[i] = (T)(c + d + beta * (double)dinv[i] * ((double)b[i] - s));
+  struct Pre {
+    T c, p, dinv, b;
+  };
+  // a null xp is a zero previous iterate (second step from a zero guess);
+  // every other caller passes alpha = 0 with it
+  __device__ __forceinline__ Pre load(int64_t i) const { return {xc[i], xp ? xp[i] : (T)0, dinv[i], b[i]}; }
+  __device__ __forceinline__ void put(int64_t i, double s, const Pre &p) const {
+    double c = (double)p.c;
+    double d = alpha * (c - (double)p.p);
+    xn[i] = (T)(c + d + beta * (double)p.dinv * ((double)p.b - s));
   }
+  __device__ __forceinline__ void operator()(int64_t i, double s) const { put(i, s, load(i)); }
 };
 template <class T>
 struct EpiInterp {
   const T *q, *b;
   T *x;
-  __device__ __forceinline__ void operator()(int64_t i, double s) const {
-    x[i] = (T)(s + (double)q[i] * (double)b[i]);
+  struct Pre {
+    T q, b;
+  };
+  __device__ __forceinline__ Pre load(int64_t i) const { return {q[i], b[i]}; }
+  __device__ __forceinline__ void put(int64_t i, double s, const Pre &p) const {
+    x[i] = (T)(s + (double)p.q * (double)p.b);
   }
+  __device__ __forceinline__ void operator()(int64_t i, double s) const { put(i, s, load(i)); }
 };
 // adds d[i] x[i] (FP64) before the wrapped epilogue: the diagonal term of an
 // FP32 operator stored in Laplacian form
@@ -68,16 +110,17 @@ struct EpiDiag {
   const double *d;
   const T *x;
   Epi e;
-  __device__ __forceinline__ void operator()(int64_t i, double s) const {
-    e(i, s + d[i] * (double)x[i]);
+  struct Pre {
+    double d;
+    T x;
+    typename Epi::Pre e;
+  };
+  __device__ __forceinline__ Pre load(int64_t i) const { return {d[i], x[i], e.load(i)}; }
+  __device__ __forceinline__ void put(int64_t i, double s, const Pre &p) const {
+    e.put(i, s + p.d * (double)p.x, p.e);
   }
+  __device__ __forceinline__ void operator()(int64_t i, double s) const { put(i, s, load(i)); }
 };
-
-// first Chebyshev step from a zero iterate: xn = beta dinv b
-template <class T>
-__device__ __forceinline__ T cheb_first(double beta, T dinv, T b) {
-  return (T)(beta * (double)dinv * (double)b);
-}
 
 // xor butterfly: every lane ends with the same bits
 template <class T>

@@ -918,7 +918,7 @@ struct Solver {
   template <class T>
   const T *rec_recurse(std::vector<TailInstr> &c, size_t l, const T *bc) {
     const DLevel &N = H[l + 1];
-    if (!o.kcycle || N.kind == LIGMG_LEVEL_ELIM) return rec_cycle<T>(c, l + 1, bc);
+    if (!inner_krylov(l + 1)) return rec_cycle<T>(c, l + 1, bc);
     KWork<T> &K = work<T>(l + 1).kw;
     TailInstr I = ti(TI_ZERO, N.A.n);
     I.p[0] = K.x.p;
@@ -926,19 +926,15 @@ struct Solver {
     rec_krylov<T>(c, l + 1, K.x.p, bc);
     return K.x.p;
   }
+  // z = precond(r), also to p when set
   template <class T>
-  void rec_precond(std::vector<TailInstr> &c, size_t lvl, const T *r, T *z) {
-    const int64_t n = H[lvl].A.n;
-    const T *cy = rec_cycle<T>(c, lvl, r);
-    TailInstr I = ti(TI_COPY, n);
+  void rec_precond(std::vector<TailInstr> &c, size_t lvl, const T *r, T *z, T *p) {
+    TailInstr I = ti(TI_CENTER);
+    I.lvl = (int32_t)lvl;
     I.p[0] = z;
-    I.p[1] = cy;
+    I.p[1] = rec_cycle<T>(c, lvl, r);
+    I.p[2] = p;
     c.push_back(I);
-    rec_dots<T>(c, lvl, 1, z, nullptr, nullptr, nullptr, -1, -1, TP_NONE);
-    TailInstr M = ti(TI_SUBMEAN, n);
-    M.lvl = (int32_t)lvl;
-    M.p[0] = z;
-    c.push_back(M);
   }
   template <class T>
   void rec_krylov(std::vector<TailInstr> &c, size_t lvl, T *x, const T *b) {
@@ -952,13 +948,10 @@ struct Solver {
     Z.p[0] = K.r.p;
     Z.p[1] = b;
     c.push_back(Z);
-    rec_dots<T>(c, lvl, 2, b, b, K.r.p, K.r.p, SC_BN2, SC_RN2, TP_CHECK);
-    rec_precond<T>(c, lvl, K.r.p, K.z.p);
-    TailInstr C = ti(TI_COPY, n);
-    C.p[0] = K.p.p;
-    C.p[1] = K.z.p;
-    c.push_back(C);
-    rec_dots<T>(c, lvl, 1, K.r.p, K.z.p, nullptr, nullptr, SC_GAMMA, SC_GAMMA, TP_NONE);
+    rec_dots<T>(c, lvl, 2, b, b, b, b, SC_BN2, SC_RN2, TP_CHECK);
+    if (o.kcycle_iters <= 0) return;
+    rec_precond<T>(c, lvl, K.r.p, K.z.p, K.p.p);
+    if (!fcg) rec_dots<T>(c, lvl, 1, K.r.p, K.z.p, nullptr, nullptr, SC_GAMMA, SC_GAMMA, TP_NONE);
     int it = 0;
     while (it < o.kcycle_iters) {
       rec_spmv<T>(c, lvl, 0, K.p.p, TE_STORE, K.q.p);
@@ -969,9 +962,9 @@ struct Solver {
       U.p[0] = x;
       c.push_back(U);
       it++;
-      rec_dots<T>(c, lvl, 1, K.r.p, K.r.p, nullptr, nullptr, SC_RN2, SC_RN2, TP_CHECK);
       if (it >= o.kcycle_iters) break;
-      rec_precond<T>(c, lvl, K.r.p, K.z.p);
+      rec_dots<T>(c, lvl, 1, K.r.p, K.r.p, nullptr, nullptr, SC_RN2, SC_RN2, TP_CHECK);
+      rec_precond<T>(c, lvl, K.r.p, K.z.p, nullptr);
       if (fcg) rec_dots<T>(c, lvl, 1, K.z.p, K.q.p, nullptr, nullptr, SC_T1, SC_T1, TP_BETA);
       else rec_dots<T>(c, lvl, 1, K.r.p, K.z.p, nullptr, nullptr, SC_GN, SC_GN, TP_BETA);
       TailInstr B = ti(TI_PUPDATE);
@@ -1045,7 +1038,7 @@ struct Solver {
       else if (L.kind == LIGMG_LEVEL_ELIM) cyc[l] = 2 + rec[l];
       else cyc[l] = 3 + std::max(pre, 1) + std::max(post, 1) + 1 + rec[l];
       // recurse(l - 1)
-      const bool k = o.kcycle && L.kind != LIGMG_LEVEL_ELIM;
+      const bool k = inner_krylov(l);
       rec[l - 1] = k ? 1 + 6 + (int64_t)m * (6 + cyc[l] + 3) : cyc[l];
     }
     return rec[e];
@@ -1149,16 +1142,25 @@ struct Solver {
     for (auto &B : w.B) B.alloc(std::max<int64_t>(n, 1));
     if (L.kind == LIGMG_LEVEL_AGG) w.R.alloc(n);
     w.b.alloc(std::max<int64_t>(n, 1));
-    bool need_kw = o.kcycle && l > 0 && L.kind != LIGMG_LEVEL_ELIM;
+    bool need_kw = l > 0 && inner_krylov(l);
     if (need_kw) w.kw.alloc(n, red[l].nb);
   }
 
   // ---------------------------------------------------------------- cycles
+  // Whether a K-cycle solves level l by inner Krylov steps.  Elimination
+  // levels pass through to the next one, and the coarsest is solved exactly
+  // by its pseudo-inverse: Krylov steps preconditioned by it would take one
+  // step of length 1 and then only round (kcycle_iters steps of about 12
+  // instructions each in the deepest, most visited place of the cycle).
+  bool inner_krylov(size_t l) const { return o.kcycle && H[l].kind == LIGMG_LEVEL_AGG; }
+
   // Applies level l's cycle to b with a zero initial guess and returns the
   // buffer holding the result.  The buffer sequence depends only on the
   // options, so replays (and graph captures) see the same pointers.
+  // first: the producer of b has already written the first Chebyshev step
+  // from zero (first_step).
   template <class T>
-  const T *cycle(size_t l, const T *b) {
+  const T *cycle(size_t l, const T *b, bool first = false) {
     DLevel &L = H[l];
     LevelWork<T> &w = work<T>(l);
     if (L.kind == LIGMG_LEVEL_COARSE || l == dense_l0) {
@@ -1166,27 +1168,61 @@ struct Solver {
       return w.B[0].p;
     }
     if (L.kind == LIGMG_LEVEL_ELIM) {
-      LevelWork<T> &wn = work<T>(l + 1);
-      op_spmv<T>(L.R, b, wn.b.p, s);
-      const T *xc = recurse<T>(l, wn.b.p);
+      const T *xc = descend<T>(l, L.R, b);
       op_interp<T>(L.P, qv<T>(L), xc, b, w.B[0].p, s);
       return w.B[0].p;
     }
     // aggregation level
     const T *dinv = dinvv<T>(L);
-    int cur = smooth_from_zero<T>(L, w, dinv, b, o.pre_smooth, l);
-    LevelWork<T> &wn = work<T>(l + 1);
+    int cur = smooth_from_zero<T>(L, w, dinv, b, o.pre_smooth, l, first);
     op_residual<T>(L.A, w.B[cur].p, b, w.R.p, s);
-    op_spmv<T>(L.M, w.R.p, wn.b.p, s);
-    const T *xc = recurse<T>(l, wn.b.p);
-    op_prolong_add<T>(L.agg.p, L.n, xc, w.B[cur].p, s);
+    DLevel &N = H[l + 1];
+    if (N.kind == LIGMG_LEVEL_ELIM && l + 1 < tail_l0 && l + 1 != dense_l0 && N.P.U.row_k == 1 &&
+        L.n <= PROLONG_INTERP_MAX_N) {
+      // the elimination level's interpolation feeds this level's correction
+      LevelWork<T> &wn = work<T>(l + 1);
+      op_spmv<T>(L.M, w.R.p, wn.b.p, s);
+      const T *xc = descend<T>(l + 1, N.R, wn.b.p);
+      op_prolong_interp<T>(L.agg.p, L.n, N.P, qv<T>(N), xc, wn.b.p, w.B[cur].p, s);
+    } else {
+      const T *xc = descend<T>(l, L.M, w.R.p);
+      op_prolong_add<T>(L.agg.p, L.n, xc, w.B[cur].p, s);
+    }
     cur = smooth_from<T>(L, w, dinv, b, cur, o.post_smooth, l);
     if (o.constant_correction) scale_vec<T>(w.B[cur].p, L.n, 4.0 / 3.0);
     return w.B[cur].p;
   }
 
+  // Above this the fused kernel's chain of gathers per vertex costs more than
+  // the launch it saves (700 K vertices: a solve 36.2 -> 36.9 ms; 65 K: 6.95 -> 6.6 ms).
+  static constexpr int64_t PROLONG_INTERP_MAX_N = (int64_t)1 << 17;
+
+  // level l + 1's correction for the right-hand side Op v
   template <class T>
-  int smooth_from_zero(DLevel &L, LevelWork<T> &w, const T *dinv, const T *b, int m, size_t l) {
+  const T *descend(size_t l, const DCsr &Op, const T *v) {
+    T *b = work<T>(l + 1).b.p;
+    FirstStep<T> f;
+    if (l + 1 < tail_l0 && !inner_krylov(l + 1)) f = first_step<T>(l + 1);
+    op_spmv_first<T>(Op, v, b, f, s);
+    return recurse<T>(l, b, f.x != nullptr);
+  }
+
+  // Where the producer of level l's right-hand side also puts the cycle's
+  // first step x_1 = beta_0 D^-1 b (none: the cycle starts otherwise).
+  template <class T>
+  FirstStep<T> first_step(size_t l) {
+    const DLevel &L = H[l];
+    FirstStep<T> f;
+    if (L.kind != LIGMG_LEVEL_AGG || l == dense_l0 || o.smoother_type == LIGMG_SMOOTHER_JACOBI || o.pre_smooth <= 0)
+      return f;
+    f.dinv = dinvv<T>(L);
+    f.x = work<T>(l).B[1].p;
+    f.beta = be_pre[l][0];
+    return f;
+  }
+
+  template <class T>
+  int smooth_from_zero(DLevel &L, LevelWork<T> &w, const T *dinv, const T *b, int m, size_t l, bool first) {
     // the reference's Jacobi smoother is one sweep whatever the step count
     // (create_smoother, smoothing.hpp:206-211)
     if (o.smoother_type == LIGMG_SMOOTHER_JACOBI) {
@@ -1198,7 +1234,7 @@ struct Solver {
       return 0;
     }
     // x_1 = beta_0 D^-1 b in B[1]; x_{k+1} in B[(k+1) % 3]
-    op_cheb_step<T>(L.A, dinv, b, nullptr, nullptr, w.B[1].p, 0.0, be_pre[l][0], s);
+    if (!first) op_cheb_step<T>(L.A, dinv, b, nullptr, nullptr, w.B[1].p, 0.0, be_pre[l][0], s);
     for (int k = 1; k < m; k++) {
       const T *xp = (k == 1) ? nullptr : w.B[(k - 1) % 3].p;
       op_cheb_step<T>(L.A, dinv, b, w.B[k % 3].p, xp, w.B[(k + 1) % 3].p, al_pre[l][k], be_pre[l][k],
@@ -1228,7 +1264,7 @@ struct Solver {
   }
 
   template <class T>
-  const T *recurse(size_t l, const T *bc) {
+  const T *recurse(size_t l, const T *bc, bool first) {
     const DLevel &N = H[l + 1];
     if (l + 1 == dense_l0) return cycle<T>(l + 1, bc);
     if (l + 1 >= tail_l0) {
@@ -1237,7 +1273,7 @@ struct Solver {
       tail_launch<T>(P.code.p, P.len, tail_ops<T>(), tail_lv<T>(), tail_p, s);
       return (const T *)P.out;
     }
-    if (!o.kcycle || N.kind == LIGMG_LEVEL_ELIM) return cycle<T>(l + 1, bc);
+    if (!inner_krylov(l + 1)) return cycle<T>(l + 1, bc, first);
     // K-cycle: kcycle_iters steps of FCG on the next level (multigrid.hpp:113-126)
     LevelWork<T> &wn = work<T>(l + 1);
     KWork<T> &K = wn.kw;
@@ -1255,29 +1291,29 @@ struct Solver {
   void iterate(size_t lvl, const DCsr &A, T *x, KWork<T> &K, bool fcg, double rtol, bool outer_solve, bool norm) {
     const RedPlan &R = red[lvl];
     const T *w = fcg ? K.q.p : K.r.p;
-    float *r32 = nullptr;
-    bool done = false;
-    if constexpr (std::is_same<T, double>::value) {
-      if (outer_solve && mixed) {
-        r32 = W32[lvl].b.p;
-        kr_center<double, float>(R, K.z.p, cycle<float>(lvl, r32), w, s);
-        done = true;
-      }
-    }
     // PETSc removes the attached nullspace from preconditioned vectors
     // (util.hpp:530-534): z is the cycle's result minus its block means
-    if (!done) kr_center<T, T>(R, K.z.p, cycle<T>(lvl, K.r.p), w, s);
+    bool f32 = false;
+    if constexpr (std::is_same<T, double>::value) f32 = outer_solve && mixed;
+    if constexpr (std::is_same<T, double>::value) {
+      if (f32) kr_center<double, float>(R, K.z.p, cycle<float>(lvl, W32[lvl].b.p, first_step<float>(lvl).x), w, s);
+    }
+    if (!f32) kr_center<T, T>(R, K.z.p, cycle<T>(lvl, K.r.p, first_step<T>(lvl).x), w, s);
     kr_pupdate<T>(R, K.p.p, K.z.p, K.sc.p, fcg, s);
     op_spmv<T>(A, K.p.p, K.q.p, s);
     kr_dots<T>(R, K.p.p, K.q.p, fcg ? K.r.p : nullptr, s);
-    kr_update<T>(R, x, K.r.p, K.p.p, K.q.p, K.sc.p, fcg, r32, s);
+    if constexpr (std::is_same<T, double>::value) {
+      if (f32)
+        kr_update<double, float>(R, x, K.r.p, K.p.p, K.q.p, K.sc.p, fcg, W32[lvl].b.p, first_step<float>(lvl), s);
+    }
+    if (!f32) kr_update<T, T>(R, x, K.r.p, K.p.p, K.q.p, K.sc.p, fcg, nullptr, first_step<T>(lvl), s);
     if (norm) kr_norm(R, K.sc.p, false, rtol, outer_solve ? kr_host.p : nullptr, kr_seq.p, s);
   }
 
   // the K-cycle's inner solve
   template <class T>
   void krylov(size_t lvl, const DCsr &A, T *x, const T *b, KWork<T> &K, int type, double rtol, int maxit) {
-    kr_begin<T>(red[lvl], b, x, K.r.p, nullptr, s);
+    kr_begin<T, T>(red[lvl], b, x, K.r.p, nullptr, first_step<T>(lvl), s);
     kr_norm(red[lvl], K.sc.p, true, rtol, nullptr, nullptr, s);
     for (int it = 0; it < maxit; it++) iterate<T>(lvl, A, x, K, fcg_like(type), rtol, false, it + 1 < maxit);
   }
@@ -1311,7 +1347,8 @@ struct Solver {
     kr_seq.ensure((size_t)R.nb);
     for (int c = 0; c < R.nb; c++) kr_host.p[c].seq = 0;  // the stream is idle here
     std::atomic_thread_fence(std::memory_order_release);
-    kr_begin<double>(R, b, x, K.r.p, mixed ? W32[lvl].b.p : nullptr, s);
+    if (mixed) kr_begin<double, float>(R, b, x, K.r.p, W32[lvl].b.p, first_step<float>(lvl), s);
+    else kr_begin<double, double>(R, b, x, K.r.p, nullptr, first_step<double>(lvl), s);
     kr_norm(R, K.sc.p, true, o.tol, kr_host.p, kr_seq.p, s);
     *status = LIGMG_CONVERGED;
     bool active = false;
@@ -1609,7 +1646,7 @@ struct Solver {
       for (auto &B : W[l].B) B.alloc(n * kp);
       if (L.kind == LIGMG_LEVEL_AGG) W[l].R.alloc(n * kp);
       W[l].b.alloc(n * kp);
-      if (o.kcycle && l > 0 && L.kind != LIGMG_LEVEL_ELIM) W[l].kw.alloc(n * kp, red[l].nb * kp);
+      if (l > 0 && inner_krylov(l)) W[l].kw.alloc(n * kp, red[l].nb * kp);
     }
   }
 
@@ -1626,7 +1663,7 @@ struct Solver {
       const DLevel &L = H[l];
       for (const DCsr *M : {&L.A, &L.M, &L.P, &L.R}) maxparts = std::max(maxparts, M->U.nparts);
       // the outer solve's levels, and those a K-cycle iterates on
-      if (l > 1 && (!o.kcycle || L.kind == LIGMG_LEVEL_ELIM)) continue;
+      if (l > 1 && !inner_krylov(l)) continue;
       bred[l].build(L.A.n, L.blocks, s, block_seg_rows(L.A.n, kp));
       maxseg = std::max<int64_t>(maxseg, bred[l].nseg);
     }
@@ -1729,7 +1766,7 @@ struct Solver {
   template <class T>
   const T *brecurse(size_t l, const T *bc, int kp) {
     const DLevel &N = H[l + 1];
-    if (!o.kcycle || N.kind == LIGMG_LEVEL_ELIM) return bcycle<T>(l + 1, bc, kp);
+    if (!inner_krylov(l + 1)) return bcycle<T>(l + 1, bc, kp);
     BLevelWork<T> &wn = bwork<T>(l + 1);
     KWork<T> &K = wn.kw;
     fill_zero<T>(K.x.p, N.A.n * kp);

@@ -314,13 +314,18 @@ __global__ void __launch_bounds__(TAIL_THREADS)
         }
         break;
       }
-      case TI_SUBMEAN: {  // k_sub_mean
+      case TI_CENTER: {  // k_kr_sum + k_kr_center
         const TailLevel<T> &L = lv[I.lvl];
-        T *a = (T *)I.p[0];
+        T *z = (T *)I.p[0], *p = (T *)I.p[2];
+        const T *cv = (const T *)I.p[1];
+        t_dots<T>(L, P, 1, cv, nullptr, nullptr, nullptr, -1, -1, TP_NONE, ws);
+        __syncthreads();
         for (int i = threadIdx.x; i < L.n; i += TAIL_THREADS) {
           const int c = t_block(L, i);
           const T m = (T)(L.bsum[c] / (double)(L.bptr[c + 1] - L.bptr[c]));
-          a[i] -= m;
+          const T zv = cv[i] - m;
+          z[i] = zv;
+          if (p) p[i] = zv;
         }
         break;
       }
@@ -345,8 +350,8 @@ void tail_schedule(const DCsr &A, TailSched &S, hipStream_t s) {
   for (int64_t u = 0; u < U.nunits; u++) {
     const int32_t nr = nrows[u];
     if (nr > 0) {
-      // the lanes k_spmv_units gives each row of the unit
-      const int K = row_lanes(rp[row0[u] + nr] - koff[u], nr, U.row_items);
+      // the lanes k_spmv_rows or k_spmv_units gives each row of the unit
+      const int K = U.row_k ? U.row_k : row_lanes(rp[row0[u] + nr] - koff[u], nr, U.row_items);
       int c = 0;
       while ((2 << c) < K) c++;
       auto &dst = K == 1 ? tr : gr[c];

@@ -73,7 +73,7 @@ enum TailOpcode : int32_t {
   TI_DOTS,       // i0 products (a0 b0, a1 b1) = (p0 p1, p2 p3) -> slots i1, i2, then scalar step i3
   TI_UPDATE,     // x (p0) += alpha p, r -= alpha q
   TI_PUPDATE,    // p = z + beta p
-  TI_SUBMEAN,    // p0 -= block means (block sums from the previous TI_DOTS with i1 < 0)
+  TI_CENTER,     // p0 = p1 minus its block means, also to p2 when set
 };
 enum TailEpi : int32_t {
   TE_STORE = 0,  // p1 = y

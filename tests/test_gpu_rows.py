@@ -1,0 +1,33 @@
+"""The row-kernel SpMV (groups of lanes straight from memory) and the rule
+that picks it, against scipy: mean row lengths on both sides of every lane
+count, and longest rows on both sides of its limit."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import ligmg_amd
+from ligmg_amd import _ffi, graphs
+
+pytestmark = pytest.mark.gpu
+
+
+def ring(n, reach, hub):
+    """Every vertex joined to the `reach` next ones; vertex 0 to `hub` others."""
+    i = np.arange(n)
+    u = np.concatenate([i] * reach + [np.zeros(hub, np.int64)])
+    v = np.concatenate([(i + d + 1) % n for d in range(reach)] + [np.arange(reach + 1, reach + 1 + hub)])
+    w = np.random.default_rng(n + reach + hub).uniform(0.5, 2.0, len(u))
+    return graphs.from_edges(n, u, v, w)
+
+
+@pytest.mark.parametrize("n,reach,hub", [(9, 1, 0), (300, 1, 25), (257, 3, 0), (500, 4, 60), (500, 4, 200),
+                                         (1500, 8, 120), (1500, 8, 200), (2000, 20, 1900), (700, 300, 0)])
+def test_level_spmv_rows(n, reach, hub):
+    g = ring(n, reach, hub)
+    s = ligmg_amd.Solver(g, ligmg_amd.Options(precision=_ffi.PREC_MIXED, elim_degree=0, always_elim=0))
+    rp, ci, v = s.level_matrix(0)
+    A = sp.csr_matrix((v, ci, rp), shape=(n, n))
+    x = np.random.default_rng(0).standard_normal(n)
+    bound = abs(A) @ abs(x) * np.diff(rp).max()  # one rounding per term
+    assert (np.abs(s.level_spmv(0, x) - A @ x) <= 2.0 ** -52 * bound).all()
+    assert (np.abs(s.level_spmv(0, x, _ffi.PREC_MIXED) - A @ x) <= 4 * 2.0 ** -24 * (abs(A) @ abs(x))).all()
