@@ -1013,9 +1013,28 @@ __global__ void k_voters(int n, const int32_t *state, const int32_t *vind, const
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   bool ok = state[i] == ST_UNDECIDED && vind[i] >= 0 && vw[i] >= thresh && vind[i] != i;
-  flag[i] = ok ? 1 : 0;
+  if (flag) flag[i] = ok ? 1 : 0;
   vf[i] = ok ? vind[i] : -1;
 }
+
+// The tally of an undecided vertex over its own row.  Its voters are
+// neighbours (a vote names the aggregate of a neighbour, and an undecided
+// vertex is an aggregate of its own), met in ascending index as the sorted
+// tally meets them, so this is the same sum without compaction, sort,
+// segments and scatter: some 15 launches and three counts read back per round
+// (a 5021-vertex graph's setup and solve 13.4 -> 8.6 ms with the sweep below).  The sums of other vertices,
+// which neighbours of their members vote for, are left out: see run_voting.
+struct OpTally : DblSum {
+  const int32_t *ci, *vf, *state;
+  const double *vw;
+  double *votes;
+  __device__ bool skip(int row) const { return state[row] != ST_UNDECIDED; }
+  __device__ void add(double &acc, int row, int k) const {
+    const int j = ci[k];
+    acc += vf[j] == row ? vw[j] : 0.0;
+  }
+  __device__ void finish(int row, double acc) const { votes[row] = acc + votes[row]; }
+};
 
 __global__ void k_voter_pairs(int64_t m, const int32_t *idx, const int32_t *vind, const double *vw,
                               uint64_t *keys, uint64_t *vals) {
@@ -1443,12 +1462,148 @@ bool transpose_positions(const DCsr &A, const HugeRows &Hr, int32_t *tpos, hipSt
   return hb == 0;
 }
 
-// One accumulator width for every T <= MAXT.  Narrower ones (N = T) lower
-// the register count and raise occupancy, but measured slower (7.6% at
-// T = 10 on R-MAT 23): more gathers of the test-vector array (n * TS * 8
-// bytes, larger than the last-level cache) in flight thrash the caches.
+// The Jacobi sweep for vectors stored at a row stride of 16 (9 to 16 test
+// vectors, the default 10 among them): lane t of a group of 16 holds vector
+// t, so a neighbour's row is one coalesced access instead of five 16-byte
+// loads that each touch 64 lines, and a wavefront has 8 or 16 of them in
+// flight.  The sums are those of the generic row kernels, which took, on R-MAT
+// 20 (32 M entries; a setup's 32 to 36 sweeps): rows of at most 64 entries 4.9 ->
+// 2.4 ms, longer ones 7.5 -> 6.4, hub chunks 2.8 -> 3.1; on 5021 vertices 71 -> 8
+// us a sweep.  Bound by the gathered rows (about 2.5 TB/s from the Infinity
+// Cache).
+constexpr int JT = 16;  // lanes per row of X
+struct JacobiTV {
+  const int32_t *rp, *ci;
+  const double *v, *X, *diag;
+  const uint8_t *hasd;
+  double *Y;
+  int T;
+  __device__ __forceinline__ void finish(int row, int t, double acc) const {
+    if (t >= T) return;
+    const double w = 2.0 / 3.0;
+    const double x = X[(int64_t)row * JT + t];
+    Y[(int64_t)row * JT + t] = hasd[row] ? w * (0.0 - acc) / diag[row] + (1 - w) * x : x;
+  }
+  // terms of N entries k, k + step, ..., all loads in flight; entries from
+  // b on read entry b - 1 and count 0.0 (which no sum from 0.0 can tell)
+  template <int N, bool FULL>
+  __device__ __forceinline__ void terms(int k, int step, int b, int t, double *q) const {
+    double a[N], x[N];
+    int c[N];
+#pragma unroll
+    for (int u = 0; u < N; u++) {
+      const int e = FULL ? k + u * step : min(k + u * step, b - 1);
+      c[u] = ci[e];
+      a[u] = v[e];
+    }
+#pragma unroll
+    for (int u = 0; u < N; u++) x[u] = X[(int64_t)c[u] * JT + t];
+#pragma unroll
+    for (int u = 0; u < N; u++) q[u] = (a[u] < 0 && (FULL || k + u * step < b)) ? a[u] * x[u] : 0.0;
+  }
+  // rows (or chunks) [a, b) of at most WAVE entries: left to right
+  __device__ __forceinline__ double fold(int a, int b, int t) const {
+    double acc = 0.0, q[8];
+    for (int k = a; k < b; k += 8) {
+      terms<8, false>(k, 1, b, t, q);
+#pragma unroll
+      for (int u = 0; u < 8; u++) acc += q[u];
+    }
+    return acc;
+  }
+  // [a, b) by one wavefront: 64 strided partials and the tree p[l] += p[l +
+  // off], off = 32..1.  Group g of 16 lanes keeps partials g, g + 4, ... of
+  // its lane's vector in registers, so the tree's first four steps are
+  // register adds and the last two cross the groups.  Valid in group 0.
+  __device__ __forceinline__ double strided(int a, int b, int lane) const {
+    const int t = lane & (JT - 1), g = lane / JT;
+    double p[16], q[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) p[u] = 0.0;
+    int base = a;
+    for (; base + WAVE <= b; base += WAVE) {
+      terms<16, true>(base + g, 4, b, t, q);
+#pragma unroll
+      for (int u = 0; u < 16; u++) p[u] += q[u];
+    }
+    if (base < b) {
+      terms<16, false>(base + g, 4, b, t, q);
+#pragma unroll
+      for (int u = 0; u < 16; u++) p[u] += q[u];
+    }
+#pragma unroll
+    for (int h = 8; h >= 1; h >>= 1)
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        if (u < h) p[u] += p[u + h];
+    p[0] += __shfl_down(p[0], 2 * JT, WAVE);
+    p[0] += __shfl_down(p[0], JT, WAVE);
+    return p[0];
+  }
+};
+
+__global__ void __launch_bounds__(256) k_jacobi_short(int n, JacobiTV J) {
+  const int row = (int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / JT), t = threadIdx.x & (JT - 1);
+  if (row >= n) return;
+  const int a = J.rp[row], b = J.rp[row + 1];
+  if (b - a > WAVE) return;
+  J.finish(row, t, J.fold(a, b, t));
+}
+__global__ void __launch_bounds__(256) k_jacobi_mid(int64_t nmid, const int32_t *__restrict__ mrow, JacobiTV J) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int64_t nw = (int64_t)gridDim.x * (blockDim.x / WAVE);
+  for (int64_t j = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / WAVE; j < nmid; j += nw) {
+    const int row = mrow[j];
+    const double acc = J.strided(J.rp[row], J.rp[row + 1], lane);
+    if (lane < JT) J.finish(row, lane, acc);
+  }
+}
+__global__ void __launch_bounds__(256) k_jacobi_chunks(int64_t nchunks, const int32_t *cstart, const int32_t *cend,
+                                                       JacobiTV J, double *cacc) {
+  const int lane = threadIdx.x & (WAVE - 1), t = lane & (JT - 1);
+  const int64_t c = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / WAVE;
+  if (c >= nchunks) return;
+  const int a = cstart[c], b = cend[c];
+  const double acc = b - a <= WAVE ? J.fold(a, b, t) : J.strided(a, b, lane);
+  if (lane < JT) cacc[c * JT + t] = acc;
+}
+__global__ void k_jacobi_huge(int64_t nrows, const int32_t *row, const int32_t *cptr, JacobiTV J, const double *cacc) {
+  const int64_t j = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / JT;
+  const int t = threadIdx.x & (JT - 1);
+  if (j >= nrows) return;
+  double acc = 0.0;
+  for (int c = cptr[j]; c < cptr[j + 1]; c++) acc += cacc[(int64_t)c * JT + t];
+  J.finish(row[j], t, acc);
+}
+
+void jacobi_tv_16(int64_t n, const DCsr &A, const JacobiTV &J, const HugeRows &Hr, hipStream_t s) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_jacobi_short, dim3((unsigned)((n * JT + 255) / 256)), dim3(256), 0, s, (int)n, J);
+  LG_LAUNCH_CHECK();
+  if (Hr.nmid) {
+    const int64_t waves = std::min<int64_t>(Hr.nmid, MID_WAVES);
+    hipLaunchKernelGGL(k_jacobi_mid, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, Hr.nmid, Hr.mrow.p, J);
+    LG_LAUNCH_CHECK();
+  }
+  if (Hr.nrows) {
+    static_assert(JT * sizeof(double) <= 192, "chunk sums fit the chunk buffer");
+    double *cacc = (double *)Hr.cacc.p;
+    hipLaunchKernelGGL(k_jacobi_chunks, dim3((unsigned)((Hr.nchunks + 3) / 4)), dim3(256), 0, s, Hr.nchunks,
+                       Hr.cstart.p, Hr.cend.p, J, cacc);
+    LG_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_jacobi_huge, dim3((unsigned)((Hr.nrows * JT + 255) / 256)), dim3(256), 0, s, Hr.nrows,
+                       Hr.row.p, Hr.cptr.p, J, (const double *)cacc);
+    LG_LAUNCH_CHECK();
+  }
+}
+
+// strides below 16: the generic row kernels
 void jacobi_tv_sweep(int64_t n, const DCsr &A, const double *X, const double *diag, const uint8_t *hasd,
                      double *Y, int T, int TS, const HugeRows &Hr, hipStream_t s) {
+  if (TS == JT) {
+    jacobi_tv_16(n, A, {A.rp.p, A.ci.p, A.v.p, X, diag, hasd, Y, T}, Hr, s);
+    return;
+  }
   run_rows(n, A.rp.p, OpJacobiTV<MAXT>{A.ci.p, A.v.p, X, diag, hasd, Y, T, TS}, Hr, s);
 }
 }  // namespace
@@ -1529,31 +1684,41 @@ int64_t run_voting(const DCsr &A, const double *S, const double *cs, const ligmg
   LG_LAUNCH_CHECK();
   fill_f64(votes.p, 0.0, n, s);
   const int kb = std::max(1, bits_for((uint64_t)n));
+  // Row tallies leave out votes for decided vertices.  Without a size limit
+  // nothing reads those (k_mark turns every Seed into a DecidedRoot whatever
+  // its votes), and without rejection or neighbour-of-neighbour votes an
+  // undecided vertex is named by its neighbours alone.  A row longer than
+  // HUGE_ROW would be one wavefront's serial chain; such levels sort.
+  const bool row_tally = Hr.nrows == 0 && o.max_agg_size < 0 && o.rejection_ratio < 0 && !o.neighbor_of_neighbor;
   for (int iter = 0; iter < o.agg_iters; iter++) {
     const double th = o.agg_init_factor * std::pow(o.agg_iter_factor, iter);
     run_rows(n, A.rp.p, OpVote{A.ci.p, state.p, ind.p, S, th, o.neighbor_of_neighbor ? 1 : 0, vst.p, vind.p, vw.p},
              Hr, s);
-    hipLaunchKernelGGL(k_voters, dim3(g1(n)), dim3(256), 0, s, (int)n, state.p, vind.p, vw.p, th, flag.p,
-                       vf.p);
+    hipLaunchKernelGGL(k_voters, dim3(g1(n)), dim3(256), 0, s, (int)n, state.p, vind.p, vw.p, th,
+                       row_tally ? nullptr : flag.p, vf.p);
     LG_LAUNCH_CHECK();
-    int64_t m = compact_flags(flag.p, n, idx.p, s);
-    fill_f64(nv.p, 0.0, n, s);
-    if (m > 0) {
-      DevBuf<uint64_t> keys(m), vals(m), uk(m);
-      DevBuf<double> us(m);
-      hipLaunchKernelGGL(k_voter_pairs, dim3(grid_for(m, 256, 8192)), dim3(256), 0, s, m, idx.p, vind.p,
-                         vw.p, keys.p, vals.p);
-      LG_LAUNCH_CHECK();
-      // stable sort: each target's voters stay in ascending voter index,
-      // the order in which tally_votes adds them (aggregation.hpp:539-547)
-      radix_sort_pairs(keys, vals, m, kb, s);
-      int64_t nu = segmented_seq_sum(keys.p, vals.p, m, uk.p, us.p, s);
-      hipLaunchKernelGGL(k_scatter_sums, dim3(grid_for(nu, 256, 8192)), dim3(256), 0, s, nu, uk.p, us.p,
-                         nv.p);
+    if (row_tally) {
+      run_rows_seq(n, A.rp.p, OpTally{{}, A.ci.p, vf.p, state.p, vw.p, votes.p}, Hr, s);
+    } else {
+      int64_t m = compact_flags(flag.p, n, idx.p, s);
+      fill_f64(nv.p, 0.0, n, s);
+      if (m > 0) {
+        DevBuf<uint64_t> keys(m), vals(m), uk(m);
+        DevBuf<double> us(m);
+        hipLaunchKernelGGL(k_voter_pairs, dim3(grid_for(m, 256, 8192)), dim3(256), 0, s, m, idx.p, vind.p,
+                           vw.p, keys.p, vals.p);
+        LG_LAUNCH_CHECK();
+        // stable sort: each target's voters stay in ascending voter index,
+        // the order in which tally_votes adds them (aggregation.hpp:539-547)
+        radix_sort_pairs(keys, vals, m, kb, s);
+        int64_t nu = segmented_seq_sum(keys.p, vals.p, m, uk.p, us.p, s);
+        hipLaunchKernelGGL(k_scatter_sums, dim3(grid_for(nu, 256, 8192)), dim3(256), 0, s, nu, uk.p, us.p,
+                           nv.p);
+        LG_LAUNCH_CHECK();
+      }
+      hipLaunchKernelGGL(k_add_votes, dim3(g1(n)), dim3(256), 0, s, (int)n, nv.p, votes.p);
       LG_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(k_add_votes, dim3(g1(n)), dim3(256), 0, s, (int)n, nv.p, votes.p);
-    LG_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_mark, dim3(g1(n)), dim3(256), 0, s, (int)n, iter == 0 ? 1 : 0, state.p, ind.p,
                        vst.p, vind.p, vf.p, votes.p, cs, (double)o.votes_to_seed,
                        (double)o.max_agg_size, o.neighbor_of_neighbor ? 1 : 0, nstate.p, nind.p);
