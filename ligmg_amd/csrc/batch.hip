@@ -78,6 +78,27 @@ struct BStore {
     bvec_store<T, VW>(y + i * kp + c, [&](int v) { return (T)s[v]; });
   }
 };
+// y = s and the next cycle's first Chebyshev step from y
+template <class T>
+struct BFirst {
+  T *y;
+  FirstStep<T> f;
+  int kp;
+  template <int VW>
+  struct Pre {
+    T dinv;
+  };
+  template <int VW>
+  __device__ __forceinline__ Pre<VW> load(int64_t i, int) const {
+    return {f.dinv[i]};
+  }
+  template <int VW>
+  __device__ __forceinline__ void store(int64_t i, int c, const double *s, const Pre<VW> &p) const {
+    const int64_t o = i * kp + c;
+    bvec_store<T, VW>(y + o, [&](int v) { return (T)s[v]; });
+    bvec_store<T, VW>(f.x + o, [&](int v) { return sdev::cheb_first<T>(f.beta, p.dinv, (T)s[v]); });
+  }
+};
 template <class T>
 struct BResid {
   const T *b;
@@ -576,32 +597,72 @@ __global__ void __launch_bounds__(256) k_bred1(int np, int kp, const T *a0, cons
   if (np > 1) bseg_sum<VW>(B, kp, acc1, red, part + ((int64_t)s * np + 1) * kp);
 }
 
-// out[blk, j, c] = sum of the segment partials of block blk: one workgroup
-// per (block, j); thread (g, c) adds segments g, g + G, ... (G = 1024 / kp)
-// in order, and the G partials of a column are added in g order.
+// The segment partials of block blk, summed per column, and what follows
+// (BlockPost): one workgroup per block.  Thread (g, c) adds segments g, g + G,
+// ... (G = 1024 / kp) in order, and the G partials of a column are added 16
+// at a time.  The scalar steps of the block's (blk, column) sets run here, so a
+// dot costs no launch beyond its two stages.
 __global__ void __launch_bounds__(1024) k_bred2(int np, int kp, int lk, const int32_t *bseg, const double *part,
-                                                double *out) {
-  const int blk = blockIdx.x, j = blockIdx.y;
+                                                BlockPost P) {
+  const int blk = blockIdx.x;
   const int G = 1024 >> lk;
   const int g = threadIdx.x >> lk, c = threadIdx.x & (kp - 1);
-  double acc = 0;
   const int end = bseg[blk + 1];
-#pragma unroll 8
-  for (int sg = bseg[blk] + g; sg < end; sg += G) acc += part[((int64_t)sg * np + j) * kp + c];
   __shared__ double red[1024];
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  // 16 partials a thread, then the rest in order
-  for (int n = G; n > 1; n = (n + 15) / 16) {
-    const int m = (n + 15) / 16;
-    double t = 0;
-    if (g < m)
-      for (int q = 16 * g; q < min(16 * g + 16, n); q++) t += red[q * kp + c];
+  double sum[2] = {0, 0};
+  for (int j = 0; j < np; j++) {
+    double acc = 0;
+#pragma unroll 8
+    for (int sg = bseg[blk] + g; sg < end; sg += G) acc += part[((int64_t)sg * np + j) * kp + c];
+    red[threadIdx.x] = acc;
     __syncthreads();
-    if (g < m) red[threadIdx.x] = t;
+    for (int n = G; n > 1; n = (n + 15) / 16) {
+      const int m = (n + 15) / 16;
+      double t = 0;
+      if (g < m)
+        for (int q = 16 * g; q < min(16 * g + 16, n); q++) t += red[q * kp + c];
+      __syncthreads();
+      if (g < m) red[threadIdx.x] = t;
+      __syncthreads();
+    }
+    sum[j] = red[c];
     __syncthreads();
   }
-  if (g == 0) out[((int64_t)blk * np + j) * kp + c] = red[c];
+  if (g != 0) return;
+  if (P.kind == BlockPost::OUT) {
+    for (int j = 0; j < np; j++) P.out[((int64_t)blk * np + j) * kp + c] = sum[j];
+    return;
+  }
+  using namespace sdev;
+  const int64_t set = (int64_t)blk * kp + c;
+  double *S = P.sc + set * SC_N;
+  switch (P.kind) {
+    case BlockPost::ALPHA:
+      S[SC_DELTA] = sum[0];
+      if (P.fcg) S[SC_T1] = sum[1];
+      kr_alpha(S, P.fcg);
+      break;
+    case BlockPost::BETA:
+      S[P.fcg ? SC_T1 : SC_GN] = sum[0];
+      kr_beta(S, P.fcg);
+      break;
+    default: {  // INIT, NORM
+      if (P.kind == BlockPost::INIT) {
+        kr_init(S);
+        S[SC_BN2] = sum[0];
+      }
+      S[SC_RN2] = sum[0];
+      kr_check(S, P.rtol);
+      if (!P.host) break;
+      const unsigned long long k = P.kind == BlockPost::INIT ? 1 : P.seq[set] + 1;
+      P.seq[set] = k;
+      volatile KrHost *h = P.host + set;
+      h->rn2 = sum[0];
+      h->active = S[SC_ACTIVE];
+      __threadfence_system();
+      h->seq = k;
+    }
+  }
 }
 
 template <class T, int VW>
@@ -623,53 +684,77 @@ __global__ void __launch_bounds__(256) k_bsub_mean(T *a, int kp, const int64_t *
   }
 }
 
-// z = c - (block mean), in FP64; with w set, also the segment partials of
-// z.w as the block dots form them (part[s * kp + c])
-template <int VW>
-__global__ void __launch_bounds__(256) k_bsub_mean_f2d(double *z, const float *cv, int kp, const int64_t *lo,
-                                                       const int64_t *hi, const int32_t *segblk,
-                                                       const int64_t *bptr, const double *sums, const double *w,
-                                                       double *part) {
+// z = c - (block mean) and the segment partials of z.w as the block dots
+// form them (part[s * kp + c])
+template <class T, class C, int VW>
+__global__ void __launch_bounds__(256) k_bcenter(T *z, const C *cv, const T *w, int kp, const int64_t *lo,
+                                                 const int64_t *hi, const int32_t *segblk, const int64_t *bptr,
+                                                 const double *sums, double *part) {
   const int s = blockIdx.x;
   const int blk = segblk[s];
   const BSeg<VW> B(lo[s], hi[s], kp);
-  double m[VW], acc[VW] = {};
+  T m[VW];
+  double acc[VW] = {};
 #pragma unroll
-  for (int v = 0; v < VW; v++) m[v] = sums[(int64_t)blk * kp + B.c + v] / (double)(bptr[blk + 1] - bptr[blk]);
+  for (int v = 0; v < VW; v++) m[v] = (T)(sums[(int64_t)blk * kp + B.c + v] / (double)(bptr[blk + 1] - bptr[blk]));
   for (int64_t i = B.lo + B.g; i < B.hi; i += 4 * B.G) {
-    typename BVec<float, VW>::type x[4];
-    typename BVec<double, VW>::type y[4];
+    typename BVec<C, VW>::type x[4];
+    typename BVec<T, VW>::type y[4];
 #pragma unroll
     for (int t = 0; t < 4; t++) {
       const int64_t o = min(i + t * B.G, B.hi - 1) * kp + B.c;
-      x[t] = bvec_load<float, VW>(cv + o);
-      if (w) y[t] = bvec_load<double, VW>(w + o);
+      x[t] = bvec_load<C, VW>(cv + o);
+      y[t] = bvec_load<T, VW>(w + o);
     }
 #pragma unroll
     for (int t = 0; t < 4; t++) {
       if (i + t * B.G >= B.hi) continue;
-      double zv[VW];
+      T zv[VW];
 #pragma unroll
       for (int v = 0; v < VW; v++) {
-        zv[v] = bvec_at<float, VW>(x[t], v) - m[v];
-        if (w) acc[v] += zv[v] * bvec_at<double, VW>(y[t], v);
+        zv[v] = (T)bvec_at<C, VW>(x[t], v) - m[v];
+        acc[v] += (double)zv[v] * bvec_at<T, VW>(y[t], v);
       }
-      bvec_store<double, VW>(z + (i + t * B.G) * kp + B.c, [&](int v) { return zv[v]; });
+      bvec_store<T, VW>(z + (i + t * B.G) * kp + B.c, [&](int v) { return zv[v]; });
     }
   }
-  if (!w) return;  // uniform over the workgroup
+  __shared__ double red[VW][256];
+  bseg_sum<VW>(B, kp, acc, red, part + (int64_t)s * kp);
+}
+
+// x = 0, r = b and the segment partials of b.b; rf and f as in k_kr_bupdate
+template <class T, class F, int VW>
+__global__ void __launch_bounds__(256) k_kr_bbegin(const T *b, T *x, T *r, F *rf, FirstStep<F> f, int kp,
+                                                   const int64_t *lo, const int64_t *hi, double *part) {
+  const int s = blockIdx.x;
+  const BSeg<VW> B(lo[s], hi[s], kp);
+  double acc[VW] = {};
+#pragma unroll 4
+  for (int64_t i = B.lo + B.g; i < B.hi; i += B.G) {
+    const int64_t o = i * kp + B.c;
+    const typename BVec<T, VW>::type v = bvec_load<T, VW>(b + o);
+    bvec_store<T, VW>(x + o, [&](int) { return (T)0; });
+    *(typename BVec<T, VW>::type *)(r + o) = v;
+    if (rf) bvec_store<F, VW>(rf + o, [&](int u) { return (F)bvec_at<T, VW>(v, u); });
+    if (f.x) {
+      const F dv = f.dinv[i];
+      bvec_store<F, VW>(f.x + o, [&](int u) { return sdev::cheb_first<F>(f.beta, dv, (F)bvec_at<T, VW>(v, u)); });
+    }
+#pragma unroll
+    for (int u = 0; u < VW; u++) acc[u] += bvec_at<T, VW>(v, u) * bvec_at<T, VW>(v, u);
+  }
   __shared__ double red[VW][256];
   bseg_sum<VW>(B, kp, acc, red, part + (int64_t)s * kp);
 }
 
 // x += alpha p, r -= alpha q per (block, column); alpha = 0 marks a finished
 // column, whose x and r stay.  Also writes the segment partials of r.r as
-// the block dots form them (part[s * kp + c]), and r in FP32 when r32 is set
-// (the mixed outer preconditioner's input).
-template <class T, int VW>
-__global__ void __launch_bounds__(256) k_kr_bupdate(T *x, T *r, const T *p, const T *q, int kp, const int64_t *lo,
-                                                    const int64_t *hi, const int32_t *segblk, const double *sc,
-                                                    double *part, float *r32) {
+// the block dots form them (part[s * kp + c]); with rf set r in the cycle's
+// type, with f.x set the cycle's first step from r.
+template <class T, class F, int VW>
+__global__ void __launch_bounds__(256) k_kr_bupdate(T *x, T *r, const T *p, const T *q, F *rf, FirstStep<F> f,
+                                                    int kp, const int64_t *lo, const int64_t *hi,
+                                                    const int32_t *segblk, const double *sc, double *part) {
   const int s = blockIdx.x;
   const BSeg<VW> B(lo[s], hi[s], kp);
   T at[VW];
@@ -684,10 +769,12 @@ __global__ void __launch_bounds__(256) k_kr_bupdate(T *x, T *r, const T *p, cons
   typedef typename BVec<T, VW>::type V;
   for (int64_t i = B.lo + B.g; i < B.hi; i += 4 * B.G) {
     V xv[4], rv[4], pv[4], qv[4];
+    F dv[4];
 #pragma unroll
     for (int t = 0; t < 4; t++) {
-      const int64_t o = min(i + t * B.G, B.hi - 1) * kp + B.c;
+      const int64_t row = min(i + t * B.G, B.hi - 1), o = row * kp + B.c;
       rv[t] = bvec_load<T, VW>(r + o);
+      if (f.x) dv[t] = f.dinv[row];
       if (any) {
         xv[t] = bvec_load<T, VW>(x + o);
         pv[t] = bvec_load<T, VW>(p + o);
@@ -716,14 +803,15 @@ __global__ void __launch_bounds__(256) k_kr_bupdate(T *x, T *r, const T *p, cons
         bvec_store<T, VW>(x + o, [&](int v) { return xn[v]; });
         bvec_store<T, VW>(r + o, [&](int v) { return rn[v]; });
       }
-      if (r32) bvec_store<float, VW>(r32 + o, [&](int v) { return (float)rn[v]; });
+      if (rf) bvec_store<F, VW>(rf + o, [&](int v) { return (F)rn[v]; });
+      if (f.x) bvec_store<F, VW>(f.x + o, [&](int v) { return sdev::cheb_first<F>(f.beta, dv[t], (F)rn[v]); });
     }
   }
   __shared__ double red[VW][256];
   bseg_sum<VW>(B, kp, acc, red, part + (int64_t)s * kp);
 }
 
-// p = z + beta p
+// p = z + beta p; where beta is 0 (the first step) p is not used
 template <class T, int VW>
 __global__ void __launch_bounds__(256) k_kr_bpupdate(T *p, const T *z, int kp, const int64_t *lo, const int64_t *hi,
                                                      const int32_t *segblk, const double *sc) {
@@ -746,8 +834,8 @@ __global__ void __launch_bounds__(256) k_kr_bpupdate(T *p, const T *z, int kp, c
     for (int t = 0; t < 4; t++)
       if (i + t * B.G < B.hi)
         bvec_store<T, VW>(p + (i + t * B.G) * kp + B.c, [&](int v) {
-          if constexpr (VW == 1) return zv[t] + bt[0] * pv[t];
-          else return zv[t][v] + bt[v] * pv[t][v];
+          if constexpr (VW == 1) return bt[0] != (T)0 ? zv[t] + bt[0] * pv[t] : zv[t];
+          else return bt[v] != (T)0 ? zv[t][v] + bt[v] * pv[t][v] : zv[t][v];
         });
   }
 }
@@ -799,6 +887,12 @@ void spmm_tile(int cfg, int *u) { *u = SPMM_U[cfg]; }
 template <class T>
 void op_bspmv(const DCsr &A, const T *X, T *Y, int kp, DevBuf<double> &parts, hipStream_t s) {
   dispatch_spmm<T>(A, X, kp, BStore<T>{Y, kp}, parts, s);
+}
+template <class T>
+void op_bspmv_first(const DCsr &A, const T *X, T *Y, const FirstStep<T> &f, int kp, DevBuf<double> &parts,
+                    hipStream_t s) {
+  if (f.x) dispatch_spmm<T>(A, X, kp, BFirst<T>{Y, f, kp}, parts, s);
+  else op_bspmv<T>(A, X, Y, kp, parts, s);
 }
 template <class T>
 void op_bresidual(const DCsr &A, const T *X, const T *B, T *R, int kp, DevBuf<double> &parts,
@@ -862,9 +956,8 @@ void op_from_block(const double *X, int64_t n, int k, int kp, double *B, const i
 }
 
 template <class T>
-void RedPlan::bdots(int np, int kp, const T *a0, const T *b0, const T *a1, const T *b1, double *out,
-                    DevBuf<double> &bpart, hipStream_t s) const {
-  if (nseg == 0) return;
+void RedPlan::bpartials(int np, int kp, const T *a0, const T *b0, const T *a1, const T *b1, DevBuf<double> &bpart,
+                        hipStream_t s) const {
   LG_CHECK(bpart.n >= (size_t)nseg * np * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
   if (kp == 1)
     hipLaunchKernelGGL((k_bred1<T, 1>), dim3(nseg), dim3(256), 0, s, np, kp, a0, b0, a1, b1, seg_lo.p, seg_hi.p,
@@ -873,29 +966,50 @@ void RedPlan::bdots(int np, int kp, const T *a0, const T *b0, const T *a1, const
     hipLaunchKernelGGL((k_bred1<T, 2>), dim3(nseg), dim3(256), 0, s, np, kp, a0, b0, a1, b1, seg_lo.p, seg_hi.p,
                        bpart.p);
   LG_LAUNCH_CHECK();
-  bdots_finish(np, kp, out, bpart, s);
 }
 
-void RedPlan::bdots_finish(int np, int kp, double *out, const DevBuf<double> &bpart, hipStream_t s) const {
+template <class T>
+void RedPlan::bdots(int np, int kp, const T *a0, const T *b0, const T *a1, const T *b1, double *out,
+                    DevBuf<double> &bpart, hipStream_t s) const {
   if (nseg == 0) return;
+  bpartials<T>(np, kp, a0, b0, a1, b1, bpart, s);
+  BlockPost P;
+  P.out = out;
+  bfinish(np, kp, P, bpart, s);
+}
+
+void RedPlan::bfinish(int np, int kp, const BlockPost &P, const DevBuf<double> &bpart, hipStream_t s) const {
+  if (nb == 0) return;
   LG_CHECK(bpart.n >= (size_t)nseg * np * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
-  hipLaunchKernelGGL(k_bred2, dim3((unsigned)nb, (unsigned)np), dim3(1024), 0, s, np, kp, log2i(kp), bseg.p, bpart.p,
-                     out);
+  hipLaunchKernelGGL(k_bred2, dim3((unsigned)nb), dim3(1024), 0, s, np, kp, log2i(kp), bseg.p,
+                     (const double *)bpart.p, P);
   LG_LAUNCH_CHECK();
 }
 
-void op_bsub_block_mean_f2d(double *z, const float *c, int kp, const RedPlan &P, const double *sums, hipStream_t s,
-                            const double *w, DevBuf<double> *bpart) {
-  if (P.nseg == 0) return;
-  if (w) LG_CHECK(bpart && bpart->n >= (size_t)P.nseg * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
+#define LG_SEGS dim3((unsigned)R.nseg), dim3(256), 0, s
+template <class T, class C>
+void op_bcenter(const RedPlan &R, T *z, const C *c, const T *w, int kp, const double *sums, DevBuf<double> &bpart,
+                hipStream_t s) {
+  LG_CHECK(bpart.n >= (size_t)R.nseg * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
   if (kp == 1)
-    hipLaunchKernelGGL(k_bsub_mean_f2d<1>, dim3(P.nseg), dim3(256), 0, s, z, c, kp, P.seg_lo.p, P.seg_hi.p,
-                       P.bseg.p + P.nb + 1, P.bptr.p, sums, w, w ? bpart->p : nullptr);
+    hipLaunchKernelGGL((k_bcenter<T, C, 1>), LG_SEGS, z, c, w, kp, R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1,
+                       R.bptr.p, sums, bpart.p);
   else
-    hipLaunchKernelGGL(k_bsub_mean_f2d<2>, dim3(P.nseg), dim3(256), 0, s, z, c, kp, P.seg_lo.p, P.seg_hi.p,
-                       P.bseg.p + P.nb + 1, P.bptr.p, sums, w, w ? bpart->p : nullptr);
+    hipLaunchKernelGGL((k_bcenter<T, C, 2>), LG_SEGS, z, c, w, kp, R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1,
+                       R.bptr.p, sums, bpart.p);
   LG_LAUNCH_CHECK();
 }
+template <class T, class F>
+void op_kr_bbegin(const RedPlan &R, const T *b, T *x, T *r, F *rf, const FirstStep<F> &f, int kp,
+                  DevBuf<double> &bpart, hipStream_t s) {
+  LG_CHECK(bpart.n >= (size_t)R.nseg * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
+  if (kp == 1)
+    hipLaunchKernelGGL((k_kr_bbegin<T, F, 1>), LG_SEGS, b, x, r, rf, f, kp, R.seg_lo.p, R.seg_hi.p, bpart.p);
+  else
+    hipLaunchKernelGGL((k_kr_bbegin<T, F, 2>), LG_SEGS, b, x, r, rf, f, kp, R.seg_lo.p, R.seg_hi.p, bpart.p);
+  LG_LAUNCH_CHECK();
+}
+#undef LG_SEGS
 
 template <class T>
 void op_bsub_block_mean(T *a, int kp, const RedPlan &P, const double *sums, hipStream_t s) {
@@ -909,17 +1023,17 @@ void op_bsub_block_mean(T *a, int kp, const RedPlan &P, const double *sums, hipS
   LG_LAUNCH_CHECK();
 }
 
-template <class T>
-void op_kr_bupdate(T *x, T *r, const T *p, const T *q, int kp, const RedPlan &P, const double *sc,
-                   DevBuf<double> &bpart, float *r32, hipStream_t s) {
-  if (P.nseg == 0) return;
-  LG_CHECK(bpart.n >= (size_t)P.nseg * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
+template <class T, class F>
+void op_kr_bupdate(const RedPlan &R, T *x, T *r, const T *p, const T *q, F *rf, const FirstStep<F> &f, int kp,
+                   const double *sc, DevBuf<double> &bpart, hipStream_t s) {
+  if (R.nseg == 0) return;
+  LG_CHECK(bpart.n >= (size_t)R.nseg * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
   if (kp == 1)
-    hipLaunchKernelGGL((k_kr_bupdate<T, 1>), dim3(P.nseg), dim3(256), 0, s, x, r, p, q, kp, P.seg_lo.p, P.seg_hi.p,
-                       P.bseg.p + P.nb + 1, sc, bpart.p, r32);
+    hipLaunchKernelGGL((k_kr_bupdate<T, F, 1>), dim3(R.nseg), dim3(256), 0, s, x, r, p, q, rf, f, kp, R.seg_lo.p,
+                       R.seg_hi.p, R.bseg.p + R.nb + 1, sc, bpart.p);
   else
-    hipLaunchKernelGGL((k_kr_bupdate<T, 2>), dim3(P.nseg), dim3(256), 0, s, x, r, p, q, kp, P.seg_lo.p, P.seg_hi.p,
-                       P.bseg.p + P.nb + 1, sc, bpart.p, r32);
+    hipLaunchKernelGGL((k_kr_bupdate<T, F, 2>), dim3(R.nseg), dim3(256), 0, s, x, r, p, q, rf, f, kp, R.seg_lo.p,
+                       R.seg_hi.p, R.bseg.p + R.nb + 1, sc, bpart.p);
   LG_LAUNCH_CHECK();
 }
 
@@ -946,14 +1060,27 @@ void op_kr_bpupdate(T *p, const T *z, int kp, const RedPlan &P, const double *sc
                               DevBuf<double> &, hipStream_t);                                        \
   template void op_bprolong_add<T>(const int32_t *, int64_t, const T *, T *, int, hipStream_t);      \
   template void op_bdense_apply<T>(const double *, int64_t, const T *, T *, int, hipStream_t);       \
+  template void RedPlan::bpartials<T>(int, int, const T *, const T *, const T *, const T *,          \
+                                      DevBuf<double> &, hipStream_t) const;                          \
   template void RedPlan::bdots<T>(int, int, const T *, const T *, const T *, const T *, double *,    \
                                   DevBuf<double> &, hipStream_t) const;                              \
   template void op_bsub_block_mean<T>(T *, int, const RedPlan &, const double *, hipStream_t);         \
-  template void op_kr_bupdate<T>(T *, T *, const T *, const T *, int, const RedPlan &, const double *,  \
-                                 DevBuf<double> &, float *, hipStream_t);                            \
+  template void op_bspmv_first<T>(const DCsr &, const T *, T *, const FirstStep<T> &, int,             \
+                                  DevBuf<double> &, hipStream_t);                                    \
   template void op_kr_bpupdate<T>(T *, const T *, int, const RedPlan &, const double *, hipStream_t);
 LG_BINST(double)
 LG_BINST(float)
 #undef LG_BINST
+#define LG_BKR(T, F)                                                                                            \
+  template void op_kr_bbegin<T, F>(const RedPlan &, const T *, T *, T *, F *, const FirstStep<F> &, int,        \
+                                   DevBuf<double> &, hipStream_t);                                             \
+  template void op_kr_bupdate<T, F>(const RedPlan &, T *, T *, const T *, const T *, F *, const FirstStep<F> &, \
+                                    int, const double *, DevBuf<double> &, hipStream_t);                       \
+  template void op_bcenter<T, F>(const RedPlan &, T *, const F *, const T *, int, const double *,              \
+                                 DevBuf<double> &, hipStream_t);
+LG_BKR(double, double)
+LG_BKR(double, float)
+LG_BKR(float, float)
+#undef LG_BKR
 
 }  // namespace lg

@@ -62,6 +62,25 @@ void op_dense_apply(const double *Pinv, int64_t n, const T *x, T *y, hipStream_t
 void op_d2f(const double *a, float *b, int64_t n, hipStream_t s);
 void op_f2d(const float *a, double *b, int64_t n, hipStream_t s);
 
+// What the host sees of a block's convergence, in pinned memory; seq counts
+// the norms of a solve from 1.
+struct KrHost {
+  double rn2, active;
+  unsigned long long seq, pad;
+};
+// What follows a block reduction: its sums to out[(blk * np + j) * kp + c],
+// or a scalar step of the Krylov sets (blk, c) on them (INIT, NORM: also for
+// the host, when host is set).
+struct BlockPost {
+  enum Kind { OUT, INIT, NORM, ALPHA, BETA };
+  Kind kind = OUT;
+  double *out = nullptr, *sc = nullptr;
+  int fcg = 0;
+  double rtol = 0;
+  KrHost *host = nullptr;
+  unsigned long long *seq = nullptr;
+};
+
 // Plan of a deterministic blocked reduction over vectors of length n split
 // into contiguous blocks (independent graphs).  Stage 1 sums fixed chunks
 // clipped to block boundaries (one workgroup each, fixed tree); stage 2
@@ -88,17 +107,14 @@ struct RedPlan {
   template <class T>
   void bdots(int np, int kp, const T *a0, const T *b0, const T *a1, const T *b1, double *out,
              DevBuf<double> &bpart, hipStream_t s) const;
-  // the second stage of bdots alone, from segment partials a fused kernel
-  // wrote to bpart in bdots' layout
-  void bdots_finish(int np, int kp, double *out, const DevBuf<double> &bpart, hipStream_t s) const;
+  // segment partials only (part[(s * np + j) * kp + c]), for bfinish
+  template <class T>
+  void bpartials(int np, int kp, const T *a0, const T *b0, const T *a1, const T *b1, DevBuf<double> &bpart,
+                 hipStream_t s) const;
+  // the second stage and what follows it, from such partials
+  void bfinish(int np, int kp, const BlockPost &P, const DevBuf<double> &bpart, hipStream_t s) const;
 };
 
-// What the host sees of a block's convergence, in pinned memory; seq counts
-// the norms of a solve from 1.
-struct KrHost {
-  double rn2, active;
-  unsigned long long seq, pad;
-};
 // One Krylov iteration on a level (sc: SC_N scalars per block): the start
 // from x = 0, the norm of r with the convergence flag, then z = c - mean
 // (with z.w: q for FCG, r for CG), p = z + beta p, the dots of q = A p (r only
@@ -125,6 +141,9 @@ template <class T> void op_sub_block_mean(T *a, const RedPlan &P, const double *
 // row-major n x kp, kp a power of two <= 64.
 template <class T>
 void op_bspmv(const DCsr &A, const T *X, T *Y, int kp, DevBuf<double> &parts, hipStream_t s);
+template <class T>
+void op_bspmv_first(const DCsr &A, const T *X, T *Y, const FirstStep<T> &f, int kp, DevBuf<double> &parts,
+                    hipStream_t s);
 // picks A's batched SpMM tile for this precision and block width by timing
 // the candidates once (kept in A.U); returns the tile id
 template <class T>
@@ -147,12 +166,6 @@ template <class T>
 void op_bdense_apply(const double *Pm, int64_t n, const T *X, T *Y, int kp, hipStream_t s);
 template <class T>
 void op_bsub_block_mean(T *a, int kp, const RedPlan &P, const double *sums, hipStream_t s);
-// z = c (FP32) minus the block means of c from sums, in FP64: the same bits as
-// converting c and then subtracting the means.  With w set, also the segment
-// partials of z.w in bpart, as RedPlan::bdots forms them (finish them with
-// bdots_finish).
-void op_bsub_block_mean_f2d(double *z, const float *c, int kp, const RedPlan &P, const double *sums, hipStream_t s,
-                            const double *w = nullptr, DevBuf<double> *bpart = nullptr);
 // Rows of a block vector's segment: 8192 entries, 16 pairs for each of a
 // workgroup's 256 threads, at most the vector dots' 4096 rows; longer where
 // there would be more than 2048 segments, whose partials one workgroup adds.
@@ -160,11 +173,18 @@ inline int64_t block_seg_rows(int64_t n, int kp) {
   const int64_t rows = kp >= 2 ? 8192 / kp : 4096;
   return std::max(rows, (n + 2047) / 2048);
 }
-// x += alpha p, r -= alpha q, the segment partials of r.r in bpart (bdots'
-// layout) and, with r32 set, r in FP32; p = z + beta p
-template <class T>
-void op_kr_bupdate(T *x, T *r, const T *p, const T *q, int kp, const RedPlan &P, const double *sc,
-                   DevBuf<double> &bpart, float *r32, hipStream_t s);
+// One block Krylov iteration, as the vector steps above: the start from x =
+// 0, z = c - mean with the partials of z.w, p = z + beta p, and x += alpha p,
+// r -= alpha q with the partials of r.r; rf, f as in kr_update.
+template <class T, class F>
+void op_kr_bbegin(const RedPlan &R, const T *b, T *x, T *r, F *rf, const FirstStep<F> &f, int kp,
+                  DevBuf<double> &bpart, hipStream_t s);
+template <class T, class C>
+void op_bcenter(const RedPlan &R, T *z, const C *c, const T *w, int kp, const double *sums, DevBuf<double> &bpart,
+                hipStream_t s);
+template <class T, class F>
+void op_kr_bupdate(const RedPlan &R, T *x, T *r, const T *p, const T *q, F *rf, const FirstStep<F> &f, int kp,
+                   const double *sc, DevBuf<double> &bpart, hipStream_t s);
 template <class T>
 void op_kr_bpupdate(T *p, const T *z, int kp, const RedPlan &P, const double *sc, hipStream_t s);
 // column-major n x k caller block <-> row-major n x kp internal block; the

@@ -40,23 +40,6 @@ namespace {
 using namespace sdev;
 
 // per-block scalar logic of CG / FCG (one thread per block)
-__global__ void k_kr_alpha(int nb, int fcg, double *sc) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < nb) kr_alpha(sc + c * SC_N, fcg);
-}
-__global__ void k_kr_check(int nb, double rtol, double *sc) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < nb) kr_check(sc + c * SC_N, rtol);
-}
-__global__ void k_kr_beta(int nb, int fcg, double *sc) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < nb) kr_beta(sc + c * SC_N, fcg);
-}
-__global__ void k_kr_init(int nb, double *sc) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < nb) kr_init(sc + c * SC_N);
-}
-
 // FGMRES: y += sum_t coef[blk * K + t] V_t (V_t = V + t ld), added in t order
 __global__ void __launch_bounds__(256) k_blk_lincomb(double *y, const double *V, int64_t ld, int k,
                                                      const double *coef, int K, const int64_t *lo,
@@ -79,14 +62,6 @@ __global__ void __launch_bounds__(256) k_blk_scale(double *y, const double *x, c
 
 inline bool fcg_like(int t) { return t == LIGMG_KSP_FCG || t == LIGMG_KSP_PIPEFCG; }
 
-// batch: dot results out[(blk * np + j) * kp + c] -> scalar sets of (blk, c)
-__global__ void k_kr_bstore(int nb, int kp, int np, const double *out, int s0, int s1, double *sc) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nb * kp) return;
-  const int blk = t / kp, c = t % kp;
-  sc[t * SC_N + s0] = out[((int64_t)blk * np) * kp + c];
-  if (np > 1) sc[t * SC_N + s1] = out[((int64_t)blk * np + 1) * kp + c];
-}
 template <class T>
 struct KWork {
   DevBuf<T> r, z, p, q, x;
@@ -134,12 +109,6 @@ struct BLevelWork {
   KWork<T> kw;  // K-cycle: vectors n*kp, scalars nb*kp sets
 };
 
-inline int ilog2(int k) {
-  int l = 0;
-  while ((1 << l) < k) l++;
-  return l;
-}
-
 struct Solver {
   ligmg_options o;
   hipStream_t s = nullptr;
@@ -171,7 +140,9 @@ struct Solver {
   // captured outer iterations, keyed by everything they read or write that
   // another solve may have moved
   std::vector<std::pair<std::array<const void *, 9>, hipGraphExec_t>> it_graphs;
-  PinnedBuf<KrHost> kr_host;         // per block, written by the norm kernel
+  // captured batched iterations, dropped whenever their work buffers move
+  std::vector<std::pair<std::array<const void *, 9>, hipGraphExec_t>> bgraphs;
+  PinnedBuf<KrHost> kr_host;         // per block (and column), written by the norm kernels
   DevBuf<unsigned long long> kr_seq;
   // fused coarse tail: levels tail_l0.. (H.size(): none), the row
   // schedules of their operators (A, P, R, M per level), the device tables
@@ -199,6 +170,7 @@ struct Solver {
   ~Solver() {
     for (auto &g : graphs) (void)hipGraphExecDestroy(g.second);
     for (auto &g : it_graphs) (void)hipGraphExecDestroy(g.second);
+    drop_batch_graphs();
     if (s) (void)hipStreamDestroy(s);
   }
 
@@ -1578,12 +1550,6 @@ struct Solver {
     }
   }
 
-  static bool any_active(const std::vector<double> &hsc, int nb) {
-    for (int c = 0; c < nb; c++)
-      if (hsc[c * SC_N + SC_ACTIVE] != 0) return true;
-    return false;
-  }
-
   // FGMRES: outer preconditioner in FP64, cycle in FP32 when mixed.  With
   // o.use_graphs the whole application (hundreds of launches on the coarse
   // levels) is captured once per (level, r, z) and replayed as a hipGraph;
@@ -1652,6 +1618,7 @@ struct Solver {
 
   void batch_buffers(int kp) {
     if (bkp == kp) return;
+    drop_batch_graphs();
     balloc<double>(kp);
     if (mixed) balloc<float>(kp);
     // scratch sized once for every operator, so no buffer is reallocated
@@ -1707,7 +1674,7 @@ struct Solver {
 
   // block version of cycle(): same buffer discipline
   template <class T>
-  const T *bcycle(size_t l, const T *b, int kp) {
+  const T *bcycle(size_t l, const T *b, int kp, bool first = false) {
     DLevel &L = H[l];
     BLevelWork<T> &w = bwork<T>(l);
     if (L.kind == LIGMG_LEVEL_COARSE || l == dense_l0) {
@@ -1715,9 +1682,7 @@ struct Solver {
       return w.B[0].p;
     }
     if (L.kind == LIGMG_LEVEL_ELIM) {
-      BLevelWork<T> &wn = bwork<T>(l + 1);
-      op_bspmv<T>(L.R, b, wn.b.p, kp, bparts, s);
-      const T *xc = brecurse<T>(l, wn.b.p, kp);
+      const T *xc = bdescend<T>(l, L.R, b, kp);
       op_binterp<T>(L.P, qv<T>(L), xc, b, w.B[0].p, kp, bparts, s);
       return w.B[0].p;
     }
@@ -1733,7 +1698,7 @@ struct Solver {
         cur = 1;
       }
     } else {
-      op_bcheb_step<T>(L.A, dinv, b, nullptr, nullptr, w.B[1].p, 0.0, be_pre[l][0], kp, bparts, s);
+      if (!first) op_bcheb_step<T>(L.A, dinv, b, nullptr, nullptr, w.B[1].p, 0.0, be_pre[l][0], kp, bparts, s);
       for (int k = 1; k < m; k++) {
         const T *xp = (k == 1) ? nullptr : w.B[(k - 1) % 3].p;
         op_bcheb_step<T>(L.A, dinv, b, w.B[k % 3].p, xp, w.B[(k + 1) % 3].p, al_pre[l][k],
@@ -1741,10 +1706,8 @@ struct Solver {
       }
       cur = m % 3;
     }
-    BLevelWork<T> &wn = bwork<T>(l + 1);
     op_bresidual<T>(L.A, w.B[cur].p, b, w.R.p, kp, bparts, s);
-    op_bspmv<T>(L.M, w.R.p, wn.b.p, kp, bparts, s);
-    const T *xc = brecurse<T>(l, wn.b.p, kp);
+    const T *xc = bdescend<T>(l, L.M, w.R.p, kp);
     op_bprolong_add<T>(L.agg.p, L.n, xc, w.B[cur].p, kp, s);
     const int mp = o.post_smooth;
     if (o.smoother_type == LIGMG_SMOOTHER_JACOBI) {
@@ -1763,135 +1726,134 @@ struct Solver {
     return w.B[cur].p;
   }
 
+  // level l + 1's correction for the right-hand sides Op V
   template <class T>
-  const T *brecurse(size_t l, const T *bc, int kp) {
-    const DLevel &N = H[l + 1];
-    if (!inner_krylov(l + 1)) return bcycle<T>(l + 1, bc, kp);
-    BLevelWork<T> &wn = bwork<T>(l + 1);
-    KWork<T> &K = wn.kw;
-    fill_zero<T>(K.x.p, N.A.n * kp);
-    bkrylov<T>(l + 1, N.A, K.x.p, bc, K, kp, o.kcycle_ksp_type, o.tol, o.kcycle_iters, false, nullptr,
-               nullptr, false);
+  const T *bdescend(size_t l, const DCsr &Op, const T *V, int kp) {
+    T *b = bwork<T>(l + 1).b.p;
+    FirstStep<T> f;
+    if (!inner_krylov(l + 1)) f = bfirst_step<T>(l + 1);
+    op_bspmv_first<T>(Op, V, b, f, kp, bparts, s);
+    if (!inner_krylov(l + 1)) return bcycle<T>(l + 1, b, kp, f.x != nullptr);
+    KWork<T> &K = bwork<T>(l + 1).kw;
+    bkrylov<T>(l + 1, H[l + 1].A, K.x.p, b, K, kp, o.kcycle_ksp_type, o.tol, o.kcycle_iters);
     return K.x.p;
   }
 
-  // z = (cycle applied to r) minus its block means.  r32_ready: the FP32
-  // copy of r for the mixed outer preconditioner is already in place.  On
-  // that path, with w set, the segment partials of z.w are also left in
-  // bpart_red (returns true); otherwise returns false.
   template <class T>
-  bool bprec(size_t lvl, const T *r, T *z, int kp, bool outer_prec, bool r32_ready = false,
-             const T *w = nullptr) {
-    const int64_t n = H[lvl].A.n;
-    if constexpr (std::is_same<T, double>::value) {
-      if (outer_prec && mixed) {
-        // the block sums come from the FP32 result itself (the FP64 copy has
-        // the same values), and one pass converts and subtracts the means
-        BLevelWork<float> &bw = BW32[lvl];
-        if (!r32_ready) op_d2f(r, bw.b.p, n * kp, s);
-        const float *c = bcycle<float>(lvl, bw.b.p, kp);
-        const RedPlan &R = bred[lvl];
-        R.bdots<float>(1, kp, c, nullptr, nullptr, nullptr, bsc_out.p, bpart_red, s);
-        op_bsub_block_mean_f2d(z, c, kp, R, bsc_out.p, s, w, &bpart_red);
-        return w != nullptr;
-      } else {
-        d2d(z, bcycle<T>(lvl, r, kp), n * kp, s);
-      }
-    } else {
-      d2d(z, bcycle<T>(lvl, r, kp), n * kp, s);
-    }
-    const RedPlan &R = bred[lvl];
-    R.bdots<T>(1, kp, z, nullptr, nullptr, nullptr, bsc_out.p, bpart_red, s);
-    op_bsub_block_mean<T>(z, kp, R, bsc_out.p, s);
-    return false;
+  FirstStep<T> bfirst_step(size_t l) {
+    FirstStep<T> f = first_step<T>(l);
+    if (f.x) f.x = bwork<T>(l).B[1].p;
+    return f;
   }
 
-  template <class T>
-  void bdot(const RedPlan &R, int kp, const T *a0, const T *b0, const T *a1, const T *b1,
-            KWork<T> &K, int s0, int s1) {
-    const int np = a1 ? 2 : 1;
-    R.bdots<T>(np, kp, a0, b0, a1, b1, K.out.p, bpart_red, s);
-    hipLaunchKernelGGL(k_kr_bstore, dim3((R.nb * kp + 63) / 64), dim3(64), 0, s, R.nb, kp, np, K.out.p,
-                       s0, s1, K.sc.p);
+  // per-(block, column) CG / FCG on block vectors: the iteration of iterate()
+  // with a set of scalars per (block, column)
+  template <class T, class F>
+  void biterate(size_t lvl, const DCsr &A, T *x, KWork<T> &K, F *rf, int kp, bool fcg, double rtol, bool norm,
+                KrHost *host) {
+    const RedPlan &R = bred[lvl];
+    const FirstStep<F> f = bfirst_step<F>(lvl);
+    const F *r = rf;
+    if constexpr (std::is_same<T, F>::value)
+      if (!rf) r = K.r.p;
+    const F *c = bcycle<F>(lvl, r, kp, f.x != nullptr);
+    R.bdots<F>(1, kp, c, nullptr, nullptr, nullptr, bsc_out.p, bpart_red, s);
+    op_bcenter<T, F>(R, K.z.p, c, fcg ? K.q.p : K.r.p, kp, bsc_out.p, bpart_red, s);
+    BlockPost P;
+    P.sc = K.sc.p;
+    P.fcg = fcg ? 1 : 0;
+    P.rtol = rtol;
+    P.kind = BlockPost::BETA;
+    R.bfinish(1, kp, P, bpart_red, s);
+    op_kr_bpupdate<T>(K.p.p, K.z.p, kp, R, K.sc.p, s);
+    op_bspmv<T>(A, K.p.p, K.q.p, kp, bparts, s);
+    R.bpartials<T>(fcg ? 2 : 1, kp, K.p.p, K.q.p, fcg ? K.p.p : nullptr, fcg ? K.r.p : nullptr, bpart_red, s);
+    P.kind = BlockPost::ALPHA;
+    R.bfinish(fcg ? 2 : 1, kp, P, bpart_red, s);
+    op_kr_bupdate<T, F>(R, x, K.r.p, K.p.p, K.q.p, rf, f, kp, K.sc.p, bpart_red, s);
+    if (!norm) return;
+    P.kind = BlockPost::NORM;
+    P.host = host;
+    P.seq = kr_seq.p;
+    R.bfinish(1, kp, P, bpart_red, s);
   }
 
-  // per-(block, column) CG / FCG on block vectors; iters_col (host, may be
-  // null) receives for every scalar set the iteration it converged at
-  template <class T>
-  int bkrylov(size_t lvl, const DCsr &A, T *x, const T *b, KWork<T> &K, int kp, int type,
-              double rtol, int maxit, bool host_check, std::vector<int> *iters_set, int *status,
-              bool outer_prec) {
+  template <class T, class F>
+  void bbegin(size_t lvl, const T *b, T *x, KWork<T> &K, F *rf, int kp, double rtol, KrHost *host) {
     const RedPlan &R = bred[lvl];
-    const int ns = R.nb * kp;
-    const bool fcg = fcg_like(type);
-    auto grid1 = dim3((ns + 63) / 64);
-    hipLaunchKernelGGL(k_kr_init, grid1, dim3(64), 0, s, ns, K.sc.p);
-    op_bresidual<T>(A, x, b, K.r.p, kp, bparts, s);
-    bdot<T>(R, kp, b, b, K.r.p, K.r.p, K, SC_BN2, SC_RN2);
-    hipLaunchKernelGGL(k_kr_check, grid1, dim3(64), 0, s, ns, rtol, K.sc.p);
-    if (status) *status = LIGMG_CONVERGED;
-    std::vector<double> hsc;
-    std::vector<char> was_active(ns, 0);
-    if (iters_set) iters_set->assign(ns, 0);
-    if (host_check) {
-      hsc = download(K.sc.p, (size_t)ns * SC_N, s);
-      for (int t = 0; t < ns; t++) was_active[t] = hsc[t * SC_N + SC_ACTIVE] != 0;
-      if (!any_active(hsc, ns)) return 0;
-    }
-    const int64_t nk = A.n * kp;
-    bprec<T>(lvl, K.r.p, K.z.p, kp, outer_prec);
-    d2d(K.p.p, K.z.p, nk, s);
-    bdot<T>(R, kp, K.r.p, K.z.p, (const T *)nullptr, (const T *)nullptr, K, SC_GAMMA, SC_GAMMA);
-    int it = 0;
-    while (it < maxit) {
-      op_bspmv<T>(A, K.p.p, K.q.p, kp, bparts, s);
-      if (fcg) bdot<T>(R, kp, K.p.p, K.q.p, K.p.p, K.r.p, K, SC_DELTA, SC_T1);
-      else bdot<T>(R, kp, K.p.p, K.q.p, (const T *)nullptr, (const T *)nullptr, K, SC_DELTA, SC_DELTA);
-      hipLaunchKernelGGL(k_kr_alpha, grid1, dim3(64), 0, s, ns, fcg ? 1 : 0, K.sc.p);
-      // the update also forms r.r's segment partials and, for the mixed
-      // outer preconditioner, the FP32 copy of r
-      float *r32 = nullptr;
-      if constexpr (std::is_same<T, double>::value)
-        if (outer_prec && mixed) r32 = BW32[lvl].b.p;
-      op_kr_bupdate<T>(x, K.r.p, K.p.p, K.q.p, kp, R, K.sc.p, bpart_red, r32, s);
-      it++;
-      R.bdots_finish(1, kp, K.out.p, bpart_red, s);
-      hipLaunchKernelGGL(k_kr_bstore, dim3((R.nb * kp + 63) / 64), dim3(64), 0, s, R.nb, kp, 1, K.out.p, SC_RN2,
-                         SC_RN2, K.sc.p);
-      hipLaunchKernelGGL(k_kr_check, grid1, dim3(64), 0, s, ns, rtol, K.sc.p);
-      if (host_check) {
-        hsc = download(K.sc.p, (size_t)ns * SC_N, s);
-        bool nan = false;
-        for (int t = 0; t < ns; t++) {
-          double r2 = hsc[t * SC_N + SC_RN2];
-          if (r2 != r2) nan = true;
-          const bool act = hsc[t * SC_N + SC_ACTIVE] != 0;
-          if (iters_set && (was_active[t] || act)) (*iters_set)[t] = it;
-          was_active[t] = act;
-        }
-        if (nan) {
-          if (status) *status = LIGMG_DIVERGED_NAN;
-          return it;
-        }
-        if (!any_active(hsc, ns)) return it;
+    op_kr_bbegin<T, F>(R, b, x, K.r.p, rf, bfirst_step<F>(lvl), kp, bpart_red, s);
+    BlockPost P;
+    P.kind = BlockPost::INIT;
+    P.sc = K.sc.p;
+    P.rtol = rtol;
+    P.host = host;
+    P.seq = kr_seq.p;
+    R.bfinish(1, kp, P, bpart_red, s);
+  }
+
+  // the K-cycle's inner solve
+  template <class T>
+  void bkrylov(size_t lvl, const DCsr &A, T *x, const T *b, KWork<T> &K, int kp, int type, double rtol, int maxit) {
+    bbegin<T, T>(lvl, b, x, K, nullptr, kp, rtol, nullptr);
+    for (int it = 0; it < maxit; it++)
+      biterate<T, T>(lvl, A, x, K, nullptr, kp, fcg_like(type), rtol, it + 1 < maxit, nullptr);
+  }
+
+  // the outer solve; its[t] receives the iteration set t = (block, column)
+  // converged at
+  int bkrylov_solve(size_t lvl, double *x, const double *b, KWork<double> &K, int kp, std::vector<int> &its,
+                    int *status) {
+    const DCsr &A = H[lvl].A;
+    const int ns = bred[lvl].nb * kp;
+    const bool fcg = fcg_like(o.outer_ksp_type);
+    kr_host.ensure((size_t)ns);
+    kr_seq.ensure((size_t)ns);
+    for (int t = 0; t < ns; t++) kr_host.p[t].seq = 0;  // the stream is idle here
+    std::atomic_thread_fence(std::memory_order_release);
+    auto body = [&] {
+      if (mixed) biterate<double, float>(lvl, A, x, K, BW32[lvl].b.p, kp, fcg, o.tol, true, kr_host.p);
+      else biterate<double, double>(lvl, A, x, K, nullptr, kp, fcg, o.tol, true, kr_host.p);
+    };
+    if (mixed) bbegin<double, float>(lvl, b, x, K, BW32[lvl].b.p, kp, o.tol, kr_host.p);
+    else bbegin<double, double>(lvl, b, x, K, nullptr, kp, o.tol, kr_host.p);
+    its.assign(ns, 0);
+    std::vector<char> was(ns, 1);
+    *status = LIGMG_CONVERGED;
+    for (int it = 0;; it++) {
+      bool active = false;
+      const double tn = wait_norm(ns, (unsigned long long)it + 1, &active);
+      for (int t = 0; t < ns; t++) {
+        const bool act = kr_host.p[t].active != 0;
+        if (it > 0 && (was[t] || act)) its[t] = it;
+        was[t] = act;
       }
-      if (it >= maxit) break;
-      // z.q (FCG) or r.z (CG): formed by the preconditioner's last pass
-      // where it can, else a block dot
-      if (bprec<T>(lvl, K.r.p, K.z.p, kp, outer_prec, true, fcg ? K.q.p : K.r.p)) {
-        R.bdots_finish(1, kp, K.out.p, bpart_red, s);
-        hipLaunchKernelGGL(k_kr_bstore, dim3((R.nb * kp + 63) / 64), dim3(64), 0, s, R.nb, kp, 1, K.out.p,
-                           fcg ? SC_T1 : SC_GN, fcg ? SC_T1 : SC_GN, K.sc.p);
-      } else if (fcg) {
-        bdot<T>(R, kp, K.z.p, K.q.p, (const T *)nullptr, (const T *)nullptr, K, SC_T1, SC_T1);
-      } else {
-        bdot<T>(R, kp, K.r.p, K.z.p, (const T *)nullptr, (const T *)nullptr, K, SC_GN, SC_GN);
+      if (it > 0 && tn != tn) {
+        *status = LIGMG_DIVERGED_NAN;
+        return it;
       }
-      hipLaunchKernelGGL(k_kr_beta, grid1, dim3(64), 0, s, ns, fcg ? 1 : 0, K.sc.p);
-      op_kr_bpupdate<T>(K.p.p, K.z.p, kp, R, K.sc.p, s);
+      if (!active) return it;
+      if (it >= o.iters) break;
+      if (!o.use_graphs) {
+        body();
+        continue;
+      }
+      const std::array<const void *, 9> key = {&A, x, K.r.p, K.z.p, K.p.p, K.q.p, K.sc.p, kr_host.p, kr_seq.p};
+      hipGraphExec_t e = nullptr;
+      for (auto &g : bgraphs)
+        if (g.first == key) e = g.second;
+      if (!e) {
+        e = capture(body);
+        bgraphs.push_back({key, e});
+      }
+      LG_HIP(hipGraphLaunch(e, s));
     }
-    if (host_check && status) *status = LIGMG_DIVERGED_ITS;
-    return it;
+    *status = LIGMG_DIVERGED_ITS;
+    return o.iters;
+  }
+
+  void drop_batch_graphs() {
+    for (auto &g : bgraphs) (void)hipGraphExecDestroy(g.second);
+    bgraphs.clear();
   }
 
   int solve_batch(int k, const double *B, double *X, int mem, ligmg_info *info, int32_t *iters_out);
@@ -1924,9 +1886,12 @@ int Solver::solve_batch(int k, const double *Bin, double *Xout, int mem, ligmg_i
   const int64_t nbse = H[base].A.n;
   int maxnb = 1;
   for (auto &r : red) maxnb = std::max(maxnb, r.nb);
-  bsc_out.ensure((size_t)maxnb * kp * 2);
-  if (bouter.x.n < (size_t)(nbse * kp) || bouter.sc.n < (size_t)(red[base].nb * kp * SC_N))
+  if (bsc_out.n < (size_t)maxnb * kp * 2 || bouter.x.n < (size_t)(nbse * kp) ||
+      bouter.sc.n < (size_t)(red[base].nb * kp * SC_N)) {
+    drop_batch_graphs();
+    bsc_out.ensure((size_t)maxnb * kp * 2);
     bouter.alloc(nbse * kp, red[base].nb * kp);
+  }
   DevBuf<double> bin(n * k), b0b(n * kp), rhs(nbse * kp), solb(n * kp), tmp(n * kp);
   if (mem == LIGMG_MEM_HOST) to_device(bin.p, Bin, n * k, s);
   else d2d(bin.p, Bin, n * k, s);
@@ -1937,11 +1902,9 @@ int Solver::solve_batch(int k, const double *Bin, double *Xout, int mem, ligmg_i
   else d2d(rhs.p, b0b.p, n * kp, s);
   bred[base].bdots<double>(1, kp, rhs.p, nullptr, nullptr, nullptr, bsc_out.p, bpart_red, s);
   op_bsub_block_mean<double>(rhs.p, kp, bred[base], bsc_out.p, s);
-  fill_zero<double>(bouter.x.p, nbse * kp);
   std::vector<int> its;
   int status = 0;
-  int iters = bkrylov<double>(base, H[base].A, bouter.x.p, rhs.p, bouter, kp, o.outer_ksp_type, o.tol,
-                              o.iters, true, &its, &status, true);
+  const int iters = bkrylov_solve(base, bouter.x.p, rhs.p, bouter, kp, its, &status);
   if (do_once) op_binterp<double>(L0.P, L0.q.p, bouter.x.p, b0b.p, solb.p, kp, bparts, s);
   else d2d(solb.p, bouter.x.p, n * kp, s);
   op_from_block(solb.p, n, k, kp, bin.p, perm.p, s);
