@@ -187,6 +187,77 @@ void degree_perm(const DCsr &A, const std::vector<int64_t> &blocks, DevBuf<int32
   LG_HIP(hipStreamSynchronize(s));
 }
 
+namespace {
+// The fine vertices under coarse vertex a: an aggregate's members (its row of
+// M), or, under an elimination level (prp set), those in its row of R whose
+// first P entry is a (the kept vertex, and each eliminated one once).
+struct Children {
+  const int32_t *rp, *ci, *prp, *pci;
+  template <class F>
+  __device__ __forceinline__ void each(int a, const F &f) const {
+    for (int k = rp[a]; k < rp[a + 1]; k++) {
+      const int v = ci[k];
+      if (!prp || (prp[v] < prp[v + 1] && pci[prp[v]] == a)) f(v);
+    }
+  }
+};
+// children of the coarse vertex at position p (cnt[nc] = 0)
+__global__ void k_child_count(int64_t nc, const int32_t *cperm, Children C, int32_t *cnt) {
+  for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p <= nc; p += (int64_t)gridDim.x * blockDim.x) {
+    int n = 0;
+    if (p < nc) C.each(cperm ? cperm[p] : (int)p, [&](int) { n++; });
+    cnt[p] = n;
+  }
+}
+__global__ void k_child_fill(int64_t nc, const int32_t *cperm, Children C, const int32_t *off, int32_t *perm,
+                             int32_t *iperm) {
+  for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < nc; p += (int64_t)gridDim.x * blockDim.x) {
+    int o = off[p];
+    C.each(cperm ? cperm[p] : (int)p, [&](int v) {
+      perm[o] = v;
+      iperm[v] = o;
+      o++;
+    });
+  }
+}
+__global__ void __launch_bounds__(256) k_max_row(int64_t n, const int32_t *rp, int32_t *longest) {
+  int32_t m = 0;
+  for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x)
+    m = max(m, rp[r + 1] - rp[r]);
+  for (int off = WAVE / 2; off >= 1; off >>= 1) m = max(m, __shfl_xor(m, off, WAVE));
+  if ((threadIdx.x & (WAVE - 1)) == 0) atomicMax(longest, m);
+}
+}  // namespace
+
+int32_t longest_row(const DCsr &A, hipStream_t s) {
+  DevBuf<int32_t> d(1);
+  fill_i32(d.p, 0, 1, s);
+  hipLaunchKernelGGL(k_max_row, dim3(grid_for(A.n, 256, 256)), dim3(256), 0, s, A.n, A.rp.p, d.p);
+  LG_LAUNCH_CHECK();
+  int32_t h = 0;
+  to_host(&h, d.p, 1, s);
+  LG_HIP(hipStreamSynchronize(s));
+  return h;
+}
+
+bool cluster_perm(const DLevel &L, const int32_t *cperm, DevBuf<int32_t> &perm, DevBuf<int32_t> &iperm, hipStream_t s) {
+  const int64_t n = L.A.n, nc = L.nc;
+  const DCsr &D = L.kind == LIGMG_LEVEL_ELIM ? L.R : L.M;
+  if (nc <= 0 || D.n != nc || !D.rp.p || !D.ci.p) return false;
+  const Children C{D.rp.p, D.ci.p, L.kind == LIGMG_LEVEL_ELIM ? L.P.rp.p : nullptr, L.P.ci.p};
+  DevBuf<int32_t> off(nc + 1);
+  hipLaunchKernelGGL(k_child_count, dim3(grid_for(nc + 1, 256, 16384)), dim3(256), 0, s, nc, cperm, C, off.p);
+  LG_LAUNCH_CHECK();
+  // a vertex without a coarse neighbour (an isolated one) has no place
+  if (exclusive_scan_i32(off.p, off.p, nc + 1, s) != n) return false;
+  perm.alloc(n);
+  iperm.alloc(n);
+  hipLaunchKernelGGL(k_child_fill, dim3(grid_for(nc, 256, 16384)), dim3(256), 0, s, nc, cperm, C,
+                     (const int32_t *)off.p, perm.p, iperm.p);
+  LG_LAUNCH_CHECK();
+  return true;
+}
+
 template <class Body>
 void for_dst_entries(int64_t n, const int32_t *nrp, const Body &body, hipStream_t s) {
   if (n <= 0) return;

@@ -62,6 +62,11 @@ void setup_aggregation(const DCsr &A, const ligmg_options &o, int level_idx, DLe
 // Renumber A's vertices by descending row length inside each block (ties
 // by ascending index); perm receives internal position -> input vertex.
 void degree_order(DCsr &A, const std::vector<int64_t> &blocks, DevBuf<int32_t> &perm, hipStream_t s);
+// Cluster order of level L from the order of the next one (cperm: position
+// to vertex, null: its own): vertices follow their coarse vertex.  False (and
+// no result) when some vertex has none.
+bool cluster_perm(const DLevel &L, const int32_t *cperm, DevBuf<int32_t> &perm, DevBuf<int32_t> &iperm, hipStream_t s);
+int32_t longest_row(const DCsr &A, hipStream_t s);
 // Degree permutation of A's rows inside blocks (perm: new -> old, iperm:
 // old -> new), the one degree_order applies.
 void degree_perm(const DCsr &A, const std::vector<int64_t> &blocks, DevBuf<int32_t> &perm, DevBuf<int32_t> &iperm,

@@ -665,14 +665,44 @@ struct Solver {
   }
 
   // Solve layout (see DLevel::sperm): levels of at least SOLVE_PERM_MIN
-  // vertices other than the coarsest get a degree permutation; the level
+  // vertices other than the coarsest are renumbered; the level
   // matrix keeps each row's entries in their order (same row sums), the
   // transfer operators are relabeled on both sides.
   static constexpr int64_t SOLVE_PERM_MIN = 1 << 16;
+  // Which permutation: levels with hubs are sorted by degree (the hubs'
+  // entries of x, gathered most, then share a few cache lines); levels of even
+  // rows, meshes and their like, take the cluster order, where vertices follow
+  // their aggregate, aggregates theirs, and so on from the coarsest level up,
+  // so a row's neighbours are mostly close by.  On a geometric graph of 700 K
+  // randomly numbered vertices the FP64 Chebyshev step goes from 81 us (degree
+  // order; 84 unsorted) to 42 us and the solve from 36.2 to 24.5 ms; on a 100^3
+  // grid, row by row already, from 178 to 165 us for 32 columns.  Power-law
+  // levels have no such clusters and gain from the hubs (R-MAT 20: 10.9 -> 9.1 ms).
+  static constexpr int64_t EVEN_ROWS = 8;  // longest row over the mean one
   void apply_solve_layout() {
     const size_t nl = H.size();
+    std::vector<char> even(nl, 0);
+    size_t last = nl;  // the finest level that takes the cluster order
+    if (H[0].blocks.size() == 2)
+      for (size_t l = nl - 1; l-- > 0;)
+        if (H[l].A.n >= SOLVE_PERM_MIN && longest_row(H[l].A, s) * H[l].A.n <= EVEN_ROWS * H[l].A.nnz) {
+          even[l] = 1;
+          last = l;
+        }
+    DevBuf<int32_t> perm_c, iperm_c;  // the order of the level below (null: its own)
+    for (size_t l = nl - 1; last < nl && l-- > last;) {
+      DevBuf<int32_t> pm, ip;
+      if (!cluster_perm(H[l], perm_c.p, pm, ip, s)) break;
+      if (even[l]) {
+        H[l].sperm.alloc(H[l].A.n);
+        d2d(H[l].sperm.p, pm.p, H[l].A.n, s);
+        H[l].siperm = std::move(ip);
+      }
+      perm_c = std::move(pm);
+    }
     for (size_t l = 0; l + 1 < nl; l++)
-      if (H[l].A.n >= SOLVE_PERM_MIN) degree_perm(H[l].A, H[l].blocks, H[l].sperm, H[l].siperm, s);
+      if (H[l].A.n >= SOLVE_PERM_MIN && !H[l].sperm.p)
+        degree_perm(H[l].A, H[l].blocks, H[l].sperm, H[l].siperm, s);
     for (size_t l = 0; l + 1 < nl; l++) {
       DLevel &V = H[l];
       const DLevel &N = H[l + 1];
