@@ -403,32 +403,49 @@ __global__ void k_bcheb_zero(const T *dinv, const T *b, T *xn, double beta, int6
     xn[t] = (T)(beta * (double)dinv[t >> lk] * (double)b[t]);
 }
 
-template <class T>
-__global__ void k_bprolong(const int32_t *agg, int64_t n, int kp, int lk, const T *xc, T *x) {
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < (n << lk);
-       t += (int64_t)gridDim.x * blockDim.x)
-    x[t] += xc[(int64_t)agg[t >> lk] * kp + (t & (kp - 1))];
+// x += xc[agg], 16 bytes a thread (or the whole row of a narrower block); lv =
+// log2 of the threads per row
+template <class T, int VW>
+__global__ void __launch_bounds__(256) k_bprolong(const int32_t *__restrict__ agg, int64_t n, int lv, const T *__restrict__ xc,
+                                                  T *__restrict__ x) {
+  typedef typename BVec<T, VW>::type V;
+  const V *c = (const V *)xc;
+  V *y = (V *)x;
+  for (int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x; t < (n << lv); t += (int64_t)gridDim.x * 256)
+    y[t] += c[((int64_t)agg[t >> lv] << lv) + (t & ((1 << lv) - 1))];
 }
 
-// column-major (ld n) <-> row-major n x kp (padding columns zero)
-// column-major caller block (vertex order given by perm, identity when
-// null) <-> row-major internal block
-__global__ void k_to_block(const double *B, int64_t n, int k, int kp, const int32_t *perm, double *X) {
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n * kp;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t i = t / kp;
-    const int c = (int)(t % kp);
-    const int64_t src = perm ? perm[i] : i;
-    X[t] = c < k ? B[(int64_t)c * n + src] : 0.0;
+// Column-major caller block (ld n, vertex order given by perm, identity when
+// null) <-> row-major internal block (padding columns zero).  A workgroup
+// turns 64 rows in LDS, so both sides are read and written along their rows
+// (one entry a thread left every access on a line of its own: 649 us for
+// 10^6 x 32, 262 us now).
+constexpr int TURN_ROWS = 64;
+__global__ void __launch_bounds__(256) k_to_block(const double *__restrict__ B, int64_t n, int k, int kp, int lk,
+                                                  const int32_t *__restrict__ perm, double *__restrict__ X) {
+  __shared__ double tile[TURN_ROWS * 65];
+  const int64_t i0 = (int64_t)blockIdx.x * TURN_ROWS;
+  const int rows = (int)min((int64_t)TURN_ROWS, n - i0);
+  const int r = threadIdx.x % TURN_ROWS;
+  if (r < rows) {
+    const int64_t src = perm ? perm[i0 + r] : i0 + r;
+    for (int c = threadIdx.x / TURN_ROWS; c < kp; c += 256 / TURN_ROWS)
+      tile[r * (kp + 1) + c] = c < k ? B[(int64_t)c * n + src] : 0.0;
   }
+  __syncthreads();
+  for (int t = threadIdx.x; t < rows << lk; t += 256) X[(i0 << lk) + t] = tile[(t >> lk) * (kp + 1) + (t & (kp - 1))];
 }
-__global__ void k_from_block(const double *X, int64_t n, int k, int kp, const int32_t *perm, double *B) {
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n * k;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t c = t / n, i = t % n;
-    const int64_t dst = perm ? perm[i] : i;
-    B[c * n + dst] = X[i * kp + c];
-  }
+__global__ void __launch_bounds__(256) k_from_block(const double *__restrict__ X, int64_t n, int k, int kp, int lk,
+                                                    const int32_t *__restrict__ perm, double *__restrict__ B) {
+  __shared__ double tile[TURN_ROWS * 65];
+  const int64_t i0 = (int64_t)blockIdx.x * TURN_ROWS;
+  const int rows = (int)min((int64_t)TURN_ROWS, n - i0);
+  for (int t = threadIdx.x; t < rows << lk; t += 256) tile[(t >> lk) * (kp + 1) + (t & (kp - 1))] = X[(i0 << lk) + t];
+  __syncthreads();
+  const int r = threadIdx.x % TURN_ROWS;
+  if (r >= rows) return;
+  const int64_t dst = perm ? perm[i0 + r] : i0 + r;
+  for (int c = threadIdx.x / TURN_ROWS; c < k; c += 256 / TURN_ROWS) B[(int64_t)c * n + dst] = tile[r * (kp + 1) + c];
 }
 
 // ------------------------------------------------------- coarse dense apply
@@ -598,15 +615,17 @@ __global__ void __launch_bounds__(256) k_bred1(int np, int kp, const T *a0, cons
 }
 
 // The segment partials of block blk, summed per column, and what follows
-// (BlockPost): one workgroup per block.  Thread (g, c) adds segments g, g + G,
-// ... (G = 1024 / kp) in order, and the G partials of a column are added 16
-// at a time.  The scalar steps of the block's (blk, column) sets run here, so a
-// dot costs no launch beyond its two stages.
-__global__ void __launch_bounds__(1024) k_bred2(int np, int kp, int lk, const int32_t *bseg, const double *part,
+// (BlockPost): one workgroup per block and cw = min(kp, 8) columns.  Thread (g,
+// c) adds segments g, g + G, ... (G = 1024 / cw) in order, and the G partials of
+// a column are added 16 at a time.  (All 32 columns of 2045 segments in one
+// workgroup took 21 us, bound by that CU's reads.)  The scalar steps of the
+// (blk, column) sets run here, so a dot costs no launch beyond its two stages.
+constexpr int BRED_COLS = 8;
+__global__ void __launch_bounds__(1024) k_bred2(int np, int kp, int lw, const int32_t *bseg, const double *part,
                                                 BlockPost P) {
   const int blk = blockIdx.x;
-  const int G = 1024 >> lk;
-  const int g = threadIdx.x >> lk, c = threadIdx.x & (kp - 1);
+  const int cw = 1 << lw, G = 1024 >> lw;
+  const int g = threadIdx.x >> lw, cl = threadIdx.x & (cw - 1), c = blockIdx.y * cw + cl;
   const int end = bseg[blk + 1];
   __shared__ double red[1024];
   double sum[2] = {0, 0};
@@ -620,12 +639,12 @@ __global__ void __launch_bounds__(1024) k_bred2(int np, int kp, int lk, const in
       const int m = (n + 15) / 16;
       double t = 0;
       if (g < m)
-        for (int q = 16 * g; q < min(16 * g + 16, n); q++) t += red[q * kp + c];
+        for (int q = 16 * g; q < min(16 * g + 16, n); q++) t += red[q * cw + cl];
       __syncthreads();
       if (g < m) red[threadIdx.x] = t;
       __syncthreads();
     }
-    sum[j] = red[c];
+    sum[j] = red[cl];
     __syncthreads();
   }
   if (g != 0) return;
@@ -917,8 +936,13 @@ void op_binterp(const DCsr &P, const T *q, const T *Xc, const T *B, T *X, int kp
 }
 template <class T>
 void op_bprolong_add(const int32_t *agg, int64_t n, const T *Xc, T *X, int kp, hipStream_t s) {
-  hipLaunchKernelGGL(k_bprolong<T>, dim3(grid_for(n * kp, 256, 16384)), dim3(256), 0, s, agg, n, kp,
-                     log2i(kp), Xc, X);
+  const int vw = spmm_vw<T>(kp), lv = log2i(kp / vw);
+  const dim3 g(grid_for(n << lv, 256, 16384));
+  switch (vw) {
+    case 1: hipLaunchKernelGGL((k_bprolong<T, 1>), g, dim3(256), 0, s, agg, n, lv, Xc, X); break;
+    case 2: hipLaunchKernelGGL((k_bprolong<T, 2>), g, dim3(256), 0, s, agg, n, lv, Xc, X); break;
+    default: hipLaunchKernelGGL((k_bprolong<T, 4>), g, dim3(256), 0, s, agg, n, lv, Xc, X);
+  }
   LG_LAUNCH_CHECK();
 }
 template <class T>
@@ -945,13 +969,14 @@ void op_bdense_apply(const double *Pm, int64_t n, const T *X, T *Y, int kp, hipS
 }
 
 void op_to_block(const double *B, int64_t n, int k, int kp, double *X, const int32_t *perm, hipStream_t s) {
-  hipLaunchKernelGGL(k_to_block, dim3(grid_for(n * kp, 256, 16384)), dim3(256), 0, s, B, n, k, kp, perm, X);
+  hipLaunchKernelGGL(k_to_block, dim3((unsigned)((n + TURN_ROWS - 1) / TURN_ROWS)), dim3(256), 0, s, B, n, k, kp,
+                     log2i(kp), perm, X);
   LG_LAUNCH_CHECK();
 }
 void op_from_block(const double *X, int64_t n, int k, int kp, double *B, const int32_t *perm,
                    hipStream_t s) {
-  hipLaunchKernelGGL(k_from_block, dim3(grid_for(n * k, 256, 16384)), dim3(256), 0, s, X, n, k, kp, perm,
-                     B);
+  hipLaunchKernelGGL(k_from_block, dim3((unsigned)((n + TURN_ROWS - 1) / TURN_ROWS)), dim3(256), 0, s, X, n, k, kp,
+                     log2i(kp), perm, B);
   LG_LAUNCH_CHECK();
 }
 
@@ -981,7 +1006,8 @@ void RedPlan::bdots(int np, int kp, const T *a0, const T *b0, const T *a1, const
 void RedPlan::bfinish(int np, int kp, const BlockPost &P, const DevBuf<double> &bpart, hipStream_t s) const {
   if (nb == 0) return;
   LG_CHECK(bpart.n >= (size_t)nseg * np * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
-  hipLaunchKernelGGL(k_bred2, dim3((unsigned)nb), dim3(1024), 0, s, np, kp, log2i(kp), bseg.p,
+  const int cw = std::min(kp, BRED_COLS);
+  hipLaunchKernelGGL(k_bred2, dim3((unsigned)nb, (unsigned)(kp / cw)), dim3(1024), 0, s, np, kp, log2i(cw), bseg.p,
                      (const double *)bpart.p, P);
   LG_LAUNCH_CHECK();
 }
