@@ -1,10 +1,10 @@
 // The coarse levels of a V-cycle as one dense matrix.
 //
 // A V-cycle with fixed smoothers is linear, so the cycle from a level of n
-// vertices down is an n x n matrix.  For the first level of at most
-// COLLAPSE_MAX_N vertices setup forms it column block by column block: every
-// operation of the cycle runs once on all n unit vectors (row-major blocks of
-// n columns, a thread per column), about ten launches per level.  The solve
+// vertices down is an n x n matrix.  For the first level that collapse_fits
+// takes, setup forms it: every operation of the cycle runs once on all n unit
+// vectors (row-major blocks of n columns, a thread per column), about ten
+// launches per level.  The solve
 // then replaces the whole coarse recursion, a chain of small dependent
 // launches, by one dense product.
 #include <algorithm>

@@ -6,11 +6,15 @@
 
 namespace lg {
 
-// Largest level collapsed.  A product with 1024^2 entries (8 MiB, resident in
-// the L2s) takes about 4 us, the levels below it 50 to 150 us of dependent
-// launches: R-MAT 10 solve 1.37 -> 0.70 ms, 256 x 256 grid 14.6 -> 12.3 ms; forming
-// it costs a setup about 0.2 ms.
-constexpr int64_t COLLAPSE_MAX_N = 1024;
+// Whether a level is small enough to collapse.  A product with 1024^2 entries
+// (8 MiB, resident in the L2s) takes about 4 us, the levels below it 50 to 150
+// us of dependent launches: R-MAT 10 solve 1.37 -> 0.70 ms, 256 x 256 grid 14.6 ->
+// 12.3 ms.  Forming the matrix takes about a dozen operations of nnz * n
+// multiply-adds per level (0.2 ms at 1024), so sparse levels may be twice as
+// large (the grid 6.5 -> 5.8 ms, 181 x 97 x 3 columns 4.7 -> 4.2 ms, a 250 K-vertex
+// gradient with its setup 39.3 -> 37.5 ms) while a dense one of 1700 vertices cost a
+// single solve 0.15 ms more than it gained.
+inline bool collapse_fits(int64_t n, int64_t nnz) { return n <= 1024 || (n <= 2048 && nnz <= 16 * n); }
 
 // What the cycle does besides its operators: smoother coefficients per level
 // (al[l][k] and be[l][k] of step k), the smoother, the constant correction.

@@ -1046,14 +1046,14 @@ struct Solver {
     return rec[e];
   }
 
-  // The first level (from the outer solve's on) of at most COLLAPSE_MAX_N
-  // vertices, with the levels below it, becomes one matrix: V-cycles only
+  // The first level (from the outer solve's on) that collapse_fits takes,
+  // with the levels below it, becomes one matrix: V-cycles only
   // (a K-cycle's inner Krylov solves are not linear).
   void setup_dense(size_t base) {
     dense_l0 = H.size();
     if (o.kcycle) return;
     size_t l = base;
-    while (H[l].A.n > COLLAPSE_MAX_N && H[l].kind != LIGMG_LEVEL_COARSE) l++;
+    while (!collapse_fits(H[l].A.n, H[l].A.nnz) && H[l].kind != LIGMG_LEVEL_COARSE) l++;
     if (H[l].kind == LIGMG_LEVEL_COARSE) return;  // already one dense matrix
     collapse_cycle(H, {al_pre, be_pre, al_post, be_post, o.pre_smooth, o.post_smooth,
                        o.smoother_type == LIGMG_SMOOTHER_JACOBI, o.constant_correction ? 4.0 / 3.0 : 1.0},

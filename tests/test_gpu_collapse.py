@@ -1,6 +1,6 @@
 """V-cycles whose coarse levels are one dense matrix (the first level of at
-most 1024 vertices and everything below it), against the oracle's cycle from
-every level: the levels above it, the collapsed one, and those below."""
+most 1024 vertices, 2048 where rows are short, and everything below it),
+against the oracle's cycle from every level: the levels above it, the collapsed one, and those below."""
 import numpy as np
 import pytest
 
@@ -20,8 +20,10 @@ VARIANTS = {
     "kcycle": {"kcycle": 1},  # nothing is collapsed
 }
 GRAPHS = {
-    "grid32": lambda: graphs.grid2d(32, 32),  # the base level has exactly 1024 vertices
-    "grid33": lambda: graphs.grid2d(41, 25, graphs.W_UNIFORM, 0.1, 10.0, 3),  # 1025: one above
+    "grid32": lambda: graphs.grid2d(64, 32),  # the base level has exactly 2048 vertices
+    "grid33": lambda: graphs.grid2d(683, 3, graphs.W_UNIFORM, 0.1, 10.0, 3),  # 2049: one above
+    "dense1024": lambda: graphs.barabasi_albert(1024, 20, seed=2),  # long rows: at the smaller bound
+    "dense1025": lambda: graphs.barabasi_albert(1025, 20, seed=2),
     "rmat12": lambda: graphs.rmat_config(12, "lognormal", pendants=True),
     "tiny": lambda: graphs.barabasi_albert(60, 2, seed=1),
 }
