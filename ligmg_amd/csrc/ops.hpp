@@ -134,6 +134,17 @@ template <class T, class F>
 void kr_update(const RedPlan &R, T *x, T *r, const T *p, const T *q, double *sc, bool fcg, F *rf,
                const FirstStep<F> &f, hipStream_t s);
 
+// Device scalars of the eigenvalue estimate's CG by step (eig_begin, eig_step
+// on a one-block plan): gamma (steps + 1), running flag (steps + 1), delta,
+// alpha, beta (steps each).
+struct EigState {
+  double *G, *A, *D, *AL, *BE;
+};
+void eig_begin(const RedPlan &R, double *r, const double *dinv, double *z, double *p, const EigState &E, hipStream_t s);
+// after q = A p
+void eig_step(const RedPlan &R, double *r, const double *dinv, double *z, double *p, const double *q,
+              const EigState &E, int it, hipStream_t s);
+
 // a -= mean of a over each block, means taken from sums[c] (device)
 template <class T> void op_sub_block_mean(T *a, const RedPlan &P, const double *sums, hipStream_t s);
 

@@ -1867,52 +1867,6 @@ __global__ void k_eig_init(int n, uint64_t seed, uint64_t stream, const int32_t 
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) r[i] = ligmg_rng::u01(seed, stream, perm ? perm[i] : i);
 }
-__global__ void k_axpy_dev(int n, const double *alpha, double sign, const double *x, double *y) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) y[i] += sign * alpha[0] * x[i];
-}
-__global__ void k_mul(int n, const double *a, const double *b, double *c) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) c[i] = a[i] * b[i];
-}
-__global__ void k_xpby_dev(int n, const double *x, const double *beta, double *p) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = x[i] + beta[0] * p[i];
-}
-
-// Scalars of the estimator.  They stay on the device; the recorded alpha and
-// beta are read once, after the last step.  The stop rules are those of the
-// loop `while gamma > 0: ...; if !(delta > 0) break`.
-enum { EG_GAMMA = 0, EG_DELTA, EG_GN, EG_ALPHA, EG_BETA, EG_ACTIVE, EG_M, EG_N };
-
-// after gamma = (r, z)
-__global__ void k_eig_start(double *sc) {
-  sc[EG_ACTIVE] = sc[EG_GAMMA] > 0 ? 1.0 : 0.0;
-  sc[EG_M] = 0;
-}
-// after delta = (p, A p): alpha = gamma / delta, or stop
-__global__ void k_eig_alpha(double *sc) {
-  double a = 0;
-  if (sc[EG_ACTIVE] != 0) {
-    if (sc[EG_DELTA] > 0) a = sc[EG_GAMMA] / sc[EG_DELTA];
-    else sc[EG_ACTIVE] = 0;
-  }
-  sc[EG_ALPHA] = a;
-}
-// after gn = (r, z): record (alpha, gn / gamma), gamma = gn, stop unless gn > 0
-__global__ void k_eig_beta(double *sc, double *al, double *be) {
-  double b = 0;
-  if (sc[EG_ACTIVE] != 0) {
-    const int m = (int)sc[EG_M];
-    b = sc[EG_GN] / sc[EG_GAMMA];
-    al[m] = sc[EG_ALPHA];
-    be[m] = b;
-    sc[EG_M] = m + 1;
-    sc[EG_GAMMA] = sc[EG_GN];
-    if (!(sc[EG_GN] > 0)) sc[EG_ACTIVE] = 0;
-  }
-  sc[EG_BETA] = b;
-}
 }  // namespace
 
 double tridiag_max_eig(const std::vector<double> &d, const std::vector<double> &e) {
@@ -1944,46 +1898,33 @@ double tridiag_max_eig(const std::vector<double> &d, const std::vector<double> &
 }
 
 double eig_estimate(const DCsr &A, const double *dinv, uint64_t seed, int level_idx, int iters,
-                    const int32_t *perm, hipStream_t s) {
+                    const int32_t *perm, const RedPlan *plan, hipStream_t s) {
   const int64_t n = A.n;
   if (n == 0) return 1.0;
-  RedPlan R;
-  R.build(n, {0, n}, s);
-  DevBuf<double> r(n), z(n), p(n), q(n), sc(EG_N), al(std::max(iters, 1)), be(std::max(iters, 1));
+  RedPlan own;
+  if (!plan || plan->nb != 1) {
+    own.build(n, {0, n}, s);
+    plan = &own;
+  }
+  const RedPlan &R = *plan;
+  const size_t st = (size_t)std::max(iters, 1) + 1;
+  DevBuf<double> r(n), z(n), p(n), q(n), sc(5 * st);
+  const EigState E{sc.p, sc.p + st, sc.p + 2 * st, sc.p + 3 * st, sc.p + 4 * st};
   hipLaunchKernelGGL(k_eig_init, dim3(g1(n)), dim3(256), 0, s, (int)n, seed,
                      ligmg_rng::STREAM_EIG + (uint64_t)level_idx, perm, r.p);
   LG_LAUNCH_CHECK();
-  R.sums(r.p, sc.p, s);
-  op_sub_block_mean(r.p, R, sc.p, s);
-  hipLaunchKernelGGL(k_mul, dim3(g1(n)), dim3(256), 0, s, (int)n, dinv, r.p, z.p);
-  d2d(p.p, z.p, n, s);
-  auto dot = [&](const double *a, const double *b, int slot) {
-    const double *A_[1] = {a}, *B_[1] = {b};
-    R.dots(1, A_, B_, sc.p + slot, s);
-  };
-  dot(r.p, z.p, EG_GAMMA);
-  hipLaunchKernelGGL(k_eig_start, dim3(1), dim3(1), 0, s, sc.p);
-  LG_LAUNCH_CHECK();
+  eig_begin(R, r.p, dinv, z.p, p.p, E, s);
   // a stopped estimator runs the remaining steps with alpha = beta = 0 and
-  // records nothing more
+  // records nothing more: the stop rules are those of the loop `while gamma >
+  // 0: ...; if !(delta > 0) break`
   for (int it = 0; it < iters; it++) {
     op_spmv<double>(A, p.p, q.p, s);
-    dot(p.p, q.p, EG_DELTA);
-    hipLaunchKernelGGL(k_eig_alpha, dim3(1), dim3(1), 0, s, sc.p);
-    hipLaunchKernelGGL(k_axpy_dev, dim3(g1(n)), dim3(256), 0, s, (int)n, sc.p + EG_ALPHA, -1.0, q.p, r.p);
-    hipLaunchKernelGGL(k_mul, dim3(g1(n)), dim3(256), 0, s, (int)n, dinv, r.p, z.p);
-    dot(r.p, z.p, EG_GN);
-    hipLaunchKernelGGL(k_eig_beta, dim3(1), dim3(1), 0, s, sc.p, al.p, be.p);
-    hipLaunchKernelGGL(k_xpby_dev, dim3(g1(n)), dim3(256), 0, s, (int)n, z.p, sc.p + EG_BETA, p.p);
-    LG_LAUNCH_CHECK();
+    eig_step(R, r.p, dinv, z.p, p.p, q.p, E, it, s);
   }
-  double h_sc[EG_N];
-  std::vector<double> ha(al.n), hb(be.n);
-  to_host(h_sc, sc.p, EG_N, s);
-  to_host(ha.data(), al.p, al.n, s);
-  to_host(hb.data(), be.p, be.n, s);
-  LG_HIP(hipStreamSynchronize(s));
-  const int m = (int)h_sc[EG_M];  // entries beyond m were never written
+  const std::vector<double> h = download(sc.p, sc.n, s);
+  const double *run = h.data() + st, *delta = h.data() + 2 * st, *ha = h.data() + 3 * st, *hb = h.data() + 4 * st;
+  int m = 0;
+  while (m < iters && run[m] != 0 && delta[m] > 0) m++;
   if (m == 0) return 1.0;
   std::vector<double> d(m), e(m > 1 ? m - 1 : 0);
   for (int j = 0; j < m; j++) {

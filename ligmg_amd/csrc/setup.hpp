@@ -4,6 +4,8 @@
 
 namespace lg {
 
+struct RedPlan;
+
 // Contract (key = row << cb | col, value) pairs into CSR (destroys the inputs).
 void contract_to_csr(DevBuf<uint64_t> &keys, DevBuf<uint64_t> &vals, int64_t m, int64_t nrows,
                      int64_t ncols, DCsr &out, hipStream_t s);
@@ -92,9 +94,10 @@ void setup_dinv(const DCsr &A, DLevel &L, bool fp32, hipStream_t s);
 // FP32 P, R = P^T and Q of an elimination level from the FP32 Laplacian form
 // of its matrix (L.A.v32 / L.A.d32 must exist).
 void make_elim32(DLevel &L, hipStream_t s);
-// perm (may be null): setup position of each row, for the start vector
+// perm (may be null): setup position of each row, for the start vector; plan:
+// A's reduction plan, used where it has one block (else one is built here)
 double eig_estimate(const DCsr &A, const double *dinv, uint64_t seed, int level_idx, int iters,
-                    const int32_t *perm, hipStream_t s);
+                    const int32_t *perm, const RedPlan *plan, hipStream_t s);
 // Dense pseudo-inverse of the coarsest level (n <= COARSE_DENSE_MAX): the
 // inverse of L + sum over components C of 1_C 1_C^T / |C|, minus those terms.
 constexpr int64_t COARSE_DENSE_MAX = 8192;

@@ -340,7 +340,7 @@ struct Solver {
         setup_dinv(L.A, L, mixed, s);
         if (o.smoother_type == LIGMG_SMOOTHER_CHEBYSHEV) {
           timed(t_eig, [&] {
-            L.lam = eig_estimate(L.A, L.dinv.p, o.seed, (int)l, o.cheby_eig_iters, L.sperm.p, s);
+            L.lam = eig_estimate(L.A, L.dinv.p, o.seed, (int)l, o.cheby_eig_iters, L.sperm.p, &red[l], s);
           });
           L.cheb_lo = o.cheby_lower * L.lam;
           L.cheb_hi = o.cheby_upper * L.lam;
