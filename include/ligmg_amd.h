@@ -127,8 +127,10 @@ typedef struct ligmg_options {
   int32_t ordering;             /* LIGMG_ORDER_NATURAL: vertex order used for
                                    setup and solve (see enum)               */
   int32_t solve_layout;         /* 1: the solve-phase copy of every large
-                                   level is stored in degree order (gather
-                                   locality; the hierarchy is unchanged);
+                                   level is stored in degree order, or
+                                   cluster by cluster where its rows are
+                                   even (gather locality; the hierarchy is
+                                   unchanged);
                                    0: setup order                           */
   int32_t tail_nnz;             /* 4096: the coarse levels whose operators
                                    hold at most this many stored entries
@@ -142,10 +144,10 @@ typedef struct ligmg_options {
   int32_t rejection_to_seed;    /* false: a rejected vertex becomes undecided;
                                    true: a seed                             */
   int32_t spmm_tune;            /* 1: batched solves time the SpMM tiles
-                                   (right-hand sides per lane, gathers in
-                                   flight) of every level operator at the
-                                   first solve of each batch width and keep
-                                   the fastest; 0: the fixed tile.  Results
+                                   (gathers in flight) of every large level
+                                   operator at the first solve of each batch
+                                   width and keep the fastest; 0, and smaller
+                                   operators: the rule's tile.  Results
                                    are the same bits either way. (new)      */
 } ligmg_options;
 

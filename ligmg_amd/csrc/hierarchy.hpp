@@ -77,8 +77,8 @@ struct Units {
   // lanes per row of the row kernel (k_spmv_rows) when the operator's rows
   // suit it, else 0: the units above
   int32_t row_k = 0;
-  // batched SpMM tile picked per precision (0 FP64, 1 FP32) and log2 of the
-  // block width; -1 until tuned (the fixed tile is used)
+  // gathers in flight of the batched SpMM, picked per precision (0 FP64, 1
+  // FP32) and log2 of the block width; -1 until tuned (the rule's is used)
   int8_t spmm_cfg[2][8] = {{-1, -1, -1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1, -1, -1}};
 };
 
@@ -128,9 +128,9 @@ struct DLevel {
   // coarse: dense pseudo-inverse, row-major n x n
   DevBuf<double> pinv;
   // Solve layout: the solve-phase copies (A, dinv, agg, M, P, R, q) of a
-  // large level are renumbered by descending degree inside blocks; sperm maps
-  // a solve position to the setup position (empty: setup order kept),
-  // siperm is its inverse.  agg_setup / new_id keep the setup-order maps for
+  // large level are renumbered inside blocks, by descending degree or, where
+  // rows are even, cluster by cluster; sperm maps a solve position to the
+  // setup position (empty: setup order kept), siperm is its inverse.  agg_setup / new_id keep the setup-order maps for
   // introspection; new_id_s is new_id in solve order.
   DevBuf<int32_t> sperm, siperm, agg_setup, new_id_s;
   std::vector<int64_t> blocks;  // contiguous vertex blocks (independent graphs)
