@@ -983,6 +983,7 @@ void op_from_block(const double *X, int64_t n, int k, int kp, double *B, const i
 template <class T>
 void RedPlan::bpartials(int np, int kp, const T *a0, const T *b0, const T *a1, const T *b1, DevBuf<double> &bpart,
                         hipStream_t s) const {
+  if (nseg == 0) return;
   LG_CHECK(bpart.n >= (size_t)nseg * np * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
   if (kp == 1)
     hipLaunchKernelGGL((k_bred1<T, 1>), dim3(nseg), dim3(256), 0, s, np, kp, a0, b0, a1, b1, seg_lo.p, seg_hi.p,
@@ -1016,6 +1017,7 @@ void RedPlan::bfinish(int np, int kp, const BlockPost &P, const DevBuf<double> &
 template <class T, class C>
 void op_bcenter(const RedPlan &R, T *z, const C *c, const T *w, int kp, const double *sums, DevBuf<double> &bpart,
                 hipStream_t s) {
+  if (R.nseg == 0) return;
   LG_CHECK(bpart.n >= (size_t)R.nseg * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
   if (kp == 1)
     hipLaunchKernelGGL((k_bcenter<T, C, 1>), LG_SEGS, z, c, w, kp, R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1,
@@ -1028,6 +1030,7 @@ void op_bcenter(const RedPlan &R, T *z, const C *c, const T *w, int kp, const do
 template <class T, class F>
 void op_kr_bbegin(const RedPlan &R, const T *b, T *x, T *r, F *rf, const FirstStep<F> &f, int kp,
                   DevBuf<double> &bpart, hipStream_t s) {
+  if (R.nseg == 0) return;
   LG_CHECK(bpart.n >= (size_t)R.nseg * kp, LIGMG_ERR_INVALID, "block reduction buffer too small");
   if (kp == 1)
     hipLaunchKernelGGL((k_kr_bbegin<T, F, 1>), LG_SEGS, b, x, r, rf, f, kp, R.seg_lo.p, R.seg_hi.p, bpart.p);

@@ -96,6 +96,7 @@ struct Wide {
 
   template <class Epi>
   void mul(const DCsr &A, const double *X, const Epi &e) const {
+    if (A.n == 0) return;  // a level that eliminates every vertex leaves none
     hipLaunchKernelGGL(k_wide<Epi>, grid(A.n), dim3(256), 0, s, A.rp.p, A.ci.p, A.v.p, X, ld, e);
     LG_LAUNCH_CHECK();
   }
@@ -108,6 +109,7 @@ struct Wide {
   void cycle(size_t l, const double *b, DevBuf<double> &x) const {
     const DLevel &L = H[l];
     const int64_t n = L.A.n;
+    if (n == 0) return;
     if (L.kind == LIGMG_LEVEL_COARSE) {
       x.alloc(n * ld);
       hipLaunchKernelGGL(k_wide_dense, grid(n), dim3(256), 0, s, L.pinv.p, n, b, ld, x.p);

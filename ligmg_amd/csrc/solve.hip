@@ -1306,6 +1306,7 @@ template void RedPlan::sums<float>(const float *, double *, hipStream_t) const;
 #define LG_SEGS dim3((unsigned)R.nseg), dim3(256), 0, s
 template <class T, class F>
 void kr_begin(const RedPlan &R, const T *b, T *x, T *r, F *rf, const FirstStep<F> &f, hipStream_t s) {
+  if (R.nseg == 0) return;
   hipLaunchKernelGGL((k_kr_begin<T, F>), LG_SEGS, b, x, r, rf, f, R.seg_lo.p, R.seg_hi.p, R.part.p);
   LG_LAUNCH_CHECK();
 }
@@ -1317,18 +1318,21 @@ void kr_norm(const RedPlan &R, double *sc, bool init, double rtol, KrHost *host,
 }
 template <class T>
 void kr_dots(const RedPlan &R, const T *p, const T *q, const T *r, hipStream_t s) {
+  if (R.nseg == 0) return;
   hipLaunchKernelGGL(k_kr_dots<T>, LG_SEGS, p, q, r, R.seg_lo.p, R.seg_hi.p, R.part.p);
   LG_LAUNCH_CHECK();
 }
 template <class T, class F>
 void kr_update(const RedPlan &R, T *x, T *r, const T *p, const T *q, double *sc, bool fcg, F *rf,
                const FirstStep<F> &f, hipStream_t s) {
+  if (R.nseg == 0) return;
   hipLaunchKernelGGL((k_kr_update<T, F>), LG_SEGS, x, r, p, q, rf, f, R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1, R.bseg.p,
                      R.part.p, sc, fcg ? 1 : 0);
   LG_LAUNCH_CHECK();
 }
 template <class T, class C>
 void kr_center(const RedPlan &R, T *z, const C *c, const T *w, hipStream_t s) {
+  if (R.nseg == 0) return;
   hipLaunchKernelGGL(k_kr_sum<C>, LG_SEGS, c, R.seg_lo.p, R.seg_hi.p, R.part.p);
   LG_LAUNCH_CHECK();
   hipLaunchKernelGGL((k_kr_center<T, C>), LG_SEGS, z, c, w, R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1, R.bseg.p,
@@ -1337,6 +1341,7 @@ void kr_center(const RedPlan &R, T *z, const C *c, const T *w, hipStream_t s) {
 }
 template <class T>
 void kr_pupdate(const RedPlan &R, T *p, const T *z, double *sc, bool fcg, hipStream_t s) {
+  if (R.nseg == 0) return;
   hipLaunchKernelGGL(k_kr_pupdate<T>, LG_SEGS, p, z, R.seg_lo.p, R.seg_hi.p, R.bseg.p + R.nb + 1, R.bseg.p,
                      (const double *)R.part.p, sc, fcg ? 1 : 0);
   LG_LAUNCH_CHECK();

@@ -1054,7 +1054,7 @@ struct Solver {
     if (o.kcycle) return;
     size_t l = base;
     while (!collapse_fits(H[l].A.n, H[l].A.nnz) && H[l].kind != LIGMG_LEVEL_COARSE) l++;
-    if (H[l].kind == LIGMG_LEVEL_COARSE) return;  // already one dense matrix
+    if (H[l].kind == LIGMG_LEVEL_COARSE || H[l].A.n == 0) return;  // already one dense matrix
     collapse_cycle(H, {al_pre, be_pre, al_post, be_post, o.pre_smooth, o.post_smooth,
                        o.smoother_type == LIGMG_SMOOTHER_JACOBI, o.constant_correction ? 4.0 / 3.0 : 1.0},
                    l, dense_m, s);

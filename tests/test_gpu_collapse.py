@@ -64,3 +64,15 @@ def test_collapsed_batch_and_blocks(k, prec):
     for c in {0, k - 1}:
         x = s.solve(np.ascontiguousarray(B[:, c])).solution
         assert np.linalg.norm(X[:, c] - x) <= 1e-7 * np.linalg.norm(x)
+
+
+@pytest.mark.parametrize("kw", [{}, {"precision": _ffi.PREC_MIXED, "outer_ksp_type": _ffi.KSP_FCG},
+                                {"outer_ksp_type": _ffi.KSP_FGMRES}, {"kcycle": 1, "outer_ksp_type": _ffi.KSP_FCG}])
+def test_empty_coarsest_level(kw):
+    """min_size = 0 coarsens on until an elimination takes every vertex: the
+    levels below are empty, and nothing is launched for them."""
+    g = graphs.barabasi_albert(300, 3, seed=4)
+    s = ligmg_amd.Solver(g, ligmg_amd.Options(min_size=0, **kw))
+    assert s.level_info(s.num_levels() - 1)[1] == 0
+    info = s.solve(graphs.rhs(g.n, 1, 0))
+    assert info.status == _ffi.CONVERGED and info.rel_residual() <= 1e-8
