@@ -947,6 +947,7 @@ void op_bprolong_add(const int32_t *agg, int64_t n, const T *Xc, T *X, int kp, h
 }
 template <class T>
 void op_bdense_apply(const double *Pm, int64_t n, const T *X, T *Y, int kp, hipStream_t s) {
+  if (n == 0) return;  // an elimination took every vertex: a grid of 0 is a launch error
   if (kp >= 16) {
     LG_CHECK(kp == 16 || kp == 32 || kp == 64, LIGMG_ERR_INVALID, "dense apply: kp must be 16, 32 or 64");
     const unsigned g = (unsigned)((n + 15) / 16);

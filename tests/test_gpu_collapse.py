@@ -76,3 +76,24 @@ def test_empty_coarsest_level(kw):
     assert s.level_info(s.num_levels() - 1)[1] == 0
     info = s.solve(graphs.rhs(g.n, 1, 0))
     assert info.status == _ffi.CONVERGED and info.rel_residual() <= 1e-8
+
+
+@pytest.mark.parametrize("k", [1, 3, 8, 16, 33])
+@pytest.mark.parametrize("kw", [{}, {"kcycle": 1, "outer_ksp_type": _ffi.KSP_FCG},
+                                {"kcycle": 1, "precision": _ffi.PREC_MIXED, "outer_ksp_type": _ffi.KSP_FCG}])
+@pytest.mark.parametrize("name", ["one", "union"])
+def test_empty_coarsest_level_batch(name, kw, k):
+    """The same in batches, at a width of every dense kernel: one graph
+    (collapsed in V-cycles, not in K-cycles), and a union of stars whose
+    first level of at most 2048 vertices is the empty one."""
+    star = graphs.from_edges(4, np.zeros(3, np.int64), np.arange(1, 4), np.ones(3))
+    u = graphs.union([graphs.barabasi_albert(300, 3, seed=4)] if name == "one" else [star] * 2100)
+    print(f"{name} {kw} k={k} n={u.n}", flush=True)
+    s = ligmg_amd.Solver(u, ligmg_amd.Options(min_size=0, **kw), comp_ptr=u.comp_ptr)
+    assert s.level_info(s.num_levels() - 1)[1] == 0
+    B = graphs.rhs(u.n, k, 3, comp_ptr=u.comp_ptr).reshape(u.n, k, order="F")
+    X, info, its = s.solve_batch(B)
+    assert info.status == _ffi.CONVERGED and info.full_rel_residual <= 1e-7
+    x = s.solve(np.ascontiguousarray(B[:, k - 1])).solution
+    A = u.to_scipy()
+    assert np.linalg.norm(A @ (X[:, k - 1] - x)) <= 2e-7 * np.linalg.norm(B[:, k - 1])
