@@ -42,6 +42,10 @@ constexpr int WAVE = 64;
 void *dev_alloc(size_t bytes);
 void dev_free(void *p);
 void dev_pool_trim();
+// Pooled pinned host memory that the GPU can write.  host_free's block may be
+// handed out at once: no queued work may still use it.
+void *host_alloc(size_t bytes);
+void host_free(void *p);
 // bracket a graph capture: the pool then never synchronises the device
 void pool_capture_begin();
 void pool_capture_end();
@@ -101,7 +105,7 @@ struct DevBuf {
   size_t bytes() const { return n * sizeof(T); }
 };
 
-// Pinned host memory the GPU writes directly.
+// Pinned host memory the GPU writes directly (pooled).
 template <class T>
 struct PinnedBuf {
   T *p = nullptr;
@@ -109,15 +113,16 @@ struct PinnedBuf {
   PinnedBuf() = default;
   PinnedBuf(const PinnedBuf &) = delete;
   PinnedBuf &operator=(const PinnedBuf &) = delete;
-  ~PinnedBuf() {
-    if (p) (void)hipHostFree(p);
-  }
+  ~PinnedBuf() { host_free(p); }
+  // keeps the block from being handed out again (queued work may write it)
+  void forget() { p = nullptr; }
+  // call with no queued work on the old block
   void ensure(size_t count) {
     if (count <= n) return;
-    if (p) (void)hipHostFree(p);
+    host_free(p);
     p = nullptr;
     n = 0;
-    LG_HIP(hipHostMalloc((void **)&p, count * sizeof(T), hipHostMallocCoherent));
+    p = (T *)host_alloc(count * sizeof(T));
     n = count;
   }
 };

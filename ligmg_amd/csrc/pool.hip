@@ -10,6 +10,10 @@
 // synchronisation gave.  No allocation happens inside a captured graph, and
 // while any handle captures one (on any thread) the pool takes fresh blocks
 // instead of synchronising the device, which would end that capture.
+//
+// Pinned host blocks are kept the same way: hipHostFree synchronises too, and
+// a solver may be destroyed (by a garbage collector, on any thread) while the
+// application captures a graph of its own, which that would invalidate.
 #include <atomic>
 #include <iterator>
 #include <map>
@@ -28,9 +32,11 @@ namespace {
 // bytes kept for reuse at most; above it released blocks go back to HIP
 constexpr size_t CACHE_MAX = (size_t)32 << 30;
 
+constexpr int HOST = -1;  // pinned host memory, for any device
+
 struct Pool {
   std::mutex m;
-  using Key = std::pair<int, size_t>;  // (device, class bytes)
+  using Key = std::pair<int, size_t>;  // (device or HOST, class bytes)
   std::map<Key, std::vector<void *>> ready, pending;
   std::unordered_map<void *, Key> live;
   size_t cached = 0;
@@ -54,11 +60,13 @@ size_t size_class(size_t b) {
   return (p2 > 256 && b <= three_quarters) ? three_quarters : p2;
 }
 
+void give_back(const Pool::Key &key, void *p) { (void)(key.first == HOST ? hipHostFree(p) : hipFree(p)); }
+
 void flush_locked(Pool &P) {
   (void)hipDeviceSynchronize();
   for (auto *lists : {&P.ready, &P.pending})
     for (auto &kv : *lists)
-      for (void *q : kv.second) (void)hipFree(q);
+      for (void *q : kv.second) give_back(kv.first, q);
   P.ready.clear();
   P.pending.clear();
   P.cached = 0;
@@ -132,7 +140,7 @@ void dev_free(void *p) {
     for (auto q = P.ready.begin(); q != P.ready.end() && P.cached > CACHE_MAX;) {
       auto &blocks = q->second;
       while (!blocks.empty() && P.cached > CACHE_MAX) {
-        (void)hipFree(blocks.back());
+        give_back(q->first, blocks.back());
         blocks.pop_back();
         P.cached -= q->first.second;
       }
@@ -142,6 +150,36 @@ void dev_free(void *p) {
   }
   P.pending[key].push_back(p);
   P.cached += key.second;
+}
+
+void *host_alloc(size_t bytes) {
+  if (bytes == 0) return nullptr;
+  const Pool::Key key{HOST, size_class(bytes)};
+  Pool &P = pool();
+  std::lock_guard<std::mutex> g(P.m);
+  void *p = nullptr;
+  auto it = P.ready.find(key);
+  if (it != P.ready.end() && !it->second.empty()) {
+    p = it->second.back();
+    it->second.pop_back();
+    P.cached -= key.second;
+  } else if (hipHostMalloc(&p, key.second, hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();
+    throw Error(LIGMG_ERR_NOMEM, "hipHostMalloc of " + std::to_string(key.second) + " bytes failed");
+  }
+  P.live[p] = key;
+  return p;
+}
+
+void host_free(void *p) {
+  if (!p) return;
+  Pool &P = pool();
+  std::lock_guard<std::mutex> g(P.m);
+  auto it = P.live.find(p);
+  if (it == P.live.end()) return;
+  P.ready[it->second].push_back(p);
+  P.cached += it->second.second;
+  P.live.erase(it);
 }
 
 // Taken under the pool lock, so a synchronisation or free that the pool has

@@ -144,6 +144,7 @@ struct Solver {
   std::vector<std::pair<std::array<const void *, 9>, hipGraphExec_t>> bgraphs;
   PinnedBuf<KrHost> kr_host;         // per block (and column), written by the norm kernels
   DevBuf<unsigned long long> kr_seq;
+  bool kr_pending = false;           // queued kernels may write kr_host: a solve is running or has failed
   // fused coarse tail: levels tail_l0.. (H.size(): none), the row
   // schedules of their operators (A, P, R, M per level), the device tables
   // the programs index, and one recorded program per entry level and
@@ -171,6 +172,7 @@ struct Solver {
     for (auto &g : graphs) (void)hipGraphExecDestroy(g.second);
     for (auto &g : it_graphs) (void)hipGraphExecDestroy(g.second);
     drop_batch_graphs();
+    if (kr_pending) kr_host.forget();
     if (s) (void)hipStreamDestroy(s);
   }
 
@@ -1345,6 +1347,7 @@ struct Solver {
     const RedPlan &R = red[lvl];
     const DCsr &A = H[lvl].A;
     const bool fcg = fcg_like(o.outer_ksp_type);
+    kr_pending = true;
     kr_host.ensure((size_t)R.nb);
     kr_seq.ensure((size_t)R.nb);
     for (int c = 0; c < R.nb; c++) kr_host.p[c].seq = 0;  // the stream is idle here
@@ -1404,7 +1407,9 @@ struct Solver {
 
   int krylov_outer(size_t base, const double *rhs, std::vector<double> &h, int *status) {
     if (o.outer_ksp_type == LIGMG_KSP_FGMRES) return fgmres(base, outer.x.p, rhs, &h, status);
-    return krylov_solve(base, outer.x.p, rhs, outer, h, status);
+    const int iters = krylov_solve(base, outer.x.p, rhs, outer, h, status);
+    kr_pending = false;  // every norm has arrived
+    return iters;
   }
 
   // FGMRES(m) outer solve: restarted flexible GMRES with PETSc KSPFGMRES's
@@ -1836,6 +1841,7 @@ struct Solver {
     const DCsr &A = H[lvl].A;
     const int ns = bred[lvl].nb * kp;
     const bool fcg = fcg_like(o.outer_ksp_type);
+    kr_pending = true;
     kr_host.ensure((size_t)ns);
     kr_seq.ensure((size_t)ns);
     for (int t = 0; t < ns; t++) kr_host.p[t].seq = 0;  // the stream is idle here
@@ -1935,6 +1941,7 @@ int Solver::solve_batch(int k, const double *Bin, double *Xout, int mem, ligmg_i
   std::vector<int> its;
   int status = 0;
   const int iters = bkrylov_solve(base, bouter.x.p, rhs.p, bouter, kp, its, &status);
+  kr_pending = false;  // every norm has arrived
   if (do_once) op_binterp<double>(L0.P, L0.q.p, bouter.x.p, b0b.p, solb.p, kp, bparts, s);
   else d2d(solb.p, bouter.x.p, n * kp, s);
   op_from_block(solb.p, n, k, kp, bin.p, perm.p, s);

@@ -94,3 +94,36 @@ def test_concurrent_handles_with_graph_capture():
         t.join(timeout=120)
     assert not any(t.is_alive() for t in ts)
     assert not errors, errors
+
+
+@pytest.mark.parametrize("mode", ["thread_local", "global"])
+@pytest.mark.parametrize("other", [False, True])
+def test_close_while_the_application_captures(mode, other):
+    """A solver that has solved is destroyed, on the capturing thread or on
+    another, while the application captures a graph: the capture goes on."""
+    import threading
+    import torch
+    g = graphs.barabasi_albert(300, 3, seed=1)
+    solvers = [ligmg_amd.Solver(g, ligmg_amd.Options(outer_ksp_type=k)) for k in (_ffi.KSP_CG, _ffi.KSP_FGMRES)]
+    B = graphs.rhs(g.n, 3, 0).reshape(g.n, 3, order="F")
+    for s in solvers:
+        s.solve(np.ascontiguousarray(B[:, 0]))
+    solvers[0].solve_batch(B)
+    x = torch.ones(1000, device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, capture_error_mode=mode):
+        y = x + 1
+        for s in solvers:
+            if other:
+                t = threading.Thread(target=s.close)
+                t.start()
+                t.join()
+            else:
+                s.close()
+        z = y * 2
+    for rep in range(3):
+        x.fill_(float(rep))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.all(z == 2.0 * (rep + 1))
