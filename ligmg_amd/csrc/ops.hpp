@@ -62,23 +62,42 @@ void op_dense_apply(const double *Pinv, int64_t n, const T *x, T *y, hipStream_t
 void op_d2f(const double *a, float *b, int64_t n, hipStream_t s);
 void op_f2d(const float *a, double *b, int64_t n, hipStream_t s);
 
-// What the host sees of a block's convergence, in pinned memory; seq counts
-// the norms of a solve from 1.
+// What the host sees of a solve's convergence, in pinned memory, by Krylov set
+// (a block, or a block's column); seq counts the norms of a solve from 1.
 struct KrHost {
   double rn2, active;
   unsigned long long seq, pad;
 };
+// Up to this many sets are written to the host one by one; more are added up
+// on the device first (kr_total), into the host's first entry.  A set's three
+// words cross the bus on their own, about 0.1 us a set (12 000 sets 1.24 ms,
+// 192 000 sets 25 ms of an iteration); adding them up takes a launch or two,
+// 2 us more at 100 sets.
+constexpr int KR_HOST_SETS = 128;
+inline int kr_host_entries(int64_t sets) { return sets <= KR_HOST_SETS ? (int)sets : 1; }
+// Where norms go besides the sets' own scalars: nowhere (host null), or to
+// KR_HOST_SETS host entries, with as many counters on the device and
+// KR_TOTAL_PARTS partials of kr_total.
+constexpr int KR_TOTAL_PARTS = 2 * 256;
+struct KrSink {
+  KrHost *host = nullptr;
+  unsigned long long *seq = nullptr;
+  double *part = nullptr;
+  // the sink a norm kernel writes set by set, none where kr_total follows
+  KrSink each(int64_t sets) const { return sets <= KR_HOST_SETS ? *this : KrSink(); }
+};
+// r.r and the active flags of all sets, into the first host entry
+void kr_total(const double *sc, int64_t sets, bool init, const KrSink &to, hipStream_t s);
 // What follows a block reduction: its sums to out[(blk * np + j) * kp + c],
 // or a scalar step of the Krylov sets (blk, c) on them (INIT, NORM: also for
-// the host, when host is set).
+// the host, when to has one).
 struct BlockPost {
   enum Kind { OUT, INIT, NORM, ALPHA, BETA };
   Kind kind = OUT;
   double *out = nullptr, *sc = nullptr;
   int fcg = 0;
   double rtol = 0;
-  KrHost *host = nullptr;
-  unsigned long long *seq = nullptr;
+  KrSink to;
 };
 
 // Plan of a deterministic blocked reduction over vectors of length n split
@@ -88,7 +107,7 @@ struct BlockPost {
 // reproducible.
 struct RedPlan {
   int64_t n = 0;
-  int nb = 1, nseg = 0;
+  int nb = 1, nseg = 0, most = 0;  // most: segments of the block that has most
   DevBuf<int64_t> seg_lo, seg_hi;  // nseg
   DevBuf<int32_t> bseg;            // nb + 1
   DevBuf<int64_t> bptr;            // nb + 1 block offsets
@@ -122,8 +141,7 @@ struct RedPlan {
 // f: the cycle's first step from r.
 template <class T, class F>
 void kr_begin(const RedPlan &R, const T *b, T *x, T *r, F *rf, const FirstStep<F> &f, hipStream_t s);
-void kr_norm(const RedPlan &R, double *sc, bool init, double rtol, KrHost *host, unsigned long long *seq,
-             hipStream_t s);
+void kr_norm(const RedPlan &R, double *sc, bool init, double rtol, const KrSink &to, hipStream_t s);
 template <class T, class C>
 void kr_center(const RedPlan &R, T *z, const C *c, const T *w, hipStream_t s);
 template <class T>

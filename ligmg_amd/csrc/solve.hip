@@ -475,7 +475,7 @@ __global__ void __launch_bounds__(256) k_kr_begin(const T *b, T *x, T *r, F *rf,
 // One wavefront per block: r.r from its partials, the convergence flag, and
 // a copy of both for the host.  init: the first one, where r.r is also b.b.
 __global__ void __launch_bounds__(WAVE) k_kr_norm(const int32_t *bseg, const double *part, double *sc, int init,
-                                                  double rtol, KrHost *host, unsigned long long *seq) {
+                                                  double rtol, KrSink to) {
   __shared__ double q[1][WAVE];
   const int c = blockIdx.x;
   double rr[1];
@@ -488,14 +488,41 @@ __global__ void __launch_bounds__(WAVE) k_kr_norm(const int32_t *bseg, const dou
   }
   S[SC_RN2] = rr[0];
   kr_check(S, rtol);
-  if (!host) return;
-  const unsigned long long k = init ? 1 : seq[c] + 1;
-  seq[c] = k;
-  volatile KrHost *h = host + c;
-  h->rn2 = rr[0];
-  h->active = S[SC_ACTIVE];
-  __threadfence_system();
-  h->seq = k;
+  if (to.host) kr_publish(to, c, init, rr[0], S[SC_ACTIVE]);
+}
+
+// r.r and active flags (their maximum) of many sets.  Each workgroup adds its
+// share, set by set in a fixed order; a grid of one, over the sets themselves
+// (stride SC_N) or the workgroups' pairs (stride 2), publishes the result.
+constexpr int KR_TOTAL_SETS = 4096;  // of a workgroup, at least
+__global__ void __launch_bounds__(1024) k_kr_total(const double *rn2, const double *act, int64_t n, int stride,
+                                                   int init, double *part, KrSink to) {
+  __shared__ double ws[2][1024 / WAVE];
+  const int64_t per = (n + gridDim.x - 1) / gridDim.x, a = blockIdx.x * per, b = min(a + per, n);
+  double t = 0, any = 0;
+#pragma unroll 4
+  for (int64_t i = a + threadIdx.x; i < b; i += 1024) {
+    t += rn2[i * stride];
+    any = max(any, act[i * stride]);
+  }
+  t = wave_sum(t);
+  for (int off = WAVE / 2; off >= 1; off >>= 1) any = max(any, __shfl_xor(any, off, WAVE));
+  if ((threadIdx.x & (WAVE - 1)) == 0) {
+    ws[0][threadIdx.x / WAVE] = t;
+    ws[1][threadIdx.x / WAVE] = any;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < 1024 / WAVE; w++) {
+    t += ws[0][w];
+    any = max(any, ws[1][w]);
+  }
+  if (to.host) {
+    kr_publish(to, 0, init, t, any);
+  } else {
+    part[2 * blockIdx.x] = t;
+    part[2 * blockIdx.x + 1] = any;
+  }
 }
 
 // partials of p.q and, with r set, p.r
@@ -1231,6 +1258,7 @@ void RedPlan::build(int64_t n_, const std::vector<int64_t> &blocks, hipStream_t 
   nb = (int)hbptr.size() - 1;
   std::vector<int64_t> lo, hi;
   std::vector<int32_t> bs(nb + 1, 0), segblk;
+  most = 0;
   for (int c = 0; c < nb; c++) {
     bs[c] = (int32_t)lo.size();
     for (int64_t a = hbptr[c]; a < hbptr[c + 1]; a += seg_rows) {
@@ -1238,6 +1266,7 @@ void RedPlan::build(int64_t n_, const std::vector<int64_t> &blocks, hipStream_t 
       hi.push_back(std::min<int64_t>(a + seg_rows, hbptr[c + 1]));
       segblk.push_back(c);
     }
+    most = std::max(most, (int)lo.size() - bs[c]);
   }
   bs[nb] = (int32_t)lo.size();
   nseg = (int)lo.size();
@@ -1310,10 +1339,26 @@ void kr_begin(const RedPlan &R, const T *b, T *x, T *r, F *rf, const FirstStep<F
   hipLaunchKernelGGL((k_kr_begin<T, F>), LG_SEGS, b, x, r, rf, f, R.seg_lo.p, R.seg_hi.p, R.part.p);
   LG_LAUNCH_CHECK();
 }
-void kr_norm(const RedPlan &R, double *sc, bool init, double rtol, KrHost *host, unsigned long long *seq,
-             hipStream_t s) {
+void kr_norm(const RedPlan &R, double *sc, bool init, double rtol, const KrSink &to, hipStream_t s) {
   hipLaunchKernelGGL(k_kr_norm, dim3((unsigned)R.nb), dim3(WAVE), 0, s, R.bseg.p, (const double *)R.part.p, sc,
-                     init ? 1 : 0, rtol, host, seq);
+                     init ? 1 : 0, rtol, to.each(R.nb));
+  LG_LAUNCH_CHECK();
+  if (to.host && R.nb > KR_HOST_SETS) kr_total(sc, R.nb, init, to, s);
+}
+void kr_total(const double *sc, int64_t sets, bool init, const KrSink &to, hipStream_t s) {
+  const double *rn2 = sc + SC_RN2, *act = sc + SC_ACTIVE;
+  int64_t n = sets;
+  int stride = SC_N;
+  if (n > KR_TOTAL_SETS) {
+    const int64_t groups = std::min<int64_t>((n + KR_TOTAL_SETS - 1) / KR_TOTAL_SETS, KR_TOTAL_PARTS / 2);
+    hipLaunchKernelGGL(k_kr_total, dim3((unsigned)groups), dim3(1024), 0, s, rn2, act, n, stride, 0, to.part, KrSink());
+    LG_LAUNCH_CHECK();
+    rn2 = to.part;
+    act = to.part + 1;
+    n = groups;
+    stride = 2;
+  }
+  hipLaunchKernelGGL(k_kr_total, dim3(1), dim3(1024), 0, s, rn2, act, n, stride, init ? 1 : 0, (double *)nullptr, to);
   LG_LAUNCH_CHECK();
 }
 template <class T>

@@ -5,7 +5,7 @@
 // level solved inside the fused tail produces the bits the separate
 // launches produce.
 #pragma once
-#include "common.hpp"
+#include "ops.hpp"
 
 namespace lg {
 namespace sdev {
@@ -137,8 +137,8 @@ __device__ __forceinline__ double group_sum(double v, int K) {
 
 // ------------------------------------------------- CG / FCG scalar logic
 // One set of scalars per (block, column): the Krylov coefficients of each
-// independent graph are kept apart.
-enum { SC_BN2 = 0, SC_RN2, SC_GAMMA, SC_DELTA, SC_T1, SC_ALPHA, SC_BETA, SC_ACTIVE, SC_GN, SC_N };
+// independent graph are kept apart.  SC_ITS counts a batched set's iterations.
+enum { SC_BN2 = 0, SC_RN2, SC_GAMMA, SC_DELTA, SC_T1, SC_ALPHA, SC_BETA, SC_ACTIVE, SC_GN, SC_ITS, SC_N };
 
 __device__ __forceinline__ void kr_init(double *S) {
   for (int j = 0; j < SC_N; j++) S[j] = 0;
@@ -150,6 +150,16 @@ __device__ __forceinline__ void kr_alpha(double *S, int fcg) {
 }
 __device__ __forceinline__ void kr_check(double *S, double rtol) {
   if (S[SC_ACTIVE] != 0 && !(sqrt(S[SC_RN2]) > rtol * sqrt(S[SC_BN2]))) S[SC_ACTIVE] = 0;
+}
+// a set's norm for the host: the counter last, once the rest is visible
+__device__ __forceinline__ void kr_publish(const KrSink &to, int64_t entry, bool init, double rn2, double active) {
+  const unsigned long long k = init ? 1 : to.seq[entry] + 1;
+  to.seq[entry] = k;
+  volatile KrHost *h = to.host + entry;
+  h->rn2 = rn2;
+  h->active = active;
+  __threadfence_system();
+  h->seq = k;
 }
 __device__ __forceinline__ void kr_beta(double *S, int fcg) {
   if (fcg) {

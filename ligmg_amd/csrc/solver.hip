@@ -142,8 +142,9 @@ struct Solver {
   std::vector<std::pair<std::array<const void *, 9>, hipGraphExec_t>> it_graphs;
   // captured batched iterations, dropped whenever their work buffers move
   std::vector<std::pair<std::array<const void *, 9>, hipGraphExec_t>> bgraphs;
-  PinnedBuf<KrHost> kr_host;         // per block (and column), written by the norm kernels
+  PinnedBuf<KrHost> kr_host;         // written by the norm kernels
   DevBuf<unsigned long long> kr_seq;
+  DevBuf<double> kr_part;
   bool kr_pending = false;           // queued kernels may write kr_host: a solve is running or has failed
   // fused coarse tail: levels tail_l0.. (H.size(): none), the row
   // schedules of their operators (A, P, R, M per level), the device tables
@@ -1311,23 +1312,35 @@ struct Solver {
         kr_update<double, float>(R, x, K.r.p, K.p.p, K.q.p, K.sc.p, fcg, W32[lvl].b.p, first_step<float>(lvl), s);
     }
     if (!f32) kr_update<T, T>(R, x, K.r.p, K.p.p, K.q.p, K.sc.p, fcg, nullptr, first_step<T>(lvl), s);
-    if (norm) kr_norm(R, K.sc.p, false, rtol, outer_solve ? kr_host.p : nullptr, kr_seq.p, s);
+    if (norm) kr_norm(R, K.sc.p, false, rtol, outer_solve ? kr_sink() : KrSink(), s);
   }
 
   // the K-cycle's inner solve
   template <class T>
   void krylov(size_t lvl, const DCsr &A, T *x, const T *b, KWork<T> &K, int type, double rtol, int maxit) {
     kr_begin<T, T>(red[lvl], b, x, K.r.p, nullptr, first_step<T>(lvl), s);
-    kr_norm(red[lvl], K.sc.p, true, rtol, nullptr, nullptr, s);
+    kr_norm(red[lvl], K.sc.p, true, rtol, KrSink(), s);
     for (int it = 0; it < maxit; it++) iterate<T>(lvl, A, x, K, fcg_like(type), rtol, false, it + 1 < maxit);
   }
 
+  KrSink kr_sink() const { return {kr_host.p, kr_seq.p, kr_part.p}; }
+
+  // before an outer solve's first norm; the stream is idle here
+  void kr_reset() {
+    kr_pending = true;
+    kr_host.ensure(KR_HOST_SETS);
+    kr_seq.ensure(KR_HOST_SETS);
+    kr_part.ensure(KR_TOTAL_PARTS);
+    for (int c = 0; c < KR_HOST_SETS; c++) kr_host.p[c].seq = 0;
+    std::atomic_thread_fence(std::memory_order_release);
+  }
+
   // Waits for the seq-th norm of the running outer solve and returns the
-  // residual norm over all blocks; active: whether any block still iterates.
-  double wait_norm(int nb, unsigned long long seq, bool *active) {
+  // residual norm over all sets; active: whether any set still iterates.
+  double wait_norm(int64_t sets, unsigned long long seq, bool *active) {
     double t = 0;
     *active = false;
-    for (int c = 0; c < nb; c++) {
+    for (int c = 0; c < kr_host_entries(sets); c++) {
       volatile KrHost *h = kr_host.p + c;
       for (uint64_t spins = 1; h->seq < seq; spins++) {
         if (spins % 4096) continue;
@@ -1347,14 +1360,10 @@ struct Solver {
     const RedPlan &R = red[lvl];
     const DCsr &A = H[lvl].A;
     const bool fcg = fcg_like(o.outer_ksp_type);
-    kr_pending = true;
-    kr_host.ensure((size_t)R.nb);
-    kr_seq.ensure((size_t)R.nb);
-    for (int c = 0; c < R.nb; c++) kr_host.p[c].seq = 0;  // the stream is idle here
-    std::atomic_thread_fence(std::memory_order_release);
+    kr_reset();
     if (mixed) kr_begin<double, float>(R, b, x, K.r.p, W32[lvl].b.p, first_step<float>(lvl), s);
     else kr_begin<double, double>(R, b, x, K.r.p, nullptr, first_step<double>(lvl), s);
-    kr_norm(R, K.sc.p, true, o.tol, kr_host.p, kr_seq.p, s);
+    kr_norm(R, K.sc.p, true, o.tol, kr_sink(), s);
     *status = LIGMG_CONVERGED;
     bool active = false;
     hist.push_back(wait_norm(R.nb, 1, &active));
@@ -1785,7 +1794,7 @@ struct Solver {
   // with a set of scalars per (block, column)
   template <class T, class F>
   void biterate(size_t lvl, const DCsr &A, T *x, KWork<T> &K, F *rf, int kp, bool fcg, double rtol, bool norm,
-                KrHost *host) {
+                const KrSink &to) {
     const RedPlan &R = bred[lvl];
     const FirstStep<F> f = bfirst_step<F>(lvl);
     const F *r = rf;
@@ -1808,61 +1817,46 @@ struct Solver {
     op_kr_bupdate<T, F>(R, x, K.r.p, K.p.p, K.q.p, rf, f, kp, K.sc.p, bpart_red, s);
     if (!norm) return;
     P.kind = BlockPost::NORM;
-    P.host = host;
-    P.seq = kr_seq.p;
+    P.to = to;
     R.bfinish(1, kp, P, bpart_red, s);
   }
 
   template <class T, class F>
-  void bbegin(size_t lvl, const T *b, T *x, KWork<T> &K, F *rf, int kp, double rtol, KrHost *host) {
+  void bbegin(size_t lvl, const T *b, T *x, KWork<T> &K, F *rf, int kp, double rtol, const KrSink &to) {
     const RedPlan &R = bred[lvl];
     op_kr_bbegin<T, F>(R, b, x, K.r.p, rf, bfirst_step<F>(lvl), kp, bpart_red, s);
     BlockPost P;
     P.kind = BlockPost::INIT;
     P.sc = K.sc.p;
     P.rtol = rtol;
-    P.host = host;
-    P.seq = kr_seq.p;
+    P.to = to;
     R.bfinish(1, kp, P, bpart_red, s);
   }
 
   // the K-cycle's inner solve
   template <class T>
   void bkrylov(size_t lvl, const DCsr &A, T *x, const T *b, KWork<T> &K, int kp, int type, double rtol, int maxit) {
-    bbegin<T, T>(lvl, b, x, K, nullptr, kp, rtol, nullptr);
+    bbegin<T, T>(lvl, b, x, K, nullptr, kp, rtol, KrSink());
     for (int it = 0; it < maxit; it++)
-      biterate<T, T>(lvl, A, x, K, nullptr, kp, fcg_like(type), rtol, it + 1 < maxit, nullptr);
+      biterate<T, T>(lvl, A, x, K, nullptr, kp, fcg_like(type), rtol, it + 1 < maxit, KrSink());
   }
 
-  // the outer solve; its[t] receives the iteration set t = (block, column)
-  // converged at
-  int bkrylov_solve(size_t lvl, double *x, const double *b, KWork<double> &K, int kp, std::vector<int> &its,
-                    int *status) {
+  // the outer solve; SC_ITS of a set is the iteration it converged at
+  int bkrylov_solve(size_t lvl, double *x, const double *b, KWork<double> &K, int kp, int *status) {
     const DCsr &A = H[lvl].A;
-    const int ns = bred[lvl].nb * kp;
+    const int64_t ns = (int64_t)bred[lvl].nb * kp;
     const bool fcg = fcg_like(o.outer_ksp_type);
-    kr_pending = true;
-    kr_host.ensure((size_t)ns);
-    kr_seq.ensure((size_t)ns);
-    for (int t = 0; t < ns; t++) kr_host.p[t].seq = 0;  // the stream is idle here
-    std::atomic_thread_fence(std::memory_order_release);
+    kr_reset();
     auto body = [&] {
-      if (mixed) biterate<double, float>(lvl, A, x, K, BW32[lvl].b.p, kp, fcg, o.tol, true, kr_host.p);
-      else biterate<double, double>(lvl, A, x, K, nullptr, kp, fcg, o.tol, true, kr_host.p);
+      if (mixed) biterate<double, float>(lvl, A, x, K, BW32[lvl].b.p, kp, fcg, o.tol, true, kr_sink());
+      else biterate<double, double>(lvl, A, x, K, nullptr, kp, fcg, o.tol, true, kr_sink());
     };
-    if (mixed) bbegin<double, float>(lvl, b, x, K, BW32[lvl].b.p, kp, o.tol, kr_host.p);
-    else bbegin<double, double>(lvl, b, x, K, nullptr, kp, o.tol, kr_host.p);
-    its.assign(ns, 0);
-    std::vector<char> was(ns, 1);
+    if (mixed) bbegin<double, float>(lvl, b, x, K, BW32[lvl].b.p, kp, o.tol, kr_sink());
+    else bbegin<double, double>(lvl, b, x, K, nullptr, kp, o.tol, kr_sink());
     *status = LIGMG_CONVERGED;
     for (int it = 0;; it++) {
       bool active = false;
       const double tn = wait_norm(ns, (unsigned long long)it + 1, &active);
-      for (int t = 0; t < ns; t++) {
-        const bool act = kr_host.p[t].active != 0;
-        if (it > 0 && (was[t] || act)) its[t] = it;
-        was[t] = act;
-      }
       if (it > 0 && tn != tn) {
         *status = LIGMG_DIVERGED_NAN;
         return it;
@@ -1938,9 +1932,8 @@ int Solver::solve_batch(int k, const double *Bin, double *Xout, int mem, ligmg_i
   else d2d(rhs.p, b0b.p, n * kp, s);
   bred[base].bdots<double>(1, kp, rhs.p, nullptr, nullptr, nullptr, bsc_out.p, bpart_red, s);
   op_bsub_block_mean<double>(rhs.p, kp, bred[base], bsc_out.p, s);
-  std::vector<int> its;
   int status = 0;
-  const int iters = bkrylov_solve(base, bouter.x.p, rhs.p, bouter, kp, its, &status);
+  const int iters = bkrylov_solve(base, bouter.x.p, rhs.p, bouter, kp, &status);
   kr_pending = false;  // every norm has arrived
   if (do_once) op_binterp<double>(L0.P, L0.q.p, bouter.x.p, b0b.p, solb.p, kp, bparts, s);
   else d2d(solb.p, bouter.x.p, n * kp, s);
@@ -1963,11 +1956,13 @@ int Solver::solve_batch(int k, const double *Bin, double *Xout, int mem, ligmg_i
   if (mem == LIGMG_MEM_HOST) to_host(Xout, bin.p, n * k, s);
   else d2d(Xout, bin.p, n * k, s);
   LG_HIP(hipStreamSynchronize(s));
+  std::vector<double> hsc;
+  if (iters_out || info) hsc = download(bouter.sc.p, (size_t)red[base].nb * kp * SC_N, s);
   if (iters_out) {
     const int nb = red[base].nb;
     for (int c = 0; c < k; c++) {
       int m = 0;
-      for (int blk = 0; blk < nb; blk++) m = std::max(m, its[(size_t)blk * kp + c]);
+      for (int blk = 0; blk < nb; blk++) m = std::max(m, (int)hsc[((size_t)blk * kp + c) * SC_N + SC_ITS]);
       iters_out[c] = m;
     }
   }
@@ -1980,7 +1975,6 @@ int Solver::solve_batch(int k, const double *Bin, double *Xout, int mem, ligmg_i
     info->time = std::chrono::duration<double>(t1 - t0).count();
     info->setup_time = setup_time;
     // worst reduced-system relative residual over (block, column) sets
-    std::vector<double> hsc = download(bouter.sc.p, (size_t)red[base].nb * kp * SC_N, s);
     double rel = 0;
     for (int t = 0; t < red[base].nb * kp; t++) {
       double bn = hsc[t * SC_N + SC_BN2];

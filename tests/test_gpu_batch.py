@@ -178,3 +178,39 @@ def test_batch_hub_rows_and_segments(k, prec):
     for c in {0, k // 2, k - 1}:
         one = s.solve(np.ascontiguousarray(B[:, c]))
         assert rel(X[0][:, c], one.solution) <= 1e-7 and abs(int(its[c]) - one.iters()) <= 1
+
+
+@pytest.mark.parametrize("sizes,k", [([40] * 2, 64), ([40] * 43, 3), ([30] * 64, 64), ([30] * 65, 64), ([12] * 600, 33),
+                                     ([2048], 64), ([2049], 64), ([2049] + [30] * 200, 64), ([30] * 129, 1)])
+@pytest.mark.parametrize("prec", [_ffi.PREC_FP64, _ffi.PREC_MIXED])
+def test_batch_many_sets(sizes, k, prec):
+    """Sets (graph, column) on both sides of 128, where the norms reach the
+    host one by one, of 4096, one workgroup's share of their sum, and blocks
+    of 16 and 17 segments of 128 rows (64 columns): counts, norms and
+    solutions of the single solves, whose blocks are checked one by one."""
+    print(f"{len(sizes)} graphs k={k} prec={prec}", flush=True)
+    u = graphs.union([graphs.barabasi_albert(n, 3, seed=i) for i, n in enumerate(sizes)])
+    s = ligmg_amd.Solver(u, ligmg_amd.Options(precision=prec, outer_ksp_type=_ffi.KSP_FCG), comp_ptr=u.comp_ptr)
+    B = graphs.rhs(u.n, k, 7, comp_ptr=u.comp_ptr).reshape(u.n, k, order="F")
+    X, info, its = s.solve_batch(B)
+    assert info.status == _ffi.CONVERGED and info.rel_residual <= 1e-8 and its.max() == info.iters
+    R = np.add.reduceat((B - u.to_scipy() @ X) ** 2, u.comp_ptr[:-1], axis=0)
+    assert (R <= 1e-14 * np.add.reduceat(B ** 2, u.comp_ptr[:-1], axis=0)).all()
+    for c in {0, k // 2, k - 1}:
+        one = s.solve(np.ascontiguousarray(B[:, c]))
+        assert one.status == _ffi.CONVERGED and abs(int(its[c]) - one.iters()) <= 1
+        assert len(one.residuals) == one.iters() + 1 and one.residuals[-1] <= 1e-8 * one.residuals[0]
+        assert np.linalg.norm(X[:, c] - one.solution) <= 1e-7 * np.linalg.norm(one.solution)
+
+
+def test_batch_of_many_graphs_costs_its_columns():
+    """64 columns of 3000 small graphs take about 5 times as long as one; with
+    every set's norm written to the host on its own it was 80 times."""
+    u = graphs.union([graphs.barabasi_albert(60, 3, seed=i) for i in range(3000)])
+    s = ligmg_amd.Solver(u, ligmg_amd.Options(precision=_ffi.PREC_MIXED, outer_ksp_type=_ffi.KSP_FCG), comp_ptr=u.comp_ptr)
+    t = {}
+    for k in (1, 64):
+        B = graphs.rhs(u.n, k, 7, comp_ptr=u.comp_ptr).reshape(u.n, k, order="F")
+        t[k] = min(s.solve_batch(B)[1].time for _ in range(4))
+    print(f"1 column {t[1] * 1e3:.2f} ms, 64 columns {t[64] * 1e3:.2f} ms")
+    assert t[64] <= 25 * t[1]
