@@ -273,6 +273,14 @@ int ligmg_dump_csv(ligmg_handle h, const char *graph, const ligmg_info *info, ch
  * *out down run in one launch per coarse-grid correction; *out equals the
  * number of levels when nothing is fused. */
 int ligmg_tail_start(ligmg_handle h, int32_t *out);
+/* (new) Diagnostic: what setup chose for a level's solve phase.  layout: 0
+ * the setup order, 1 degree order, 2 cluster order (solve_layout);
+ * row_lanes: lanes per row where the level matrix's SpMV goes row by row, 0
+ * where it goes by staged units; segments: the most segments of one block in
+ * the vector reductions; dense: 1 at the level from which V-cycles are one
+ * dense matrix. */
+int ligmg_level_plan(ligmg_handle h, int32_t level, int32_t *layout,
+                     int32_t *row_lanes, int32_t *segments, int32_t *dense);
 int ligmg_setup_time(ligmg_handle h, double *out);
 int ligmg_level_info(ligmg_handle h, int32_t level, int32_t *kind, int64_t *n,
                      int64_t *nnz, int64_t *n_coarse);

@@ -99,6 +99,7 @@ SOLVER_PROTOS = {
     "ligmg_dump_hierarchy": (C.c_int, [HANDLE, C.c_char_p]),
     "ligmg_load_hierarchy": (C.c_int, [C.c_char_p, P(ligmg_options), P(HANDLE)]),
     "ligmg_dump_csv": (C.c_int, [HANDLE, C.c_char_p, P(ligmg_info), C.c_char_p, i64]),
+    "ligmg_level_plan": (C.c_int, [HANDLE, i32, P(i32), P(i32), P(i32), P(i32)]),
     "ligmg_setup_time": (C.c_int, [HANDLE, P(f64)]),
     "ligmg_level_info": (C.c_int, [HANDLE, i32, P(i32), P(i64), P(i64), P(i64)]),
     "ligmg_level_matrix": (C.c_int, [HANDLE, i32, P(i32), P(i32), P(f64)]),

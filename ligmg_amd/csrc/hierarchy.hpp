@@ -130,9 +130,11 @@ struct DLevel {
   // Solve layout: the solve-phase copies (A, dinv, agg, M, P, R, q) of a
   // large level are renumbered inside blocks, by descending degree or, where
   // rows are even, cluster by cluster; sperm maps a solve position to the
-  // setup position (empty: setup order kept), siperm is its inverse.  agg_setup / new_id keep the setup-order maps for
-  // introspection; new_id_s is new_id in solve order.
+  // setup position (empty: setup order kept), siperm is its inverse.
+  // agg_setup / new_id keep the setup-order maps for introspection; new_id_s
+  // is new_id in solve order.
   DevBuf<int32_t> sperm, siperm, agg_setup, new_id_s;
+  int layout = 0;  // sperm is: 0 empty, 1 the degree order, 2 the cluster order
   std::vector<int64_t> blocks;  // contiguous vertex blocks (independent graphs)
 };
 

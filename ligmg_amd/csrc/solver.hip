@@ -700,12 +700,15 @@ struct Solver {
         H[l].sperm.alloc(H[l].A.n);
         d2d(H[l].sperm.p, pm.p, H[l].A.n, s);
         H[l].siperm = std::move(ip);
+        H[l].layout = 2;
       }
       perm_c = std::move(pm);
     }
     for (size_t l = 0; l + 1 < nl; l++)
-      if (H[l].A.n >= SOLVE_PERM_MIN && !H[l].sperm.p)
+      if (H[l].A.n >= SOLVE_PERM_MIN && !H[l].sperm.p) {
         degree_perm(H[l].A, H[l].blocks, H[l].sperm, H[l].siperm, s);
+        H[l].layout = 1;
+      }
     for (size_t l = 0; l + 1 < nl; l++) {
       DLevel &V = H[l];
       const DLevel &N = H[l + 1];
@@ -2385,6 +2388,17 @@ int ligmg_num_levels(ligmg_handle h, int32_t *out) {
 int ligmg_tail_start(ligmg_handle h, int32_t *out) {
   if (!h || !out) return LIGMG_ERR_INVALID;
   *out = (int32_t)h->S.tail_l0;
+  return LIGMG_OK;
+}
+
+int ligmg_level_plan(ligmg_handle h, int32_t l, int32_t *layout, int32_t *row_lanes, int32_t *segments,
+                     int32_t *dense) {
+  if (!h || l < 0 || l >= (int)h->S.H.size() || !layout || !row_lanes || !segments || !dense) return LIGMG_ERR_INVALID;
+  const lg::Solver &S = h->S;
+  *layout = S.H[l].layout;
+  *row_lanes = S.H[l].A.U.row_k;
+  *segments = S.red[l].most;
+  *dense = (size_t)l == S.dense_l0 ? 1 : 0;
   return LIGMG_OK;
 }
 

@@ -287,6 +287,13 @@ class Solver:
         _check(self._lib.ligmg_tail_start(self._h, C.byref(n)), "ligmg_tail_start")
         return n.value
 
+    def level_plan(self, l):
+        """What setup chose for the level's solve phase: (layout, row_lanes,
+        segments, dense), see ligmg_level_plan."""
+        v = [C.c_int32() for _ in range(4)]
+        _check(self._lib.ligmg_level_plan(self._h, l, *(C.byref(x) for x in v)), "ligmg_level_plan")
+        return tuple(x.value for x in v)
+
     def level_info(self, l):
         k, n, nnz, nc = C.c_int32(), C.c_int64(), C.c_int64(), C.c_int64()
         _check(self._lib.ligmg_level_info(self._h, l, C.byref(k), C.byref(n), C.byref(nnz),

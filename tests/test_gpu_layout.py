@@ -32,6 +32,13 @@ def test_cluster_layout_is_invisible(name, g, prec):
     a = ligmg_amd.Solver(g, ligmg_amd.Options(**kw))
     b = ligmg_amd.Solver(g, ligmg_amd.Options(solve_layout=0, **kw))
     assert a.num_levels() == b.num_levels()
+    # the order each is there for: degree order where a row is longer than 8
+    # mean ones, cluster order where none is
+    layouts = [a.level_plan(l)[0] for l in range(a.num_levels())]
+    rows = [np.diff(a.level_matrix(l)[0]) for l in range(a.num_levels() - 1)]
+    assert layouts == [0 if len(r) < 1 << 16 else 1 if r.max() > 8 * r.mean() else 2 for r in rows] + [0]
+    assert layouts[0] == (1 if name == "hub" else 2)
+    assert not any(b.level_plan(l)[0] for l in range(b.num_levels()))
     rng = np.random.default_rng(3)
     for l in range(a.num_levels()):
         assert a.level_info(l) == b.level_info(l)

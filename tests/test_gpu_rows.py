@@ -1,6 +1,6 @@
 """The row-kernel SpMV (groups of lanes straight from memory) and the rule
-that picks it, against scipy: mean row lengths on both sides of every lane
-count, and longest rows on both sides of its limit."""
+that picks it, against scipy: mean row lengths of several lane counts, and
+longest rows on both sides of the limit of 32 entries a lane."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -20,12 +20,15 @@ def ring(n, reach, hub):
     return graphs.from_edges(n, u, v, w)
 
 
-@pytest.mark.parametrize("n,reach,hub", [(9, 1, 0), (300, 1, 25), (257, 3, 0), (500, 4, 60), (500, 4, 200),
-                                         (1500, 8, 120), (1500, 8, 200), (2000, 20, 1900), (700, 300, 0)])
-def test_level_spmv_rows(n, reach, hub):
+@pytest.mark.parametrize("n,reach,hub,lanes", [(9, 1, 0, 1), (300, 1, 25, 1), (300, 1, 29, 1), (300, 1, 30, 0), (257, 3, 0, 2),
+                                               (500, 4, 60, 4), (500, 4, 119, 4), (500, 4, 120, 0), (500, 4, 200, 0),
+                                               (1500, 8, 120, 8), (1500, 8, 200, 8), (1500, 8, 239, 8), (1500, 8, 240, 0),
+                                               (2000, 20, 1900, 0), (700, 300, 0, 64)])
+def test_level_spmv_rows(n, reach, hub, lanes):
     g = ring(n, reach, hub)
     s = ligmg_amd.Solver(g, ligmg_amd.Options(precision=_ffi.PREC_MIXED, elim_degree=0, always_elim=0))
     rp, ci, v = s.level_matrix(0)
+    assert s.level_plan(0)[1] == lanes  # the kernel this case is there for
     A = sp.csr_matrix((v, ci, rp), shape=(n, n))
     x = np.random.default_rng(0).standard_normal(n)
     bound = abs(A) @ abs(x) * np.diff(rp).max()  # one rounding per term
