@@ -359,7 +359,13 @@ __global__ void k_dense_apply(const double *__restrict__ Pm, int64_t n, const T 
 // Dot-product segment: one workgroup each.  4096 (not 16384) gives mid-size
 // vectors enough workgroups (R-MAT 22 K-cycle 0.408 -> 0.359 s, batched 160^3
 // grid 61 -> 50 ms per right-hand side).
+// From 8.4 M rows they are longer, whole batches of a workgroup each: the
+// Krylov kernels add their block's partials in every workgroup
+// (block_partials), so with 4096 rows whatever the size that work grew with
+// the square of it (20 iterations on a grid of 25 M vertices 101.5 -> 98.1 ms,
+// 49 M 195 -> 187 ms).
 constexpr int RED_CHUNK = 4096;
+constexpr int RED_MAX_SEGS = 2048;
 
 // Items lo + vt, lo + vt + 256, ... of a segment in batches of RED_BATCH:
 // load(t, i) asks for item i into slot t (past the end: the last item), then
@@ -1251,7 +1257,10 @@ LG_INST(float)
 #undef LG_INST
 
 void RedPlan::build(int64_t n_, const std::vector<int64_t> &blocks, hipStream_t s, int64_t seg_rows) {
-  if (seg_rows <= 0) seg_rows = RED_CHUNK;
+  if (seg_rows <= 0) {
+    constexpr int64_t step = 256 * RED_BATCH;
+    seg_rows = std::max<int64_t>(RED_CHUNK, ((n_ + RED_MAX_SEGS - 1) / RED_MAX_SEGS + step - 1) / step * step);
+  }
   n = n_;
   hbptr = blocks;
   if (hbptr.size() < 2) hbptr = {0, n};

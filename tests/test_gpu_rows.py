@@ -34,3 +34,19 @@ def test_level_spmv_rows(n, reach, hub, lanes):
     bound = abs(A) @ abs(x) * np.diff(rp).max()  # one rounding per term
     assert (np.abs(s.level_spmv(0, x) - A @ x) <= 2.0 ** -52 * bound).all()
     assert (np.abs(s.level_spmv(0, x, _ffi.PREC_MIXED) - A @ x) <= 4 * 2.0 ** -24 * (abs(A) @ abs(x))).all()
+
+
+@pytest.mark.parametrize("nx", [2896, 2900])
+def test_reduction_segments_are_capped(nx):
+    """8,386,816 and 8,410,000 vertices, on both sides of 2048 segments of
+    4096 rows: a block never has more, and the norms are numpy's."""
+    g = graphs.grid2d(nx, nx)
+    s = ligmg_amd.Solver(g, ligmg_amd.Options(always_elim=0, top_elim=0, iters=2))
+    n = s.level_info(0)[1]
+    assert n == g.n and s.level_plan(0)[2] == (2048 if nx == 2896 else -(-n // 6144))
+    b = graphs.rhs(n, 1, 0)
+    info = s.solve(b)
+    r = b - g.to_scipy() @ info.solution
+    assert info.residuals[0] == pytest.approx(np.linalg.norm(b), rel=1e-12)
+    assert info.residuals[-1] == pytest.approx(np.linalg.norm(r), rel=1e-7)  # recurrence and true residual
+    assert info.full_rel_residual == pytest.approx(np.linalg.norm(r) / np.linalg.norm(b), rel=1e-9)
