@@ -136,7 +136,9 @@ typedef struct ligmg_options {
                                    hold at most this many stored entries
                                    (with every coarser level) run as one
                                    single-workgroup launch per coarse-grid
-                                   correction, same results; 0: off         */
+                                   correction, same results (V-cycles: no
+                                   level above those that are one dense
+                                   matrix); 0: off                          */
   double rejection_ratio;       /* -1: conductance rejection off; >= 0: in the
                                    second half of the voting rounds, joined
                                    vertices whose external / internal edge

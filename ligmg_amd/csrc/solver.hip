@@ -751,7 +751,7 @@ struct Solver {
   // ------------------------------------------------------ fused coarse tail
   // A level joins the tail when its solve operators hold at most
   // o.tail_nnz entries; the tail is the longest run of such levels that
-  // ends at the coarsest one.
+  // ends at the coarsest one, from the collapsed level on where there is one.
   bool tail_ok(const DLevel &L) const {
     const int64_t lim = o.tail_nnz;
     auto unsliced = [](const DCsr &A) { return A.slices[0].size() <= 1 && A.slices[1].size() <= 1; };
@@ -889,9 +889,9 @@ struct Solver {
   const T *rec_cycle(std::vector<TailInstr> &c, size_t l, const T *b) {
     DLevel &L = H[l];
     LevelWork<T> &w = work<T>(l);
-    if (L.kind == LIGMG_LEVEL_COARSE || l == dense_l0) {
+    if (L.kind == LIGMG_LEVEL_COARSE) {
       TailInstr I = ti(TI_DENSE, L.A.n);
-      I.p[0] = l == dense_l0 ? dense_m.p : L.pinv.p;
+      I.p[0] = L.pinv.p;
       I.p[1] = b;
       I.p[2] = w.B[0].p;
       c.push_back(I);
@@ -1077,14 +1077,17 @@ struct Solver {
     // bounded program size (a deep K-cycle tail grows geometrically)
     while (l0 < nl && tail_count(l0 - 1) > TAIL_MAX_INSTR) l0++;
     if (l0 >= nl) return;
-    tail_l0 = l0;
-    // a tail that starts at the collapsed level or below is only entered by
-    // solves and cycles from there (need_tail)
-    if (tail_l0 < dense_l0) record_tail();
+    // Never above the collapsed level, whose product the tail's one workgroup
+    // would stream alone (a 256 x 256 grid with tail_nnz = 65536: the solve 177
+    // ms with the product in the tail, 38 with its levels there instead, 6.0
+    // with the tail from the collapsed level on).  Such a tail is only entered
+    // by solves and cycles from below it, which record it (need_tail).
+    tail_l0 = dense_l0 < nl ? std::max(l0, dense_l0) : l0;
+    if (dense_l0 == nl) record_tail();
   }
 
-  // Called before a cycle from level lvl: its corrections enter the tail
-  // where the collapsed level does not come first.
+  // Called before a cycle from level lvl: below the collapsed level its
+  // corrections enter the tail.
   void need_tail(size_t lvl) {
     if (lvl > dense_l0 && tail_l0 < H.size() && tail_sched.empty()) record_tail();
   }

@@ -100,3 +100,28 @@ def test_tail_graph_replays_and_repeat_solves():
         assert np.array_equal(again.residuals, first.residuals)
     eager = ligmg_amd.Solver(g, ligmg_amd.Options(tail_nnz=1 << 15, use_graphs=0, kcycle=1, **FCG))
     assert np.array_equal(eager.solve(b).solution, first.solution)
+
+
+@pytest.mark.parametrize("name,tail_nnz", [("grid", 4096), ("grid", 1 << 15), ("grid", 1 << 16), ("grid", 1 << 17),
+                                           ("grid3d", 1 << 15), ("grid3d", 1 << 17), ("grid3d", 1 << 20)])
+@pytest.mark.parametrize("prec", [_ffi.PREC_FP64, _ffi.PREC_MIXED])
+def test_tail_above_the_dense_cycle(name, prec, tail_nnz):
+    """A V-cycle's tail never holds a level above the collapsed one, whose
+    product one workgroup would stream alone there.  The same bits as without
+    a tail, from every level, and no time lost."""
+    g = graphs.grid2d(200, 190) if name == "grid" else graphs.grid3d(31, 33, 35)
+    on, off = pair(g, tail_nnz, precision=prec, **FCG)
+    dense = [l for l in range(on.num_levels()) if on.level_plan(l)[3]]
+    assert len(dense) == 1
+    n = on.level_info(dense[0])[1]
+    print(f"{name} {tail_nnz}: {on.num_levels()} levels, dense from {dense[0]} ({n}), tail from {on.tail_start()}", flush=True)
+    assert on.tail_start() >= dense[0]
+    base = 1 if on.level_info(0)[0] == _ffi.LEVEL_ELIM else 0
+    for l in range(base, on.num_levels()):
+        m = on.level_info(l)[1]
+        u = graphs.rhs(m, 1, 7)
+        assert np.array_equal(on.apply_cycle(l, u), off.apply_cycle(l, u)), l
+    b = graphs.rhs(g.n, 1, 0)
+    same_solve(on, off, b)
+    t_on, t_off = (min(s.solve(b).time() for _ in range(3)) for s in (on, off))
+    assert t_on <= 2 * t_off, (t_on, t_off)
