@@ -214,3 +214,31 @@ def test_batch_of_many_graphs_costs_its_columns():
         t[k] = min(s.solve_batch(B)[1].time for _ in range(4))
     print(f"1 column {t[1] * 1e3:.2f} ms, 64 columns {t[64] * 1e3:.2f} ms")
     assert t[64] <= 25 * t[1]
+
+
+@pytest.mark.parametrize("kw", [{}, {"precision": _ffi.PREC_MIXED, "outer_ksp_type": _ffi.KSP_FCG},
+                                {"kcycle": 1, "outer_ksp_type": _ffi.KSP_FCG}])
+def test_batch_alternating_widths(kw):
+    """A handle keeps the buffers of its widest batch and each width's
+    captured iteration: widths in any order give a fresh handle's bits, and
+    taking turns costs about what each width costs by itself."""
+    import time
+    g = graphs.barabasi_albert(3000, 3, seed=1)
+    B = graphs.rhs(g.n, 64, 11).reshape(g.n, 64, order="F")
+    ref = {k: ligmg_amd.Solver(g, ligmg_amd.Options(**kw)).solve_batch(B[:, :k])[0] for k in (1, 3, 16, 33, 64)}
+    s = ligmg_amd.Solver(g, ligmg_amd.Options(**kw))
+    for k in (3, 16, 3, 64, 33, 1, 16, 64, 3):
+        assert np.array_equal(s.solve_batch(B[:, :k])[0], ref[k]), k
+
+    def seconds(ks):
+        t = []
+        for _ in range(9):
+            t0 = time.perf_counter()
+            for k in ks:
+                s.solve_batch(B[:, :k])
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    alone, turns = seconds([3] * 4) + seconds([16] * 4), seconds([3, 16] * 4)
+    print(f"{kw}: by itself {alone * 1e3:.2f} ms, in turn {turns * 1e3:.2f} ms")
+    assert turns <= 1.1 * alone
