@@ -162,7 +162,9 @@ typedef struct ligmg_info {
   int32_t base_level;          /* 1 when the level-0 elimination was applied   */
   double rel_residual;         /* last / first of the reduced-system history   */
   double full_rel_residual;    /* ||b - L x|| / ||b|| on the caller's system   */
-  double time;                 /* solve wall time (s)                          */
+  double time;                 /* solve wall time (s) from the right-hand      */
+                               /* side's arrival in device memory to the       */
+                               /* solution's presence there                    */
   double work;                 /* iters * (1 + cycle complexity)               */
   double cycle_complexity;     /* work / iters                                 */
   double cf, ecf, wda;

@@ -2084,20 +2084,14 @@ int Solver::solve(const double *b, double *x, int mem, ligmg_info *info, double 
   // caller order -> solve layout: the input permutation and level 0's
   // layout for level 0, the level's own layout below it
   const int32_t *ip = from == 0 ? perm.p : L0.sperm.p;
-  LG_HIP(hipStreamSynchronize(s));  // idle, unless an earlier solve failed
-  if (ip) {
-    const double *src = b;
-    if (mem == LIGMG_MEM_HOST) {
-      to_device(tmp0.p, b, n, s);
-      src = tmp0.p;
-    }
-    gather_vec(n, ip, src, b0.p, s);
-  } else if (mem == LIGMG_MEM_HOST) {
-    to_device(b0.p, b, n, s);
-  } else {
-    d2d(b0.p, b, n, s);
-  }
+  const bool host = mem == LIGMG_MEM_HOST;
+  if (host) to_device(ip ? tmp0.p : b0.p, b, n, s);
+  // info->time counts from b's arrival on the device, as a batch's does; idle
+  // also where an earlier solve failed
+  LG_HIP(hipStreamSynchronize(s));
   auto t0 = std::chrono::steady_clock::now();
+  if (ip) gather_vec(n, ip, host ? tmp0.p : b, b0.p, s);
+  else if (!host) d2d(b0.p, b, n, s);
   const bool do_once = o.top_elim && L0.kind == LIGMG_LEVEL_ELIM;
   const size_t base = do_once ? (size_t)from + 1 : (size_t)from;
   const DLevel &B = H[base];

@@ -362,6 +362,22 @@ def test_device_resident_inputs():
     assert np.array_equal(info.solution.cpu().numpy(), xh)
 
 
+def test_solve_time_excludes_the_transfers():
+    """info.time is the solve's own: the same for a right-hand side on the host,
+    and for a pinned one, whose copy is asynchronous and takes about as long as
+    these two iterations."""
+    import torch
+    g = graphs.grid2d(2000, 2000)
+    s = ligmg_amd.Solver(g, ligmg_amd.Options(iters=2))
+    b = graphs.rhs(g.n, 1, 0)
+    d = torch.from_numpy(b).cuda()
+    pinned = torch.from_numpy(b).pin_memory().numpy()
+    t_host, t_pinned, t_dev = (min(s.solve(x).time() for _ in range(5)) for x in (b, pinned, d))
+    print(f"host {t_host * 1e3:.3f} ms, pinned {t_pinned * 1e3:.3f} ms, device {t_dev * 1e3:.3f} ms")
+    assert max(t_host, t_pinned) <= 1.15 * t_dev
+
+
+
 def test_blocks_solve_independently():
     gs = [graphs.barabasi_albert(n, 4, seed=s) for s, n in enumerate([3000, 800, 5000])]
     u = graphs.union(gs)
