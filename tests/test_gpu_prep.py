@@ -159,3 +159,24 @@ def test_prep_entry_chunks(n, hub, diagonal):
     dn[int(keep[0])] = len(keep)
     torch.cuda.synchronize()
     assert lib.ligmg_extract(*args, orp.data_ptr(), oci.data_ptr(), ov.data_ptr()) == _ffi.ERR_INVALID
+
+
+@pytest.mark.parametrize("scale", [14, 15, 16, 17])
+def test_prep_chunk_sizes(scale):
+    """Entry counts whose passes take chunks of 128 to 1024 entries (64 is in
+    the cases above), with hubs that cross many of them."""
+    import torch
+    A = adjacency_of(graphs.rmat_config(scale, "lognormal", pendants=True))
+    assert (1 << 18) << (scale - 14) < A.nnz and (scale == 17 or A.nnz <= (1 << 19) << (scale - 14))
+    print(f"scale={scale} n={A.shape[0]} nnz={A.nnz}", flush=True)
+    n, (rp, ci, v) = A.shape[0], (A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data)
+    d = tuple(torch.from_numpy(a).cuda() for a in (rp, ci, v))
+    lab, k = prep.components(d)
+    nc, c = sp.csgraph.connected_components(A, directed=False)
+    top = np.full(nc, -1)
+    np.maximum.at(top, c, np.arange(n))
+    assert k == nc and np.array_equal(lab.cpu().numpy(), top[c])
+    for got, want in ((prep.adjacency_to_laplacian(d), O.adjacency_to_laplacian(rp, ci, v)),
+                      (prep.largest_component(d), O.largest_component(rp, ci, v))):
+        for a, b in zip(got, want):
+            assert np.array_equal(a.cpu().numpy(), b)
