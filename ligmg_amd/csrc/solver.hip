@@ -66,14 +66,16 @@ template <class T>
 struct KWork {
   DevBuf<T> r, z, p, q, x;
   DevBuf<double> sc, out;
+  // x is allocated last and released first: where it is large enough, all are
   void alloc(int64_t n, int nb) {
+    x.release();
     r.alloc(n);
     z.alloc(n);
     p.alloc(n);
     q.alloc(n);
-    x.alloc(n);
     sc.alloc((size_t)nb * SC_N);
     out.alloc((size_t)nb * 4);
+    x.alloc(n);
   }
 };
 

@@ -127,3 +127,25 @@ def test_close_while_the_application_captures(mode, other):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.all(z == 2.0 * (rep + 1))
+
+
+def test_batch_after_one_that_did_not_fit():
+    """A batch for which memory runs out is refused, and the next narrower
+    one does not take the buffers it left half allocated."""
+    import torch
+    g = graphs.barabasi_albert(200000, 4, seed=1)
+    s = ligmg_amd.Solver(g)
+    B = graphs.rhs(g.n, 64, 0).reshape(g.n, 64, order="F")
+    ref = s.solve_batch(B[:, :3])[0]
+    ligmg_amd.trim_memory()
+    torch.cuda.empty_cache()
+    hold = torch.empty(torch.cuda.mem_get_info()[0] - (1 << 30), dtype=torch.uint8, device="cuda")
+    print(f"holding {hold.numel() >> 30} GiB", flush=True)
+    with pytest.raises(ligmg_amd.LigmgError) as e:
+        s.solve_batch(B)
+    assert e.value.code == _ffi.ERR_NOMEM
+    assert np.array_equal(s.solve_batch(B[:, :3])[0], ref)
+    del hold
+    torch.cuda.empty_cache()
+    X = s.solve_batch(B)[0]
+    assert np.linalg.norm(X[:, :3] - ref) <= 1e-7 * np.linalg.norm(ref)
