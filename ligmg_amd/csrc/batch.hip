@@ -1133,13 +1133,13 @@ void op_kr_bpupdate(T *p, const T *z, int kp, const RedPlan &P, const double *sc
                                       DevBuf<double> &, hipStream_t) const;                          \
   template void RedPlan::bdots<T>(int, int, const T *, const T *, const T *, const T *, double *,    \
                                   DevBuf<double> &, hipStream_t) const;                              \
-  template void op_bsub_block_mean<T>(T *, int, const RedPlan &, const double *, hipStream_t);         \
   template void op_bspmv_first<T>(const DCsr &, const T *, T *, const FirstStep<T> &, int,             \
                                   DevBuf<double> &, hipStream_t);                                    \
   template void op_kr_bpupdate<T>(T *, const T *, int, const RedPlan &, const double *, hipStream_t);
 LG_BINST(double)
 LG_BINST(float)
 #undef LG_BINST
+template void op_bsub_block_mean<double>(double *, int, const RedPlan &, const double *, hipStream_t);
 #define LG_BKR(T, F)                                                                                            \
   template void op_kr_bbegin<T, F>(const RedPlan &, const T *, T *, T *, F *, const FirstStep<F> &, int,        \
                                    DevBuf<double> &, hipStream_t);                                             \

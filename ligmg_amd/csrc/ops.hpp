@@ -16,6 +16,7 @@ namespace lg {
 constexpr int64_t UNITS_DEVICE_MIN_ROWS = 65536;
 void build_units(DCsr &A, hipStream_t s);
 void build_units_host(DCsr &A, hipStream_t s);
+int32_t longest_row(const DCsr &A, hipStream_t s);
 // Column-sliced copy of A for precision prec (0: FP64, 1: FP32) with
 // slices of `width` columns (width >= ncols: no slicing).
 void build_slices(DCsr &A, int prec, int64_t width, hipStream_t s);

@@ -220,25 +220,7 @@ __global__ void k_child_fill(int64_t nc, const int32_t *cperm, Children C, const
     });
   }
 }
-__global__ void __launch_bounds__(256) k_max_row(int64_t n, const int32_t *rp, int32_t *longest) {
-  int32_t m = 0;
-  for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x)
-    m = max(m, rp[r + 1] - rp[r]);
-  for (int off = WAVE / 2; off >= 1; off >>= 1) m = max(m, __shfl_xor(m, off, WAVE));
-  if ((threadIdx.x & (WAVE - 1)) == 0) atomicMax(longest, m);
-}
 }  // namespace
-
-int32_t longest_row(const DCsr &A, hipStream_t s) {
-  DevBuf<int32_t> d(1);
-  fill_i32(d.p, 0, 1, s);
-  hipLaunchKernelGGL(k_max_row, dim3(grid_for(A.n, 256, 256)), dim3(256), 0, s, A.n, A.rp.p, d.p);
-  LG_LAUNCH_CHECK();
-  int32_t h = 0;
-  to_host(&h, d.p, 1, s);
-  LG_HIP(hipStreamSynchronize(s));
-  return h;
-}
 
 bool cluster_perm(const DLevel &L, const int32_t *cperm, DevBuf<int32_t> &perm, DevBuf<int32_t> &iperm, hipStream_t s) {
   const int64_t n = L.A.n, nc = L.nc;

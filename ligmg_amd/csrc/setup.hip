@@ -1714,9 +1714,9 @@ int64_t run_voting(const DCsr &A, const double *S, const double *cs, const ligmg
   const HugeRows &Hr = huge_of(A, s);
   state.alloc(n);
   ind.alloc(n);
-  DevBuf<int32_t> nstate(n), nind(n), vind(n), vf(n), flag(n), idx(n);
+  DevBuf<int32_t> nstate(n), nind(n), vind(n), vf(n);
   DevBuf<int8_t> vst(n);
-  DevBuf<double> vw(n), votes(n), nv(n);
+  DevBuf<double> vw(n), votes(n);
   hipLaunchKernelGGL(k_init_states, dim3(g1(n)), dim3(256), 0, s, (int)n, state.p, ind.p);
   LG_LAUNCH_CHECK();
   fill_f64(votes.p, 0.0, n, s);
@@ -1727,6 +1727,9 @@ int64_t run_voting(const DCsr &A, const double *S, const double *cs, const ligmg
   // undecided vertex is named by its neighbours alone.  A row longer than
   // HUGE_ROW would be one wavefront's serial chain; such levels sort.
   const bool row_tally = Hr.nrows == 0 && o.max_agg_size < 0 && o.rejection_ratio < 0 && !o.neighbor_of_neighbor;
+  const int64_t ns = row_tally ? 0 : n;
+  DevBuf<int32_t> flag(ns), idx(ns);
+  DevBuf<double> nv(ns);
   for (int iter = 0; iter < o.agg_iters; iter++) {
     const double th = o.agg_init_factor * std::pow(o.agg_iter_factor, iter);
     run_rows(n, A.rp.p, OpVote{A.ci.p, state.p, ind.p, S, th, o.neighbor_of_neighbor ? 1 : 0, vst.p, vind.p, vw.p},

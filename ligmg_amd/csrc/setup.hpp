@@ -68,7 +68,6 @@ void degree_order(DCsr &A, const std::vector<int64_t> &blocks, DevBuf<int32_t> &
 // to vertex, null: its own): vertices follow their coarse vertex.  False (and
 // no result) when some vertex has none.
 bool cluster_perm(const DLevel &L, const int32_t *cperm, DevBuf<int32_t> &perm, DevBuf<int32_t> &iperm, hipStream_t s);
-int32_t longest_row(const DCsr &A, hipStream_t s);
 // Degree permutation of A's rows inside blocks (perm: new -> old, iperm:
 // old -> new), the one degree_order applies.
 void degree_perm(const DCsr &A, const std::vector<int64_t> &blocks, DevBuf<int32_t> &perm, DevBuf<int32_t> &iperm,

@@ -968,7 +968,23 @@ void set_units(Units &U, int64_t nnz, const std::vector<int32_t> &row0, const st
   LG_HIP(hipStreamSynchronize(s));
 }
 
+// d: A's longest row
+void queue_longest_row(const DCsr &A, int32_t *d, hipStream_t s) {
+  fill_i32(d, 0, 1, s);
+  hipLaunchKernelGGL(k_longest_row, dim3(grid_for(A.n, 256, 256)), dim3(256), 0, s, A.n, A.rp.p, d);
+  LG_LAUNCH_CHECK();
+}
+
 }  // namespace
+
+int32_t longest_row(const DCsr &A, hipStream_t s) {
+  DevBuf<int32_t> d(1);
+  queue_longest_row(A, d.p, s);
+  int32_t h = 0;
+  to_host(&h, d.p, 1, s);
+  LG_HIP(hipStreamSynchronize(s));
+  return h;
+}
 
 // The greedy packing on the host, row by row.
 void build_units_host(DCsr &A, hipStream_t s) {
@@ -1041,9 +1057,7 @@ void build_units(DCsr &A, hipStream_t s) {
   const int64_t nlong = exclusive_scan_i32(islong.p, loff.p, M + 1, s);
   Units &U = A.U;
   DevBuf<int32_t> longest(1);
-  fill_i32(longest.p, 0, 1, s);
-  hipLaunchKernelGGL(k_longest_row, dim3(grid_for(n, 256, 256)), dim3(256), 0, s, n, A.rp.p, longest.p);
-  LG_LAUNCH_CHECK();
+  queue_longest_row(A, longest.p, s);
   int32_t ends[3];
   to_host(&ends[0], A.rp.p, 1, s);
   to_host(&ends[1], A.rp.p + n, 1, s);
@@ -1337,10 +1351,7 @@ void op_sub_block_mean(T *a, const RedPlan &P, const double *sums, hipStream_t s
 
 template void RedPlan::dots<double>(int, const double *const *, const double *const *, double *,
                                     hipStream_t) const;
-template void RedPlan::dots<float>(int, const float *const *, const float *const *, double *,
-                                   hipStream_t) const;
 template void RedPlan::sums<double>(const double *, double *, hipStream_t) const;
-template void RedPlan::sums<float>(const float *, double *, hipStream_t) const;
 #define LG_SEGS dim3((unsigned)R.nseg), dim3(256), 0, s
 template <class T, class F>
 void kr_begin(const RedPlan &R, const T *b, T *x, T *r, F *rf, const FirstStep<F> &f, hipStream_t s) {
@@ -1437,6 +1448,5 @@ template void kr_center<double, float>(const RedPlan &, double *, const float *,
 template void kr_center<float, float>(const RedPlan &, float *, const float *, const float *, hipStream_t);
 
 template void op_sub_block_mean<double>(double *, const RedPlan &, const double *, hipStream_t);
-template void op_sub_block_mean<float>(float *, const RedPlan &, const double *, hipStream_t);
 
 }  // namespace lg

@@ -39,7 +39,6 @@ namespace {
 // ------------------------------------------------------------ Krylov kernels
 using namespace sdev;
 
-// per-block scalar logic of CG / FCG (one thread per block)
 // FGMRES: y += sum_t coef[blk * K + t] V_t (V_t = V + t ld), added in t order
 __global__ void __launch_bounds__(256) k_blk_lincomb(double *y, const double *V, int64_t ld, int k,
                                                      const double *coef, int K, const int64_t *lo,
@@ -65,7 +64,7 @@ inline bool fcg_like(int t) { return t == LIGMG_KSP_FCG || t == LIGMG_KSP_PIPEFC
 template <class T>
 struct KWork {
   DevBuf<T> r, z, p, q, x;
-  DevBuf<double> sc, out;
+  DevBuf<double> sc;
   // x is allocated last and released first: where it is large enough, all are
   void alloc(int64_t n, int nb) {
     x.release();
@@ -74,7 +73,6 @@ struct KWork {
     p.alloc(n);
     q.alloc(n);
     sc.alloc((size_t)nb * SC_N);
-    out.alloc((size_t)nb * 4);
     x.alloc(n);
   }
 };
@@ -1438,7 +1436,7 @@ struct Solver {
   // the device.  The history logs the true residual at each cycle start and
   // the Givens estimate after each iteration, as PETSc's KSPGMRESCycle.
   static constexpr int FGMRES_RESTART = 30;
-  DevBuf<double> gm_V, gm_Z, gm_coef;
+  DevBuf<double> gm_V, gm_Z, gm_coef, gm_dots;
 
   int fgmres(size_t lvl, double *x, const double *b, std::vector<double> *hist, int *status) {
     const RedPlan &R = red[lvl];
@@ -1450,13 +1448,14 @@ struct Solver {
     gm_V.ensure((size_t)(m + 1) * n);
     gm_Z.ensure((size_t)m * n);
     gm_coef.ensure((size_t)nb * (m + 1));
+    gm_dots.ensure((size_t)nb * 4);
     KWork<double> &K = outer;
     const int32_t *segblk = R.bseg.p + R.nb + 1;
     auto V = [&](int j) { return gm_V.p + (size_t)j * n; };
     auto Z = [&](int j) { return gm_Z.p + (size_t)j * n; };
     auto dots = [&](int np, const double *const *a, const double *const *bb) {
-      R.dots<double>(np, a, bb, K.out.p, s);
-      return download(K.out.p, (size_t)nb * np, s);
+      R.dots<double>(np, a, bb, gm_dots.p, s);
+      return download(gm_dots.p, (size_t)nb * np, s);
     };
     auto upload = [&](const std::vector<double> &c) {
       to_device(gm_coef.p, c.data(), c.size(), s);
