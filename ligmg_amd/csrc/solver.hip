@@ -1366,7 +1366,7 @@ struct Solver {
   int krylov_solve(size_t lvl, double *x, const double *b, KWork<double> &K, std::vector<double> &hist, int *status) {
     const RedPlan &R = red[lvl];
     const DCsr &A = H[lvl].A;
-    const bool fcg = fcg_like(o.outer_ksp_type);
+    const bool fcg = fcg_like(o.outer_ksp_type), replay = replays(lvl, false);
     kr_reset();
     if (mixed) kr_begin<double, float>(R, b, x, K.r.p, W32[lvl].b.p, first_step<float>(lvl), s);
     else kr_begin<double, double>(R, b, x, K.r.p, nullptr, first_step<double>(lvl), s);
@@ -1376,7 +1376,7 @@ struct Solver {
     hist.push_back(wait_norm(R.nb, 1, &active));
     if (!active) return 0;
     for (int it = 1; it <= o.iters; it++) {
-      if (!o.use_graphs) iterate<double>(lvl, A, x, K, fcg, o.tol, true, true);
+      if (!replay) iterate<double>(lvl, A, x, K, fcg, o.tol, true, true);
       else LG_HIP(hipGraphLaunch(iteration_graph(lvl, A, x, K, fcg), s));
       const double tn = wait_norm(R.nb, (unsigned long long)it + 1, &active);
       hist.push_back(tn);
@@ -1398,6 +1398,28 @@ struct Solver {
     hipGraphExec_t e = capture([&] { iterate<double>(lvl, A, x, K, fcg, o.tol, true, true); });
     it_graphs.push_back({key, e});
     return e;
+  }
+
+  // Kernel launches of one cycle from level l, nearly: a K-cycle's grow by
+  // kcycle_iters a level, to 10^8 on fifteen levels with three.
+  double cycle_launches(size_t l, bool batched) const {
+    double below = 0;  // a visit of the level below
+    for (size_t k = H.size(); k-- > l;) {
+      double c = 3 + o.pre_smooth + o.post_smooth + below;
+      if (H[k].kind == LIGMG_LEVEL_ELIM) c = 2 + below;
+      if (H[k].kind == LIGMG_LEVEL_COARSE || k == dense_l0) c = 1;
+      below = k > l && inner_krylov(k) ? 2 + o.kcycle_iters * (c + 10) : c;
+      if (!batched && k > l && k >= tail_l0) below = 1;
+    }
+    return below;
+  }
+  // Whether iterations from level l are replayed from a graph.  HIP could not
+  // instantiate one of 180 000 launches (the process ended; 60 000 were fine),
+  // and a launch takes 2 kilobytes of host memory in it.  K-cycles of the
+  // default two inner steps have 2500 launches on a million vertices.
+  static constexpr double GRAPH_MAX_LAUNCHES = 1 << 15;
+  bool replays(size_t l, bool batched) const {
+    return o.use_graphs && cycle_launches(l, batched) <= GRAPH_MAX_LAUNCHES;
   }
 
   template <class F>
@@ -1607,7 +1629,7 @@ struct Solver {
   // levels) is captured once per (level, r, z) and replayed as a hipGraph;
   // it contains no host synchronisation and no memset nodes.
   void precond_outer(size_t lvl, const double *r, double *z) {
-    if (o.use_graphs) {
+    if (replays(lvl, false)) {
       for (auto &g : graphs)
         if (g.first.lvl == lvl && g.first.r == r && g.first.z == z) {
           LG_HIP(hipGraphLaunch(g.second, s));
@@ -1867,7 +1889,7 @@ struct Solver {
   int bkrylov_solve(size_t lvl, double *x, const double *b, KWork<double> &K, int kp, int *status) {
     const DCsr &A = H[lvl].A;
     const int64_t ns = (int64_t)bplan(lvl, kp).nb * kp;
-    const bool fcg = fcg_like(o.outer_ksp_type);
+    const bool fcg = fcg_like(o.outer_ksp_type), replay = replays(lvl, true);
     kr_reset();
     auto body = [&] {
       if (mixed) biterate<double, float>(lvl, A, x, K, BW32[lvl].b.p, kp, fcg, o.tol, true, kr_sink());
@@ -1885,7 +1907,7 @@ struct Solver {
       }
       if (!active) return it;
       if (it >= o.iters) break;
-      if (!o.use_graphs) {
+      if (!replay) {
         body();
         continue;
       }

@@ -242,3 +242,25 @@ def test_batch_alternating_widths(kw):
     alone, turns = seconds([3] * 4) + seconds([16] * 4), seconds([3, 16] * 4)
     print(f"{kw}: by itself {alone * 1e3:.2f} ms, in turn {turns * 1e3:.2f} ms")
     assert turns <= 1.1 * alone
+
+
+def test_deep_kcycle_is_not_captured():
+    """A K-cycle of half a million launches an iteration (three inner steps on
+    each of nine levels) runs as it is launched: HIP cannot instantiate a graph
+    of that size, nor one of a third of it."""
+    import resource
+    g = graphs.grid2d(40, 25)
+    kw = dict(kcycle=1, kcycle_iters=3, max_agg_size=3, max_levels=10, min_size=100, always_elim=0, top_elim=0, tail_nnz=0,
+              outer_ksp_type=_ffi.KSP_FCG, iters=1)
+    s = ligmg_amd.Solver(g, ligmg_amd.Options(**kw))
+    assert s.num_levels() == 11
+    B = graphs.rhs(g.n, 2, 3).reshape(g.n, 2, order="F")
+    before = resource.getrusage(resource.RUSAGE_SELF).ru_maxrss
+    X, info, its = s.solve_batch(B)
+    print(f"batch done, {info.time:.2f} s", flush=True)
+    x = s.solve(np.ascontiguousarray(B[:, 0]))
+    print(f"solve done, {x.time():.2f} s", flush=True)
+    grown = (resource.getrusage(resource.RUSAGE_SELF).ru_maxrss - before) >> 10
+    print(f"host memory grew by {grown} MiB")
+    assert its.max() == 1 and np.linalg.norm(X[:, 0] - x.solution) <= 1e-7 * np.linalg.norm(x.solution)
+    assert grown < 128
