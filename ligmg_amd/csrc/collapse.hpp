@@ -7,8 +7,9 @@
 namespace lg {
 
 // Whether a level is small enough to collapse.  A product with 1024^2 entries
-// (8 MiB, resident in the L2s) takes about 4 us, the levels below it 50 to 150
-// us of dependent launches: R-MAT 10 solve 1.37 -> 0.70 ms, 256 x 256 grid 14.6 ->
+// (8 MiB, a quarter of the L2s' 32) takes about 4 us, one with 2048^2 (32 MiB,
+// read from the Infinity Cache) about 10, the levels below 50 to 150 us of
+// dependent launches: R-MAT 10 solve 1.37 -> 0.70 ms, 256 x 256 grid 14.6 ->
 // 12.3 ms.  Forming the matrix takes about a dozen operations of nnz * n
 // multiply-adds per level (0.2 ms at 1024), so sparse levels may be twice as
 // large (the grid 6.5 -> 5.8 ms, 181 x 97 x 3 columns 4.7 -> 4.2 ms, a 250 K-vertex

@@ -54,8 +54,12 @@ inline int row_items_for(int64_t nnz) { return nnz >= ROW_ITEMS_BIG_NNZ ? 16 : 4
 // chain of latencies, which the row kernel shortens (Chebyshev step of a
 // 65 K-vertex grid's levels 6.3 -> 3.7 us, a 97-workgroup interpolation 4.0 ->
 // 2.7 us); large ones are bound by cache accesses, which the units' coalesced
-// streams save (9.1 M entries: 81 us staged, 88 us by rows; at 1.2 M the rows
-// still win).
+// streams save (9.1 M entries: 81 us staged, 88 us by rows).  In between the
+// two cross more than once: Chebyshev steps by rows are 1.2 to 1.6 times as fast
+// at 0.5 M entries; from 1.5 to 2 M 1.0 to 1.1 times in FP32, 0.94 to 1.0 on grids
+// and 0.8 on geometric graphs in FP64.  Solves with the line here against 1 M:
+// 3-D grids and small-world graphs of 1.3 to 1.7 M 2 to 4% faster, geometric
+// graphs of 1.5 to 1.9 M 1% faster in FP32, 2% slower in FP64.
 constexpr int ROW_U = 4;
 constexpr int ROW_ROUNDS = 8;
 constexpr int64_t ROW_MAX_NNZ = (int64_t)2 << 20;

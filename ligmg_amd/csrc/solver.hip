@@ -682,6 +682,12 @@ struct Solver {
   // order; 84 unsorted) to 42 us and the solve from 36.2 to 24.5 ms; on a 100^3
   // grid, row by row already, from 178 to 165 us for 32 columns.  Power-law
   // levels have no such clusters and gain from the hubs (R-MAT 20: 10.9 -> 9.1 ms).
+  // The line errs to the old order.  Solves in cluster order against degree
+  // order, by longest row over mean row, graphs with some random long rows:
+  // 3.3: 1.20x, 3.8: 1.10x, 5.5: 1.28x, 5.9: 1.05x, 6.7: 1.10x, 7.4: 1.01x;
+  // above it 8.5: 1.25x, 9.3: 1.07x, 11.3: 1.06x, 13.7: 1.21x, 30.7: 1.19x;
+  // Barabasi-Albert at 197: 0.97 to 0.99x, R-MAT 17 at 368: 1.00x.  A random graph of
+  // 16 neighbours a vertex (2.2) has no clusters: 1.00x.
   static constexpr int64_t EVEN_ROWS = 8;  // longest row over the mean one
   void apply_solve_layout() {
     const size_t nl = H.size();
@@ -1206,7 +1212,8 @@ struct Solver {
   }
 
   // Above this the fused kernel's chain of gathers per vertex costs more than
-  // the launch it saves (700 K vertices: a solve 36.2 -> 36.9 ms; 65 K: 6.95 -> 6.6 ms).
+  // the launch it saves (700 K vertices: a solve 36.2 -> 36.9 ms; 65 K: 6.95 -> 6.6 ms;
+  // solves of 100 to 190 K were 1 to 3% faster with it, on either side of the line).
   static constexpr int64_t PROLONG_INTERP_MAX_N = (int64_t)1 << 17;
 
   // level l + 1's correction for the right-hand side Op v

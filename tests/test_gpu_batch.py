@@ -121,10 +121,9 @@ def test_union_with_collapsing_blocks(prec):
 @pytest.mark.parametrize("k", [1, 2, 7, 16, 64])
 @pytest.mark.parametrize("prec", [_ffi.PREC_FP64, _ffi.PREC_MIXED])
 def test_spmm_tiles_tuned_equal_fixed(k, prec):
-    """The batched SpMM tile tuner (right-hand sides per lane, gathers in
-    flight, picked per level operator by timing) changes no bit: every
-    (row, right-hand side) sum of a complete row is one lane adding the
-    row's entries in order, whatever the tile; hub-row chunks keep one tile."""
+    """spmm_tune changes no bit.  Operators this small take the rule's tile
+    either way (test_batch_hub_rows_and_segments has timed ones): the groups a
+    row is split over, and so its sum, do not depend on the tile."""
     g = graphs.union([graphs.rmat_config(12, "lognormal", pendants=True),
                       graphs.grid3d(12, 10, 9, wkind=_ffi.W_UNIFORM, p0=0.1, p1=10.0, seed=2)])
     B = graphs.rhs(g.n, k, 5, comp_ptr=g.comp_ptr).reshape(g.n, k, order="F")

@@ -20,8 +20,8 @@ VARIANTS = {
     "kcycle": {"kcycle": 1},  # nothing is collapsed
 }
 GRAPHS = {
-    "grid32": lambda: graphs.grid2d(64, 32),  # the base level has exactly 2048 vertices
-    "grid33": lambda: graphs.grid2d(683, 3, graphs.W_UNIFORM, 0.1, 10.0, 3),  # 2049: one above
+    "grid64x32": lambda: graphs.grid2d(64, 32),  # the base level has exactly 2048 vertices
+    "grid683x3": lambda: graphs.grid2d(683, 3, graphs.W_UNIFORM, 0.1, 10.0, 3),  # 2049: one above
     "dense1024": lambda: graphs.barabasi_albert(1024, 20, seed=2),  # long rows: at the smaller bound
     "dense1025": lambda: graphs.barabasi_albert(1025, 20, seed=2),
     "rmat12": lambda: graphs.rmat_config(12, "lognormal", pendants=True),
