@@ -203,8 +203,8 @@ def test_batch_many_sets(sizes, k, prec):
 
 
 def test_batch_of_many_graphs_costs_its_columns():
-    """64 columns of 3000 small graphs take about 5 times as long as one; with
-    every set's norm written to the host on its own it was 80 times."""
+    """64 columns of 3000 small graphs take about 3 times as long as one; with
+    every set's norm written to the host on its own it was 90 times."""
     u = graphs.union([graphs.barabasi_albert(60, 3, seed=i) for i in range(3000)])
     s = ligmg_amd.Solver(u, ligmg_amd.Options(precision=_ffi.PREC_MIXED, outer_ksp_type=_ffi.KSP_FCG), comp_ptr=u.comp_ptr)
     t = {}
